@@ -16,70 +16,91 @@
 //           between 2^-17 and 65504), sequence b at rows koff_b .. koff_b +
 //           prefix_b + q_b - 1 (koff_b = sum over b' < b of prefix_b' + q_b');
 //           HBM-bound, read once per call instead of once per query block.
-//   attend  a block takes BM consecutive (token, head) query rows of one
-//           sequence (all heads share the keys: MQA) and walks its keys in
-//           tiles of 64, each copied from the workspace into LDS by the whole
-//           block while the previous tile is consumed (double-buffered, one
-//           barrier per tile). Per wave and tile:
-//   S^T[64 keys, RW rows] = K . Q^T   on fp16 MFMA 16x16x32 (Q converted to fp16
+//   attend  a block takes 128 consecutive (token, head) query rows of one
+//           sequence (all heads share the keys: MQA), 32 per wave, and walks
+//           its keys in tiles copied from the workspace into a ring of LDS
+//           buffers. Per wave and 32 keys:
+//   S^T[32 keys, 32 rows] = K . Q^T   on fp16 MFMA 32x32x16 (Q converted to fp16
 //                                     once, held in registers: exact products);
-//   the causal mask only on tiles that reach past the block's first query position
+//   the causal mask only on keys that reach past the block's first query position
 //   softmax in the log2 domain against a per-row reference (the row's maximum
-//   over the first tile + 8); a tile whose scores pass it by more than 15
-//   moves it to the tile's maximum + 8 and scales O and the row sum by the
-//   difference in place (scale_acc16), so every probability fits fp16
-//   O[RW rows, D] += P . V           on fp16 MFMA 16x16x32 per 32-key half, the keys of
-//                                     each lane taken in the order the score MFMA left
+//   over its first keys + 8); scores that pass it by more than 15 move it to
+//   their maximum + 8 and scale O and the row sum by the difference in place
+//   (scale_acc32x8), so every probability fits fp16
+//   O^T[D, 32 rows] += V^T . P^T      on fp16 MFMA 32x32x16, the keys of each
+//                                     lane taken in the order the score MFMA left
 //                                     them, P rounded to fp16 (relative error 2^-12).
 // A sequence whose key rows do not fit the workspace (the caller's key_rows
 // was short of the true sum) gets NaN outputs.
 #include "rolaq_common.h"
 #include "rolaq_args.h"
 
+#include <type_traits>
+
 namespace rolaq {
 
-constexpr int kExtKeys = 64;          // keys per tile
-constexpr int kExtMK = kExtKeys / 16;  // 16-key blocks per tile
-constexpr int kExtKH = kExtKeys / 32;  // 32-key halves (K-steps of the output MFMA)
 constexpr float kExtSlack = 15.0f;    // max exp2 argument: a probability stays <= 2^15 (fp16)
 constexpr float kExtHeadroom = 8.0f;  // a reference sits this far above the maximum it was set from
-constexpr float kExtMasked = -1.0e30f;
+constexpr float kExtNoRef = -1.0e30f;  // reference of a row that has seen no key yet (log2 units)
 
 template <int D, int R>
 struct ExtGeo {
   static constexpr int DR = D + R;
-  static constexpr int KSQ = DR / 32;               // K-steps of the score MFMA
-  static constexpr int NBR = 1;                     // 16-row blocks per wave
-  static constexpr int RW = 16 * NBR;               // query rows per wave
-  // D = 256: 8 waves, two per SIMD (one wave's softmax and tile build overlap
-  // the other's MFMAs; 16 rows per wave keep it within 256 registers);
-  // D = 512: 4 waves, one per SIMD (the 32 output blocks need the registers)
-  static constexpr int WAVES = D == 256 ? 8 : 4;
+  static constexpr int RB = 2 * DR;                 // bytes per key row (workspace and LDS)
+  static constexpr int CPR = RB / 16;               // 16-byte chunks per key row
+  static constexpr int WAVES = 4;                   // one per SIMD: O and Q fill its 512 registers
+  static constexpr int RW = 32;                     // query rows per wave
   static constexpr int BM = WAVES * RW;             // query rows per block
-  static constexpr int ND = D / 16;                 // output column blocks
-  static constexpr int KSTR = 2 * DR + 32;          // bytes per key row in LDS (padding measured: +32 B fastest)
-  static constexpr int KBYTES = kExtKeys * KSTR;
-  static constexpr int BUF = KBYTES;                // one tile: key rows only
-  // tiles per barrier: D = 256 keeps a ring of four tiles in LDS and meets at
-  // a barrier every second tile (fewer points where all eight waves align);
-  // D = 512's tiles allow two buffers, one barrier per tile
-  static constexpr int TPB = D == 256 ? 2 : 1;
-  static constexpr int NBUF = 2 * TPB;
-  static constexpr int OPT = D / 256;               // latent octets per loader thread
+  static constexpr int KT = D == 256 ? 64 : 32;     // keys per step: one 36,864-byte tile at both widths
+  static constexpr int KSQ = DR / 16;               // K-steps of the score MFMA
+  static constexpr int ND = D / 32;                 // output column blocks
+  static constexpr int TILE = KT * RB;
+  static constexpr int NBUF = 4;                    // ring of tiles in LDS
+  static constexpr int WROWS = KT / WAVES;          // key rows that one wave copies
+  static constexpr int NDMA = WROWS * CPR / 64;     // its 16-byte-per-lane copies per tile
+  static_assert(WROWS * CPR % 64 == 0 && NDMA == 9 && TILE == 36864, "tile copy");
 };
 
-__device__ __forceinline__ float max_over_rows(float v) {
-  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+// Swizzle of a key row in LDS: 16-byte chunk c of row r sits at chunk
+// c ^ ext_sw(r) (only the low 3 / 2 bits change, so it stays in its row). A
+// row is 72 (D = 512) or 36 chunks, 8 or 4 modulo the 16 chunks that the 64
+// banks hold: with these bits the 16 rows of one column that a quarter wave of
+// a score read touches, and the 4 rows x 64 bytes of half a wave of a
+// transposed read, fall on 16 distinct chunk positions each.
+template <int D>
+__device__ __forceinline__ int ext_sw(int r) {
+  return D == 512 ? ((r & 2) << 1) | ((r >> 1) & 2) | ((r >> 3) & 1) : (r >> 2) & 3;
 }
 
-__device__ __forceinline__ float add_over_rows(float v) {
+// Up to four 1 KB copies of 16 bytes per lane into LDS, past the registers:
+// copy j from base + off_j + 1024 j (off per lane) to lds + 1024 j + 16 lane
+// (the instruction's offset counts on both sides). In assembly because the
+// compiler, which tracks such copies, would wait for all of them before any
+// LDS read that follows; the kernel waits by count instead (meet). Nothing is
+// returned to a register.
+__device__ __forceinline__ void copy_to_lds(uint64_t base, uint32_t o0, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(o0), "s"(base)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void copy_to_lds4(uint64_t base, uint32_t o0, uint32_t o1, uint32_t o2, uint32_t o3,
+                                             uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\t"
+      "global_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+      "global_load_lds_dwordx4 %3, %5 offset:2048\n\t"
+      "global_load_lds_dwordx4 %4, %5 offset:3072" ::"s"(lds),
+      "v"(o0), "v"(o1), "v"(o2), "v"(o3), "s"(base)
+      : "memory", "m0");
+}
+
+__device__ __forceinline__ float max_over_halves(float v) {
   const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
+
+__device__ __forceinline__ float add_over_halves(float v) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
 // Workspace row of key 0 of sequence b.
@@ -136,26 +157,36 @@ __global__ __launch_bounds__(256) void extend_gather_kernel(ExtendArgs a) {
   }
 }
 
-// 64 bits of the output MFMA's B operand, read transposed out of the key rows
-// (ds_read_b64_tr_b16: within each 16-lane group, lane 4s + e receives element
-// e of the chunks addressed by lanes s, s + 4, s + 8, s + 12). Lane (gq, la)
-// addresses key row tau(gq, 4h + (la >> 2)) at latent columns 16 nd + 4 (la & 3),
-// so it receives rows tau(gq, 4h + 0..3) of column 16 nd + la: K-index
-// 8 gq + 4h + k of B is key tau(gq, 4h + k), the order P is held in.
-__device__ __forceinline__ u32x2 read_v_tr(const uint8_t* kb, int kstr, int gq, int la, int nd, int h) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  const int key = 16 * h + 4 * gq + (la >> 2);
-  const uint8_t* p = kb + key * kstr + 2 * (16 * nd + 4 * (la & 3));
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-  return __builtin_bit_cast(u32x2, v);
-}
-
+// ---------------------------------------------------------------------------
+// Attend. What bounds it: the matrix cores and their power. 16-row waves on
+// 16x16x32 MFMA (the form before) read 1 KB of LDS per 16-cycle MFMA, all of
+// the CU's 256 bytes per clock; 32 rows per wave on 32x32x16 need half of
+// that. One wave per SIMD (O and Q fill its registers) issues an instruction
+// every 4 to 5 cycles, so the instructions are counted (below), and all VALU
+// work sits behind MFMAs, in whose shadow it is free: a 32x32x16 MFMA alone
+// takes 14 to 15 ns, with six VALU operations behind it 16.
+// Measured, before -> after: 4 x 2048 queries over 14336 keys, 40 heads, D =
+// 256: 5.42 -> 4.47 ms (1.22 PFLOP/s, 3108 cycles per 64 keys and wave, of
+// which 2176 are MFMAs, at 1.62 GHz: the clock falls with the matrix cores'
+// power); six ragged chunks, 16 heads, D = 512: 1.04 -> 0.43 ms; 96 queries
+// over 12345 keys: 0.89 -> 0.58 ms.
+//
+// A lane holds one query row (column la32 of the MFMAs): its scores, its
+// reference, its sum and its outputs, so nothing crosses lanes but the two
+// halves' maximum. The softmax of 32 keys runs behind the MFMAs of the
+// previous keys' output (D = 512), and at D = 256, where registers allow a
+// second S, behind those of the next keys' scores as well.
+//
+// Key tiles are copied from the workspace straight into the ring: while the
+// MFMAs read tiles i - 1 (V), i and i + 1 (K), the copies of later tiles are in
+// flight, each requested after the barrier that ends the use of its buffer and
+// awaited by count at a later one.
+// ---------------------------------------------------------------------------
 template <int D, int R>
 __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(ExtendArgs a) {
   using G = ExtGeo<D, R>;
-  constexpr int KSQ = G::KSQ, NBR = G::NBR, RW = G::RW, BM = G::BM, ND = G::ND;
-  define_acc_macros();
+  constexpr int RB = G::RB, CPR = G::CPR, KT = G::KT, KSQ = G::KSQ, ND = G::ND, BM = G::BM, RW = G::RW;
+  define_acc32_macros();
   extern __shared__ __attribute__((aligned(16))) uint8_t s_buf[];
 
   const int b = blockIdx.x;
@@ -170,7 +201,7 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   const int64_t koff = key_offset(a, b);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int gq = lane >> 4, la = lane & 15;
+  const int g = lane >> 5, la32 = lane & 31;
   if (koff + L > a.ws_rows) {
     // the sequence's key rows did not fit the workspace: its outputs are NaN
     for (int64_t e = tid; e < (int64_t)BM * D; e += 64 * G::WAVES) {
@@ -182,225 +213,414 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   // last query token of the block -> keys 0 .. prefix + t_last
   const int64_t t_last = min(nrows - 1, r0 + BM - 1) / a.H;
   const int kend = (int)(prefix + t_last + 1);
-  const int ntiles = (kend + kExtKeys - 1) / kExtKeys;
+  const int n = (kend + KT - 1) / KT;  // steps
 
-  // tile copy: thread tid moves 16-byte chunks tid, tid + NT, ... of the tile's
-  // key rows (keys past the block's last key are zeros)
-  constexpr int DR = D + R, CPR = DR / 8, CH = kExtKeys * CPR, NT = 64 * G::WAVES, NCH = (CH + NT - 1) / NT;
-  u32x4 raw[NCH];
-  auto load_keys = [&](int k0) {
+  // ---- tile copies: this wave's rows of a tile, 16-byte chunk 64 j + lane ------
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)s_buf;
+  // byte offset of the chunk from kBias bytes before the wave's first row, less
+  // the 1024 (j % 4) that the copy's own offset adds (kBias keeps the
+  // unsigned offsets from wrapping, also when clamp_rows moves them to row 0)
+  constexpr int kBias = 3 * 1024;
+  uint32_t doff[G::NDMA];
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      const int ci = tid + NT * j;
-      const int key = ci / CPR, c = ci - key * CPR;
-      const int64_t kp = k0 + key;
-      raw[j] = (ci < CH && kp < kend) ? gload<u32x4>(a.ws + (koff + kp) * DR + 8 * c) : u32x4{0u, 0u, 0u, 0u};
+  for (int j = 0; j < G::NDMA; ++j) {
+    const int ci = 64 * j + lane, row = ci / CPR, pc = ci - row * CPR;
+    doff[j] = kBias + row * RB + 16 * (pc ^ ext_sw<D>(G::WROWS * wave + row)) - 1024 * (j % 4);
+  }
+  const uint64_t keys_v = reinterpret_cast<uint64_t>(a.ws) + (uint64_t)koff * RB - kBias;
+  const uint64_t keys = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)keys_v) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(keys_v >> 32)) << 32;
+  // Third p of the copies of tile i. Rows past the block's last key read that
+  // key again: they are masked (clamp_rows(i) comes before the parts). In
+  // place of tiles past the last one that one is copied again, to buffers that
+  // nothing reads any more, so that every step issues the same copies.
+  auto clamp_rows = [&](int i) {
+    if (__builtin_expect(i == n - 1, 0)) {
+      asm volatile("");  // a branch, taken once
+      const int last = max(kend - 1 - KT * i - G::WROWS * wave, 0);
+#pragma unroll
+      for (int j = 0; j < G::NDMA; ++j) {
+        const int row = (64 * j + lane) / CPR;
+        doff[j] -= (row - min(row, last)) * RB;
+      }
     }
   };
-  auto store_keys = [&](uint8_t* buf) {
-#pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      const int ci = tid + NT * j;
-      const int key = ci / CPR, c = ci - key * CPR;
-      if (ci < CH) *reinterpret_cast<u32x4*>(buf + key * G::KSTR + 16 * c) = raw[j];
-    }
+  auto copy_part = [&](int i, int p) {
+    const int row0 = min(KT * min(i, n - 1) + G::WROWS * wave, kend - 1);
+    const uint64_t src = keys + (uint64_t)row0 * RB;
+    const uint32_t dst = lds0 + (i % G::NBUF) * G::TILE + G::WROWS * RB * wave + 4096 * p;
+    if (p < 2)
+      copy_to_lds4(src, doff[4 * p], doff[4 * p + 1], doff[4 * p + 2], doff[4 * p + 3], dst);
+    else
+      copy_to_lds(src, doff[8], dst);
   };
-
-  // ---- query rows of this wave: Q^T fragments (fp16) and positions ------------
-  u32x4 qf[NBR][KSQ];
-  int64_t qpos[NBR];
 #pragma unroll
-  for (int nb = 0; nb < NBR; ++nb) {
-    const int64_t r = r0 + RW * wave + 16 * nb + la;
+  for (int t = 0; t < 3; ++t) {
+    clamp_rows(t);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) copy_part(t, p);
+  }
+
+  // ---- query rows of this wave: Q^T fragments (fp16) and causal limits --------
+  u32x4 qf[KSQ];
+  int qp;  // causal limit of the lane's row (-1: no row)
+  {
+    const int64_t r = r0 + RW * wave + la32;
     const bool ok = r < nrows;
     const int64_t t = ok ? r / a.H : 0, h = ok ? r % a.H : 0;
-    qpos[nb] = ok ? prefix + t : -1;
-    const uint16_t* qr = a.q + (qo0 + t) * a.q_st + h * a.q_sh + 8 * gq;
+    qp = ok ? (int)(prefix + t) : -1;
+    const uint16_t* qr = a.q + (qo0 + t) * a.q_st + h * a.q_sh + 8 * g;
 #pragma unroll
     for (int ks = 0; ks < KSQ; ++ks)
-      qf[nb][ks] = ok ? bf16x8_to_f16x8(*reinterpret_cast<const u32x4*>(qr + 32 * ks)) : u32x4{0u, 0u, 0u, 0u};
+      qf[ks] = ok ? bf16x8_to_f16x8(gload<u32x4>(qr + 16 * ks)) : u32x4{0u, 0u, 0u, 0u};
   }
-
   const float c2 = a.sm_scale * kLog2e;
   const int qfirst = (int)(prefix + r0 / a.H);  // causal limit of the block's first row
-  int qp[NBR];  // causal limit of each lane's rows (-1: no row)
-#pragma unroll
-  for (int nb = 0; nb < NBR; ++nb) qp[nb] = (int)qpos[nb];
 
-  f32x4 acc_o[NBR][ND];
-  float m_ref[NBR], l_run[NBR];
+  // ---- LDS read addresses: a few lane bases plus immediate offsets ------------
+  // score operand of K-step ks: row la32 of the unit's 32 keys, chunk 2 ks + g
+  constexpr int KB = D == 512 ? 4 : 2;   // K-steps per swizzled group of chunks
+  uint32_t kbase[KB];
 #pragma unroll
-  for (int nb = 0; nb < NBR; ++nb) {
+  for (int k = 0; k < KB; ++k) kbase[k] = la32 * RB + 16 * ((2 * k + g) ^ ext_sw<D>(la32));
+  // transposed reads of V (ds_read_b64_tr_b16: within each 16-lane group, lane
+  // 4s + e receives element e of the chunks addressed by lanes s, s + 4,
+  // s + 8, s + 12): half h of MFMA m's 16 keys and column block nd: lane
+  // addresses key 16 m + 8 h + 4 g + (la >> 2) at columns 32 nd + 16 ((lane >>
+  // 4) & 1) + 4 (la & 3), and receives keys 16 m + 8 h + 4 g + 0..3 of column
+  // 32 nd + la32: the order in which the score MFMA leaves a lane's keys
+  constexpr int VB = D == 512 ? 2 : 1;   // column blocks per swizzled group
+  uint32_t vbase[VB][2];
+  {
+    const int la = lane & 15, x = 2 * ((lane >> 4) & 1) + ((la & 3) >> 1);
 #pragma unroll
-    for (int nd = 0; nd < ND; ++nd) acc_o[nb][nd] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m_ref[nb] = kExtMasked;
-    l_run[nb] = 0.f;
+    for (int h = 0; h < 2; ++h) {
+      const int row = 8 * h + 4 * g + (la >> 2);
+#pragma unroll
+      for (int v = 0; v < VB; ++v) vbase[v][h] = row * RB + 16 * ((4 * v + x) ^ ext_sw<D>(row)) + 8 * (la & 1);
+    }
   }
-
-  constexpr int TPB = G::TPB, NBUF = G::NBUF;
+  auto kread = [&](const uint8_t* kb, int ks) {
+    return *reinterpret_cast<const u32x4*>(kb + kbase[ks % KB] + 32 * KB * (ks / KB));
+  };
+  auto vread = [&](const uint8_t* vb, int m, int nd) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    u32x2 v[2];
 #pragma unroll
-  for (int t = 0; t < TPB; ++t) {
-    if (t < ntiles) {
-      load_keys(t * kExtKeys);
-      store_keys(s_buf + t * G::BUF);
+    for (int h = 0; h < 2; ++h) {
+      const uint8_t* p = vb + vbase[nd % VB][h] + 64 * VB * (nd / VB) + 16 * m * RB;
+      v[h] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p)));
     }
-  }
-  __syncthreads();
+    return u32x4{v[0].x, v[0].y, v[1].x, v[1].y};
+  };
 
-  // Tile it is read from buffer it % NBUF; tile it + TPB is loaded during
-  // tile it and stored after it into the buffer of tile it - TPB, which every
-  // wave finished before the barrier that ended the previous group of TPB tiles.
-  for (int it = 0; it < ntiles; ++it) {
-    const uint8_t* kb = s_buf + (it % NBUF) * G::BUF;
-    const int k0 = it * kExtKeys;
-    // loads of a later tile first: they have this tile's compute to land
-    if (it + TPB < ntiles) load_keys(k0 + TPB * kExtKeys);
+  f32x16 O[ND];  // O^T: columns d = 32 nd + 8 (j / 4) + 4 g + j % 4 of the lane's row
+#pragma unroll
+  for (int nd = 0; nd < ND; ++nd)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) O[nd][j] = 0.f;
+  float m_ref = kExtNoRef, l_run = 0.f;
 
-    // ---- scores S^T[key, row] ----------------------------------------------
-    f32x4 s[kExtMK][NBR];
+  // The MFMAs of a 32-key unit, KSQ for its scores and 2 ND for an output,
+  // run in pairs whose LDS operands are read kAhead pairs before and awaited
+  // once per pair; the scheduling barriers keep the order in which it is
+  // written. One wave issues an instruction every 4 to 5 cycles, so each
+  // one counts (a wait before every MFMA, one M0 setting per copy and
+  // per-copy row clamps cost 160 of 550 per 64 keys).
+  constexpr int kAhead = 2, kRing = 2 * (kAhead + 1);
+  constexpr int kAllK = KSQ, kAllV = 2 * ND;
+  u32x4 kf[kRing], vf[kRing];
+  // MFMA k of a unit's scores S^T (K rows kb of 32 keys). The accumulators are
+  // VGPRs, written by MFMAs in assembly: left to the compiler, which gives
+  // every MFMA of a kernel with AGPR accumulators an AGPR one, each score
+  // would be copied before its softmax. The compiler does not see the
+  // results' latency: between a unit's last score MFMA and the first use of
+  // its scores there are output MFMAs, or settle().
+  auto score_mfma = [&](f32x16& S, int k) {
+    if (k == 0)
+      asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=v"(S) : "v"(kf[0]), "v"(qf[0]));
+    else
+      asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(S) : "v"(kf[k % kRing]), "v"(qf[k]));
+  };
+  auto settle = [&](f32x16& S) { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 2" : "+v"(S)); };
+  auto output_mfma = [&](const u32x4 (&P)[2], int k) {
+    O[k % ND] = mfma32x32x16_f16(vf[k % kRing], P[k / ND], O[k % ND]);
+  };
+  // the operands of MFMAs k and k + 1
+  auto kfetch = [&](const uint8_t* kb, int k) {
+    kf[k % kRing] = kread(kb, k);
+    kf[(k + 1) % kRing] = kread(kb, k + 1);
+  };
+  auto vfetch = [&](const uint8_t* vb, int k) {
+    vf[k % kRing] = vread(vb, k / ND, k % ND);
+    vf[(k + 1) % kRing] = vread(vb, (k + 1) / ND, (k + 1) % ND);
+  };
+  // LDS reads but the last n have returned (the lgkmcnt field; n <= 15)
+  auto landed = [&](auto n) {
+    __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4) | (decltype(n)::value << 8));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Pairs of score MFMAs of a unit's rows at kb, the next pairs' reads ahead
+  // of them (the last ones those of the output that follows, at vb); each
+  // slot's other work is done by `slice`
+  auto score_phase = [&](f32x16& S, const uint8_t* kb, const uint8_t* vb, auto slice) {
 #pragma unroll
-    for (int mk = 0; mk < kExtMK; ++mk)
+    for (int k = 0; k < kAllK; k += 2) {
+      const int a2 = k + 2 * kAhead;
+      if (a2 < kAllK)
+        kfetch(kb, a2);
+      else
+        vfetch(vb, a2 - kAllK);
+      __builtin_amdgcn_sched_barrier(0);
+      // reads after this pair's: K pairs have two, V pairs four
+      if (a2 < kAllK)
+        landed(std::integral_constant<int, 4>{});
+      else if (a2 == kAllK)
+        landed(std::integral_constant<int, 6>{});
+      else
+        landed(std::integral_constant<int, 8>{});
 #pragma unroll
-      for (int nb = 0; nb < NBR; ++nb) s[mk][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the K operands of K-step ks + 1 are read while step ks's MFMAs run
-    auto kread = [&](int ks, int mk) {
-      return *reinterpret_cast<const u32x4*>(kb + (16 * mk + la) * G::KSTR + 64 * ks + 16 * gq);
-    };
-    u32x4 kf[2][kExtMK];
-#pragma unroll
-    for (int mk = 0; mk < kExtMK; ++mk) kf[0][mk] = kread(0, mk);
-#pragma unroll
-    for (int ks = 0; ks < KSQ; ++ks) {
-      if (ks + 1 < KSQ) {
-#pragma unroll
-        for (int mk = 0; mk < kExtMK; ++mk) kf[(ks + 1) & 1][mk] = kread(ks + 1, mk);
+      for (int q = 0; q < 2; ++q) {
+        score_mfma(S, k + q);
+        slice(k + q);
+        __builtin_amdgcn_sched_barrier(0);
       }
+    }
+  };
+  // Pairs of output MFMAs; the reads of the next unit's scores (kn) go out
+  // ahead of the last ones. With `cross`, kn is another tile: it is awaited
+  // where every V operand is in registers, and its first reads go out under
+  // the remaining MFMAs.
+  auto output_phase = [&](const u32x4 (&P)[2], const uint8_t* vb, const uint8_t* kn, bool cross, auto slice,
+                          auto meet) {
 #pragma unroll
-      for (int mk = 0; mk < kExtMK; ++mk)
+    for (int k = 0; k < kAllV; k += 2) {
+      const int a2 = k + 2 * kAhead;
+      if (a2 == kAllV && cross) meet();
+      if (a2 < kAllV)
+        vfetch(vb, a2);
+      else
+        kfetch(kn, a2 - kAllV);
+      __builtin_amdgcn_sched_barrier(0);
+      if (a2 < kAllV)
+        landed(std::integral_constant<int, 8>{});
+      else if (a2 == kAllV)
+        landed(std::integral_constant<int, 6>{});
+      else
+        landed(std::integral_constant<int, 4>{});
 #pragma unroll
-        for (int nb = 0; nb < NBR; ++nb) s[mk][nb] = mfma16x16x32_f16(kf[ks & 1][mk], qf[nb][ks], s[mk][nb]);
-      if (ks + 1 < KSQ) {
-        __builtin_amdgcn_sched_group_barrier(0x100, kExtMK, 0);  // the next step's reads
-        __builtin_amdgcn_sched_group_barrier(0x008, kExtMK * NBR, 0);
+      for (int q = 0; q < 2; ++q) {
+        output_mfma(P, k + q);
+        slice(k + q);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-
-    // ---- softmax (row = 16 nb + la; keys 16 mk + 4 gq + i) -------------------
-    // Scores stay in raw units (the scale c2 > 0 is applied inside the exp2's
-    // argument, by one FMA). A tile that ends before the block's first query
-    // position needs no causal mask (rows past the last query, qp = -1, stay
-    // masked).
-    const bool open = k0 + kExtKeys - 1 <= qfirst;
+  };
+  // keys past a row's causal limit (only in units that reach past the block's
+  // first row): -inf, so that a row without any key in the unit adds nothing
+  auto mask = [&](f32x16& S, int key0) {
+    if (__builtin_expect(key0 + 31 > qfirst, 0)) {
+      asm volatile("");  // a branch, not selects in every unit
+      const int lim = qp < 0 ? -1 : qp - key0 - 4 * g;
 #pragma unroll
-    for (int nb = 0; nb < NBR; ++nb) {
-      // key k0 + 16 mk + 4 gq + i is visible to the row when 16 mk + i <= lim
-      const int lim = qp[nb] < 0 ? -1 : (open ? kExtKeys : qp[nb] - k0 - 4 * gq);
-#pragma unroll
-      for (int mk = 0; mk < kExtMK; ++mk)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s[mk][nb][i] = 16 * mk + i <= lim ? s[mk][nb][i] : kExtMasked;
+      for (int j = 0; j < 16; ++j) S[j] = 8 * (j / 4) + j % 4 <= lim ? S[j] : -__builtin_inff();
     }
-    float mx[NBR];
-    uint64_t need[NBR];  // lanes whose row passes its reference by more than the slack
+  };
+  // Softmax of a unit's S against the row's reference (log2 domain, the scale
+  // inside the exp2's argument): a unit that passes the reference by more than
+  // the slack moves it to the unit's maximum + 8; f scales what was summed
+  // before. It runs in `slots` slices, one behind each of that many MFMAs: the
+  // maximum in slices 1..4, the reference, then the probabilities of eight
+  // pairs of keys, six operations each, spread over the remaining slices.
+  float mx, f, mn, t0, t1;
+  uint64_t need;
+  auto softmax_slice = [&](const f32x16& S, u32x4 (&p)[2], int k, int slots) {
+    constexpr int kFirst = 6, kOps = 48;
+    if (k >= 1 && k <= 4) {
 #pragma unroll
-    for (int nb = 0; nb < NBR; ++nb) {
-      mx[nb] = kExtMasked;
-#pragma unroll
-      for (int mk = 0; mk < kExtMK; ++mk)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mx[nb] = fmaxf(mx[nb], s[mk][nb][i]);
-      mx[nb] *= c2;  // log2 units (a masked maximum stays far below any reference)
-      need[nb] = __builtin_amdgcn_ballot_w64(it > 0 && mx[nb] > m_ref[nb] + kExtSlack);
+      for (int e = 4 * (k - 1); e < 4 * k; ++e) mx = e == 0 ? S[0] : fmaxf(mx, S[e]);
     }
-    // the first tile sets each row's reference (key 0 is visible to every row)
-    if (it == 0) {
-#pragma unroll
-      for (int nb = 0; nb < NBR; ++nb) m_ref[nb] = max_over_rows(mx[nb]) + kExtHeadroom;
+    if (k == 5) {
+      mx = max_over_halves(mx) * c2;
+      const bool over = mx > m_ref + kExtSlack;
+      mn = over ? mx + kExtHeadroom : m_ref;
+      need = __builtin_amdgcn_ballot_w64(over);
+      f = __builtin_amdgcn_exp2f(m_ref - mn);
+      m_ref = mn;
+      l_run *= f;
     }
-    // rows past the slack: reference to the tile's maximum + 8, O and the sum
-    // scaled by the difference (O's lane holds rows 4 gq + i, whose factors
-    // come from the lanes whose row la is that row)
+    if (k >= kFirst) {
+      const int span = slots - kFirst;
 #pragma unroll
-    for (int nb = 0; nb < NBR; ++nb) {
-      float fj[4] = {1.f, 1.f, 1.f, 1.f};
-      if (need[nb]) {
-        const float mt = max_over_rows(mx[nb]);
-        const float mn = mt > m_ref[nb] + kExtSlack ? mt + kExtHeadroom : m_ref[nb];
-        const float f = __builtin_amdgcn_exp2f(m_ref[nb] - mn);
-        l_run[nb] *= f;
-        m_ref[nb] = mn;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) fj[i] = __shfl(f, 4 * gq + i);
-      }
-      static_assert(ND % 16 == 0, "rescale in groups of 16 column blocks");
-#pragma unroll
-      for (int nd = 0; nd < ND; nd += 16)
-        scale_acc16(*reinterpret_cast<f32x4(*)[16]>(&acc_o[nb][nd]), fj, need[nb]);
-    }
-    u32x4 pf[kExtKH][NBR];
-#pragma unroll
-    for (int kh = 0; kh < kExtKH; ++kh)
-#pragma unroll
-      for (int nb = 0; nb < NBR; ++nb) {
-        float p[2][4];
-#pragma unroll
-        for (int mk = 0; mk < 2; ++mk)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            p[mk][i] = __builtin_amdgcn_exp2f(fmaf(s[2 * kh + mk][nb][i], c2, -m_ref[nb]));  // masked: 0
+      for (int o = (k - kFirst) * kOps / span; o < (k + 1 - kFirst) * kOps / span; ++o) {
+        const int e = o / 6, m = e / 4, d = e % 4;
+        switch (o % 6) {
+          case 0: t0 = fmaf(S[8 * m + 2 * d], c2, -mn); break;
+          case 1: t1 = fmaf(S[8 * m + 2 * d + 1], c2, -mn); break;
+          case 2: t0 = __builtin_amdgcn_exp2f(t0); break;
+          case 3: t1 = __builtin_amdgcn_exp2f(t1); break;
+          case 4:  // the sum of the fp16 probabilities the output MFMA uses, a pair behind
+            if (e > 0) l_run = sum_f16x2_fma(p[(e - 1) / 4][(e - 1) % 4], l_run);
+            break;
+          default: {
+            uint32_t pk = pack_f16(t0, t1);
+            asm volatile("" : "+v"(pk));  // formed here, not where a later unit uses it
+            p[m][d] = pk;
           }
-        pf[kh][nb] = u32x4{pack_f16(p[0][0], p[0][1]), pack_f16(p[0][2], p[0][3]), pack_f16(p[1][0], p[1][1]),
-                           pack_f16(p[1][2], p[1][3])};
-        // the row sum of the fp16 probabilities the output MFMA uses
-#pragma unroll
-        for (int d = 0; d < 4; ++d) l_run[nb] = sum_f16x2(pf[kh][nb][d], l_run[nb]);
+        }
       }
+      if (k == slots - 1) l_run = sum_f16x2_fma(p[1][3], l_run);
+    }
+  };
+  auto rescale = [&]() {
+#pragma unroll
+    for (int nd = 0; nd < ND; nd += 8) scale_acc32x8(*reinterpret_cast<f32x16(*)[8]>(&O[nd]), f, need);
+  };
+  // this wave's copies of the next tile have landed (those of one more tile
+  // may be in flight) and its LDS reads are done; then every wave's
+  auto meet = [&]() {
+    asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto buf = [&](int i) { return (const uint8_t*)s_buf + (i % G::NBUF) * G::TILE; };
 
-    // ---- O[row, d] += P . V --------------------------------------------------
+  asm volatile("s_waitcnt vmcnt(18)" ::: "memory");  // tile 0
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+
+  auto nothing = [](int) {};
+  if constexpr (D == 256) {
+    // Units u of 32 keys, two per tile. During unit u the matrix cores run
+    // S_{u+1} and O += V_{u-1} P_{u-1} while the VALU turns S_u into P_u.
+    constexpr int kSlots = kAllK + kAllV;
+    f32x16 S0, S1;
+    u32x4 P0[2], P1[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
 #pragma unroll
-    for (int kh = 0; kh < kExtKH; ++kh)
+    for (int k = 0; k < kAhead; ++k) kfetch(buf(0), 2 * k);
+    score_phase(S0, buf(0), buf(0), nothing);
+    settle(S0);
 #pragma unroll
-      for (int nd = 0; nd < ND; ++nd) {
-        const uint8_t* kv = kb + 32 * kh * G::KSTR;
-        const u32x2 v0 = read_v_tr(kv, G::KSTR, gq, la, nd, 0), v1 = read_v_tr(kv, G::KSTR, gq, la, nd, 1);
-        const u32x4 vf = {v0.x, v0.y, v1.x, v1.y};
+    for (int k = 0; k < kAhead; ++k) kfetch(buf(0) + 32 * RB, 2 * k);
+    int t = 0;
+    do {
+      const uint8_t* const kb = buf(t);
+      // the first pass has no output pending: zero probabilities on tile 0
+      const uint8_t* const vb = buf(t > 0 ? t - 1 : 0) + 32 * RB;
+      const uint8_t* const kn = buf(t + 1);
+      // ---- unit 2t: S_{2t+1} from tile t, V_{2t-1} from tile t - 1 ----
+      mask(S0, KT * t);
+      __builtin_amdgcn_sched_barrier(0);
+      score_phase(S1, kb + 32 * RB, vb, [&](int k) { softmax_slice(S0, P0, k, kSlots); });
+      output_phase(P1, vb, kn, true, [&](int k) { softmax_slice(S0, P0, kAllK + k, kSlots); }, meet);
+      rescale();
+      // ---- unit 2t + 1: S_{2t+2} from tile t + 1 (after the last tile: not used), V_{2t} from tile t ----
+      mask(S1, KT * t + 32);
+      clamp_rows(t + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      score_phase(S0, kn, kb, [&](int k) {
+        softmax_slice(S1, P1, k, kSlots);
+        if (k % 6 == 1) copy_part(t + 3, k / 6);
+      });
+      output_phase(P0, kb, kn + 32 * RB, false, [&](int k) { softmax_slice(S1, P1, kAllK + k, kSlots); }, meet);
+      rescale();
+    } while (++t < n);
+    const uint8_t* const vb = buf(n - 1) + 32 * RB;
 #pragma unroll
-        for (int nb = 0; nb < NBR; ++nb) acc_o[nb][nd] = mfma16x16x32_f16(pf[kh][nb], vf, acc_o[nb][nd]);
+    for (int k = 0; k < kAhead; ++k) vfetch(vb, 2 * k);
+    output_phase(P1, vb, vb, false, nothing, meet);
+  } else {
+    // One 32-key unit per tile, and no registers for a second S: during step
+    // i the matrix cores run S_i, then O += V_{i-1} P_{i-1} while the VALU
+    // turns S_i into P_i.
+    f32x16 S;
+    u32x4 P[2], pn[2];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) kfetch(buf(0), 2 * k);
+    score_phase(S, buf(0), buf(0), nothing);
+    settle(S);
+    mask(S, 0);
+#pragma unroll
+    for (int k = 0; k < kAllV; ++k) softmax_slice(S, P, k, kAllV);
+    meet();
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) kfetch(buf(1), 2 * k);
+    for (int i = 1; i <= n; ++i) {
+      const uint8_t* const vb = buf(i - 1);
+      if (i < n) {
+        clamp_rows(i + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        score_phase(S, buf(i), vb, [&](int k) {
+          if (k % 12 == 1) copy_part(i + 2, k / 12);
+        });
+        settle(S);
+        mask(S, KT * i);
+      } else {
+        // after the last step: its output alone
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) vfetch(vb, 2 * k);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) S[j] = -__builtin_inff();
       }
-
-    // ---- tile it + TPB into the buffer of tile it - TPB ---------------------
-    if (it + TPB < ntiles) store_keys(s_buf + ((it + TPB) % NBUF) * G::BUF);
-    if (it % TPB == TPB - 1 || it + 1 == ntiles) __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+      output_phase(P, vb, buf(i + 1), true, [&](int k) { softmax_slice(S, pn, k, kAllV); }, meet);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) P[m] = pn[m];
+      rescale();
+    }
   }
+
+  // no copy may outlive the block's LDS
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- normalise and store -----------------------------------------------------
+  const float l = add_over_halves(l_run);
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  const int64_t r = r0 + RW * wave + la32;
+  const bool ok = r < nrows;
+  uint16_t* const dst = a.out + (qo0 + (ok ? r / a.H : 0)) * a.o_st + (ok ? r % a.H : 0) * a.o_sh;
 #pragma unroll
-  for (int nb = 0; nb < NBR; ++nb) {
-    const float l = add_over_rows(l_run[nb]);
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+  for (int nd = 0; nd < ND; ++nd) {
+    uint32_t w[4][2];  // columns 32 nd + 8 q + 4 g + (0..3)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float ii = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (4 * gq + i), __float_as_int(inv)));
-      const int64_t r = r0 + RW * wave + 16 * nb + 4 * gq + i;
-      if (r >= nrows) continue;
-      const int64_t t = r / a.H, h = r % a.H;
-      uint16_t* dst = a.out + (qo0 + t) * a.o_st + h * a.o_sh + la;
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int nd = 0; nd < ND; ++nd) dst[16 * nd] = float_to_bf16(acc_o[nb][nd][i] * ii);
+      for (int k = 0; k < 2; ++k) w[q][k] = pack_bf16(O[nd][4 * q + 2 * k] * inv, O[nd][4 * q + 2 * k + 1] * inv);
+    if (a.o_vec) {
+      // the halves' pieces joined to 8 consecutive columns per lane: columns
+      // 32 nd + 16 p + 8 g + (0..7)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const auto x = __builtin_amdgcn_permlane32_swap(w[2 * p][0], w[2 * p + 1][0], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(w[2 * p][1], w[2 * p + 1][1], false, false);
+        if (ok) *reinterpret_cast<u32x4*>(dst + 32 * nd + 16 * p + 8 * g) = u32x4{x[0], y[0], x[1], y[1]};
+      }
+    } else if (ok) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          dst[32 * nd + 8 * q + 4 * g + 2 * k] = (uint16_t)w[q][k];
+          dst[32 * nd + 8 * q + 4 * g + 2 * k + 1] = (uint16_t)(w[q][k] >> 16);
+        }
     }
   }
 }
 
 }  // namespace rolaq
 
-hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& a, int D, int R, int max_q_len, hipStream_t stream) {
+hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& args, int D, int R, int max_q_len, hipStream_t stream) {
   using namespace rolaq;
+  ExtendArgs a = args;
+  // 16-byte output stores where the rows allow them
+  a.o_vec = (reinterpret_cast<uintptr_t>(a.out) % 16) == 0 && a.o_st % 8 == 0 && a.o_sh % 8 == 0;
 #define ROLAQ_EXT(DD, RR)                                                                               \
   if (D == DD && R == RR) {                                                                             \
     using G = ExtGeo<DD, RR>;                                                                           \
     const int64_t rows = (int64_t)max_q_len * a.H;                                                      \
     const dim3 grid((unsigned)a.B, (unsigned)((rows + G::BM - 1) / G::BM));                             \
-    const int lds = G::NBUF * G::BUF;                                                                         \
+    const int lds = G::NBUF * G::TILE;                                                                  \
     const hipError_t e = hipFuncSetAttribute((const void*)extend_kernel<DD, RR>,                        \
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);          \
     if (e != hipSuccess) return e;                                                                      \

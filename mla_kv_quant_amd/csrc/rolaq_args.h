@@ -93,6 +93,7 @@ struct ExtendArgs {
   int64_t ws_rows;
   uint16_t* out;            // [T, H, D] bf16, strides (o_st, o_sh)
   int64_t o_st, o_sh;
+  int o_vec;                // output rows allow 16-byte stores (set by the launcher)
 };
 
 struct AssembleArgs {

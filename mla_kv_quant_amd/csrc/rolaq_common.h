@@ -8,6 +8,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -33,6 +34,14 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ f32x4 mfma16x16x32_f16(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
+                                                0, 0);
+}
+
+// D = A(32x16) * B(16x32) + C on fp16 inputs, fp32 accumulate. Lane l holds
+// A[l%32][8(l/32)+i], B[8(l/32)+i][l%32] (i = 0..7, two per dword, low half
+// first) and C[8(j/4) + 4(l/32) + j%4][l%32] (j = 0..15).
+__device__ __forceinline__ f32x16 mfma32x32x16_f16(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
                                                 0, 0);
 }
 
@@ -228,11 +237,105 @@ __device__ __forceinline__ void scale_acc16(f32x4 (&o)[16], const float (&f)[4],
       : "scc");
 }
 
+// The same in-place scaling for the 16-register accumulators of the 32x32
+// MFMAs (AGPR tuples a[b:b+15]), all by one factor per lane.
+#define ROLAQ_ACC_CASE(k, k15) "  .ifc \\t, a[" #k ":" #k15 "]\n    .set rolaq_acc_b, " #k "\n  .endif\n"
+#define ROLAQ_ACC32_CASES \
+  ROLAQ_ACC_CASE(0, 15) ROLAQ_ACC_CASE(2, 17) ROLAQ_ACC_CASE(4, 19) ROLAQ_ACC_CASE(6, 21) ROLAQ_ACC_CASE(8, 23) ROLAQ_ACC_CASE(10, 25) \
+  ROLAQ_ACC_CASE(12, 27) ROLAQ_ACC_CASE(14, 29) ROLAQ_ACC_CASE(16, 31) ROLAQ_ACC_CASE(18, 33) ROLAQ_ACC_CASE(20, 35) ROLAQ_ACC_CASE(22, 37) \
+  ROLAQ_ACC_CASE(24, 39) ROLAQ_ACC_CASE(26, 41) ROLAQ_ACC_CASE(28, 43) ROLAQ_ACC_CASE(30, 45) ROLAQ_ACC_CASE(32, 47) ROLAQ_ACC_CASE(34, 49) \
+  ROLAQ_ACC_CASE(36, 51) ROLAQ_ACC_CASE(38, 53) ROLAQ_ACC_CASE(40, 55) ROLAQ_ACC_CASE(42, 57) ROLAQ_ACC_CASE(44, 59) ROLAQ_ACC_CASE(46, 61) \
+  ROLAQ_ACC_CASE(48, 63) ROLAQ_ACC_CASE(50, 65) ROLAQ_ACC_CASE(52, 67) ROLAQ_ACC_CASE(54, 69) ROLAQ_ACC_CASE(56, 71) ROLAQ_ACC_CASE(58, 73) \
+  ROLAQ_ACC_CASE(60, 75) ROLAQ_ACC_CASE(62, 77) ROLAQ_ACC_CASE(64, 79) ROLAQ_ACC_CASE(66, 81) ROLAQ_ACC_CASE(68, 83) ROLAQ_ACC_CASE(70, 85) \
+  ROLAQ_ACC_CASE(72, 87) ROLAQ_ACC_CASE(74, 89) ROLAQ_ACC_CASE(76, 91) ROLAQ_ACC_CASE(78, 93) ROLAQ_ACC_CASE(80, 95) ROLAQ_ACC_CASE(82, 97) \
+  ROLAQ_ACC_CASE(84, 99) ROLAQ_ACC_CASE(86, 101) ROLAQ_ACC_CASE(88, 103) ROLAQ_ACC_CASE(90, 105) ROLAQ_ACC_CASE(92, 107) ROLAQ_ACC_CASE(94, 109) \
+  ROLAQ_ACC_CASE(96, 111) ROLAQ_ACC_CASE(98, 113) ROLAQ_ACC_CASE(100, 115) ROLAQ_ACC_CASE(102, 117) ROLAQ_ACC_CASE(104, 119) ROLAQ_ACC_CASE(106, 121) \
+  ROLAQ_ACC_CASE(108, 123) ROLAQ_ACC_CASE(110, 125) ROLAQ_ACC_CASE(112, 127) ROLAQ_ACC_CASE(114, 129) ROLAQ_ACC_CASE(116, 131) ROLAQ_ACC_CASE(118, 133) \
+  ROLAQ_ACC_CASE(120, 135) ROLAQ_ACC_CASE(122, 137) ROLAQ_ACC_CASE(124, 139) ROLAQ_ACC_CASE(126, 141) ROLAQ_ACC_CASE(128, 143) ROLAQ_ACC_CASE(130, 145) \
+  ROLAQ_ACC_CASE(132, 147) ROLAQ_ACC_CASE(134, 149) ROLAQ_ACC_CASE(136, 151) ROLAQ_ACC_CASE(138, 153) ROLAQ_ACC_CASE(140, 155) ROLAQ_ACC_CASE(142, 157) \
+  ROLAQ_ACC_CASE(144, 159) ROLAQ_ACC_CASE(146, 161) ROLAQ_ACC_CASE(148, 163) ROLAQ_ACC_CASE(150, 165) ROLAQ_ACC_CASE(152, 167) ROLAQ_ACC_CASE(154, 169) \
+  ROLAQ_ACC_CASE(156, 171) ROLAQ_ACC_CASE(158, 173) ROLAQ_ACC_CASE(160, 175) ROLAQ_ACC_CASE(162, 177) ROLAQ_ACC_CASE(164, 179) ROLAQ_ACC_CASE(166, 181) \
+  ROLAQ_ACC_CASE(168, 183) ROLAQ_ACC_CASE(170, 185) ROLAQ_ACC_CASE(172, 187) ROLAQ_ACC_CASE(174, 189) ROLAQ_ACC_CASE(176, 191) ROLAQ_ACC_CASE(178, 193) \
+  ROLAQ_ACC_CASE(180, 195) ROLAQ_ACC_CASE(182, 197) ROLAQ_ACC_CASE(184, 199) ROLAQ_ACC_CASE(186, 201) ROLAQ_ACC_CASE(188, 203) ROLAQ_ACC_CASE(190, 205) \
+  ROLAQ_ACC_CASE(192, 207) ROLAQ_ACC_CASE(194, 209) ROLAQ_ACC_CASE(196, 211) ROLAQ_ACC_CASE(198, 213) ROLAQ_ACC_CASE(200, 215) ROLAQ_ACC_CASE(202, 217) \
+  ROLAQ_ACC_CASE(204, 219) ROLAQ_ACC_CASE(206, 221) ROLAQ_ACC_CASE(208, 223) ROLAQ_ACC_CASE(210, 225) ROLAQ_ACC_CASE(212, 227) ROLAQ_ACC_CASE(214, 229) \
+  ROLAQ_ACC_CASE(216, 231) ROLAQ_ACC_CASE(218, 233) ROLAQ_ACC_CASE(220, 235) ROLAQ_ACC_CASE(222, 237) ROLAQ_ACC_CASE(224, 239) ROLAQ_ACC_CASE(226, 241) \
+  ROLAQ_ACC_CASE(228, 243) ROLAQ_ACC_CASE(230, 245) ROLAQ_ACC_CASE(232, 247) ROLAQ_ACC_CASE(234, 249) ROLAQ_ACC_CASE(236, 251) ROLAQ_ACC_CASE(238, 253) \
+  ROLAQ_ACC_CASE(240, 255)
+__device__ __forceinline__ void define_acc32_macros() {
+  asm volatile(
+    ".ifndef rolaq_acc32_macros\n"
+    ".set rolaq_acc32_macros, 1\n"
+    ".macro ROLAQ_ACC32_SCALE t, t0, t1, t2, t3, f\n"
+    "  .set rolaq_acc_b, -1\n" ROLAQ_ACC32_CASES
+    "  .if rolaq_acc_b < 0\n"
+    "    .error \"ROLAQ_ACC32_SCALE: not an AGPR tuple\"\n"
+    "  .endif\n"
+    "  .set rolaq_acc_i, rolaq_acc_b\n"
+    "  .rept 4\n"
+    "    v_accvgpr_read_b32 \\t0, a[rolaq_acc_i]\n"
+    "    v_accvgpr_read_b32 \\t1, a[rolaq_acc_i+1]\n"
+    "    v_accvgpr_read_b32 \\t2, a[rolaq_acc_i+2]\n"
+    "    v_accvgpr_read_b32 \\t3, a[rolaq_acc_i+3]\n"
+    "    s_nop 1\n"
+    "    v_mul_f32_e32 \\t0, \\t0, \\f\n"
+    "    v_mul_f32_e32 \\t1, \\t1, \\f\n"
+    "    v_mul_f32_e32 \\t2, \\t2, \\f\n"
+    "    v_mul_f32_e32 \\t3, \\t3, \\f\n"
+    "    s_nop 1\n"
+    "    v_accvgpr_write_b32 a[rolaq_acc_i], \\t0\n"
+    "    v_accvgpr_write_b32 a[rolaq_acc_i+1], \\t1\n"
+    "    v_accvgpr_write_b32 a[rolaq_acc_i+2], \\t2\n"
+    "    v_accvgpr_write_b32 a[rolaq_acc_i+3], \\t3\n"
+    "    .set rolaq_acc_i, rolaq_acc_i+4\n"
+    "  .endr\n"
+    ".endm\n"
+    ".endif\n");
+}
+#undef ROLAQ_ACC32_CASES
+#undef ROLAQ_ACC_CASE
+
+// Eight such accumulators times f when need (a lane mask) is not 0; the
+// leading waits cover the longest 32x32 MFMA writing them just before.
+__device__ __forceinline__ void scale_acc32x8(f32x16 (&o)[8], float f, uint64_t need) {
+  float t0, t1, t2, t3;
+  asm volatile(
+      "s_cmp_lg_u64 %13, 0\n\t"
+      "s_cbranch_scc0 1f\n\t"
+      "s_nop 7\n\ts_nop 7\n\ts_nop 7\n\t"
+      "ROLAQ_ACC32_SCALE %0, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %1, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %2, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %3, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %4, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %5, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %6, %8, %9, %10, %11, %12\n\t"
+      "ROLAQ_ACC32_SCALE %7, %8, %9, %10, %11, %12\n\t"
+      "s_nop 7\n"
+      "1:"
+      : "+a"(o[0]), "+a"(o[1]), "+a"(o[2]), "+a"(o[3]), "+a"(o[4]), "+a"(o[5]), "+a"(o[6]), "+a"(o[7]),
+        "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+      : "v"(f), "s"(need)
+      : "scc");
+}
+
 // acc + lo + hi of a packed pair of fp16 values (exact products by one,
 // FP32 accumulation: v_dot2_f32_f16)
 __device__ __forceinline__ float sum_f16x2(uint32_t v, float acc) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, v), h2{(_Float16)1.0f, (_Float16)1.0f}, acc, false);
+}
+
+// The same sum with two mixed-precision FMAs by one, for use behind 32x32
+// MFMAs: v_dot2 runs on the matrix pipe, where it waits for the MFMA in flight
+// and holds up the next one (a 32x32x16 MFMA with four v_dot2 behind it: 27.5
+// ns; with four FMAs: 16).
+__device__ __forceinline__ float sum_f16x2_fma(uint32_t v, float acc) {
+  asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+      : "+v"(acc)
+      : "v"(v));
+  return acc;
 }
 
 // all-ones when keep, else zero: a branch-free "keep ? v : 0" on bit patterns

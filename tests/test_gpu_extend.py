@@ -317,3 +317,35 @@ def test_extend_output_independent_of_page_layout(D, R, H):
     assert torch.isfinite(outs[0].float()).all()
     for o in outs[1:]:
         assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
+
+
+@pytest.mark.parametrize("D,R,H", [(512, 64, 16), (256, 32, 16), (256, 32, 40)])
+def test_extend_at_the_edges_of_rows_and_tiles(D, R, H):
+    """Query rows around a block's 128 and a wave's 32 (1, 8, 9 and 17 tokens),
+    keys around the 32- and 64-key tiles and the ring of four (1 .. 321), and an
+    output whose row stride forbids 16-byte stores: same bits as the aligned
+    one. Tolerance: the readers' bar (bf16 outputs, fp16 probabilities)."""
+    prefixes = [0, 0, 0, 24, 25, 55, 56, 57, 120, 121, 250, 304]
+    chunks = [1, 8, 33, 8, 8, 8, 8, 8, 8, 9, 17, 17]
+    P, W, page = 4, 16, 16
+    sm = 1.0 / math.sqrt(96 if D == 256 else 192)
+    pool, slots, pages, reqs, rot = build_pool(prefixes, D, R, P, W, page, seed=29)
+    gp = pool_to_gpu(pool)
+    T = sum(chunks)
+    q = synth.make_normal((T, H, D + R), 30, std=2.0 / (sm * math.sqrt(D + R)))
+    kc = torch.cat([rotated_latent(T, D, 3, 31, rot), synth.make_normal((T, R), 32)], 1)
+    qo = np.concatenate([[0], np.cumsum(chunks)]).astype(np.int32)
+    indptr, indices = index_lists(slots, pages, page)
+    outs = [torch.full((T, H, D), float("nan"), dtype=torch.bfloat16, device=DEV),
+            torch.full((T, H * D + 4), float("nan"), dtype=torch.bfloat16, device=DEV)[:, 4:].unflatten(1, (H, D))]
+    for out in outs:
+        kernels.extend_fwd(q.to(DEV), kc.to(DEV), torch.from_numpy(qo).to(DEV), indptr, indices,
+                           torch.tensor(prefixes, device=DEV), torch.tensor(reqs, dtype=torch.int64, device=DEV),
+                           gp["codes"], gp["params"], gp["rope"], gp["hp"], max(chunks), out, sm, P, W, page)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].contiguous().view(torch.int16))
+    for b in range(len(prefixes)):
+        s, e = qo[b], qo[b + 1]
+        ref, _ = attention.extend(pool, q[s:e, :, :D], q[s:e, :, D:], kc[s:e, :D], kc[s:e, D:], slots[b],
+                                  prefixes[b], int(reqs[b]), P, W, sm, D, dtype=torch.float64)
+        torch.testing.assert_close(outs[0][s:e].double().cpu(), ref, rtol=RTOL, atol=ATOL)
