@@ -245,6 +245,11 @@ int rolaq_decode_merge(const float* attn_logits, const float* attn_lse, const in
  * shorter than key_rows is rejected (ROLAQ_ERR_INVALID, nothing launched).
  * Rows past workspace_rows are never written; a sequence whose rows do not
  * fit (key_rows short of the device-side sum) gets NaN outputs.
+ * A workspace longer than key_rows by at least what rolaq_extend_scratch_rows
+ * returns lets the call split the keys of a block of query rows over several
+ * compute units (FP32 partials and their merge, in the workspace's last rows):
+ * short chunks over long prefixes and ragged batches are much faster with it.
+ * The results differ by FP32 summation order only.
  * Latent values are carried in fp16 as for rolaq_decode_fwd.
  */
 int rolaq_extend_fwd(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_chunk,
@@ -254,6 +259,14 @@ int rolaq_extend_fwd(const void* q, int64_t q_stride_t, int64_t q_stride_h, cons
                      const void* rope_buf, const void* hp_c, int B, int H, int D, int R, int P, int W,
                      int max_q_len, float sm_scale, void* workspace, int64_t workspace_rows, int64_t key_rows,
                      void* out, int64_t out_stride_t, int64_t out_stride_h, void* stream);
+
+/*
+ * Workspace rows past key_rows with which rolaq_extend_fwd splits keys on the
+ * current device, written to *rows (0: it would not split). At most
+ * 2 * compute units * 128 * D * 4 bytes of partials and a few hundred KB. Host
+ * only: no launch, no synchronisation. No counterpart in the reference.
+ */
+int rolaq_extend_scratch_rows(int B, int H, int D, int R, int max_q_len, int64_t key_rows, int64_t* rows);
 
 /*
  * Cache rows as bf16 [latent | rope] rows (MHA-style prefill over a packed

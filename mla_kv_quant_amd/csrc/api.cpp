@@ -406,6 +406,15 @@ int rolaq_decode_merge(const float* attn_logits, const float* attn_lse, const in
                     "decode_merge launch");
 }
 
+int rolaq_extend_scratch_rows(int B, int H, int D, int R, int max_q_len, int64_t key_rows, int64_t* rows) {
+  if (B < 0 || H <= 0 || H > 4096 || max_q_len < 0 || key_rows < 0 || !((D == 256 && R == 32) || (D == 512 && R == 64)) ||
+      !rows)
+    return fail(ROLAQ_ERR_INVALID, "extend_scratch_rows: invalid B, H, (D, R), max_q_len, key_rows or null rows");
+  *rows = B == 0 || max_q_len == 0 ? 0 : rolaq_extend_plan_rows(B, H, D, R, max_q_len, key_rows, cu_count());
+  g_err[0] = '\0';
+  return ROLAQ_OK;
+}
+
 int rolaq_extend_fwd(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_chunk,
                      int64_t kc_stride_t, const int32_t* qo_indptr, const int32_t* kv_indptr,
                      const int32_t* kv_indices, int page_size, const int64_t* prefix_lens,
@@ -468,7 +477,8 @@ int rolaq_extend_fwd(const void* q, int64_t q_stride_t, int64_t q_stride_h, cons
   a.out = static_cast<uint16_t*>(out);
   a.o_st = out_stride_t;
   a.o_sh = out_stride_h;
-  return hip_status(rolaq_launch_extend(a, D, R, max_q_len, static_cast<hipStream_t>(stream)), "extend_fwd launch");
+  return hip_status(rolaq_launch_extend(a, D, R, max_q_len, key_rows, cu_count(), static_cast<hipStream_t>(stream)),
+                    "extend_fwd launch");
 }
 
 int rolaq_assemble_rows(const int64_t* slots, int64_t n, const uint8_t* codes, const float* params,

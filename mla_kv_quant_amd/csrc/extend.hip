@@ -9,7 +9,7 @@
 // W positions of the extended sequence, which are the BF16 window rows; the
 // chunk's rows enter as the given BF16 keys; attention is causal.
 //
-// Layout of the work: two launches.
+// Layout of the work: two launches, or three where the keys are split.
 //   gather  every key row of the extended sequences -- [latent | rope], INT2
 //           rows dequantized and rounded to bf16 once -- into the caller's
 //           workspace as fp16 (the same numbers: a bf16 value is exact in fp16
@@ -35,6 +35,7 @@
 #include "rolaq_common.h"
 #include "rolaq_args.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rolaq {
@@ -103,20 +104,298 @@ __device__ __forceinline__ float add_over_halves(float v) {
   return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
-// Workspace row of key 0 of sequence b.
-__device__ __forceinline__ int64_t key_offset(const ExtendArgs& a, int b) {
-  int64_t off = 0;
-  for (int i = 0; i < b; ++i) off += a.prefix_lens[i] + (a.qo_indptr[i + 1] - a.qo_indptr[i]);
-  return off;
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uniform(int64_t v) {
+  return (int64_t)((uint64_t)(uint32_t)uniform((int)v) | (uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32);
+}
+
+// ---------------------------------------------------------------------------
+// Splitting the keys. Where the blocks of 128 query rows alone would leave
+// CUs idle (a short chunk over a long prefix) or end unevenly (ragged
+// batches), a block's keys are split over several work items, whose FP32
+// partials and LSE go to scratch and are merged by a third launch. The plan
+// needs the lengths, which only the device has: one block of the gather
+// launch makes it, in the shadow of the others, and writes it to the scratch:
+// the end of the caller's workspace past the key rows, when it is long enough
+// (rolaq_extend_scratch_rows). Without it the blocks take whole sequences.
+// Measured without -> with: 96 queries over 12345 keys, 16 heads, D = 512: 580
+// -> 80 us (gather 10, attend 53, merge 14); six ragged chunks: 443 -> 424 us.
+// ---------------------------------------------------------------------------
+struct ExtItem {        // 64 bytes: all that a block of the attend launch starts from
+  int64_t r0, nrows;    // first query row (token * H + head) in the sequence, the sequence's rows
+  int64_t koff;         // workspace row of the sequence's key 0
+  int32_t qo0, prefix;
+  int32_t s0, s1;       // steps of KT keys (s0 == s1: nothing to do)
+  int32_t slot;         // partial slot, or -1: the block writes the output
+  int32_t pad[5];
+};
+struct ExtMerge {       // 32 bytes: a block of query rows and its partials
+  int64_t r0, nrows;
+  int32_t qo0, slot0, n, pad;  // n < 2: nothing to merge
+};
+struct ExtHead {
+  int32_t items, merges;  // items < 0: no plan
+  int32_t pad[62];
+};
+constexpr int kExtRows = 128;    // query rows per item
+constexpr int kExtMinSteps = 4;  // least steps worth an item of its own
+
+struct ExtScratch {
+  ExtHead* head;
+  ExtItem* items;
+  ExtMerge* merges;
+  float* lse;  // [slots, 128], log2 domain
+  float* o;    // [slots, 128 * D], in the attend kernel's lane order
+};
+__host__ __device__ inline ExtScratch ext_scratch(uint8_t* base, int items, int slots) {
+  ExtScratch x;
+  x.head = reinterpret_cast<ExtHead*>(base);
+  x.items = reinterpret_cast<ExtItem*>(base + sizeof(ExtHead));
+  x.merges = reinterpret_cast<ExtMerge*>(x.items + items);
+  x.lse = reinterpret_cast<float*>(x.merges + (slots + 1) / 2 * 2);
+  x.o = x.lse + (int64_t)slots * kExtRows;
+  return x;
+}
+
+// Sum over the wave, the same on every lane: DPP scans within rows of 16, the
+// rows' totals broadcast (VALU only; as 64-bit shuffles this was 24 dependent
+// LDS permutes on the way to every block's first load).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int64_t add_dpp(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xF, false);
+  return v + (int64_t)((uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ int64_t wave_sum64(int64_t v) {
+  v = add_dpp<0x111, 0xF>(v);  // row_shr 1, 2, 4, 8: lane 15 of a row has its total
+  v = add_dpp<0x112, 0xF>(v);
+  v = add_dpp<0x114, 0xF>(v);
+  v = add_dpp<0x118, 0xF>(v);
+  v = add_dpp<0x142, 0xA>(v);  // lane 15 of rows 0 and 2 to rows 1 and 3
+  v = add_dpp<0x143, 0xC>(v);  // lane 31 to rows 2 and 3
+  const uint32_t lo = __builtin_amdgcn_readlane((int)v, 63), hi = __builtin_amdgcn_readlane((int)(v >> 32), 63);
+  return (int64_t)((uint64_t)hi << 32 | lo);
+}
+// Workspace row of key 0 of sequence b and the key rows of all sequences
+// (every lane of a wave takes part).
+__device__ __forceinline__ void key_rows(const ExtendArgs& a, int b, int64_t* koff, int64_t* total) {
+  int64_t before = 0, all = 0;
+  for (int i = threadIdx.x & 63; i < a.B; i += 64) {
+    const int64_t n = a.prefix_lens[i] + (a.qo_indptr[i + 1] - a.qo_indptr[i]);
+    before += i < b ? n : 0;
+    all += n;
+  }
+  *koff = wave_sum64(before);
+  *total = wave_sum64(all);
+}
+
+// Whether the key rows end before the scratch. If they do not (the caller
+// stated fewer than there are) the gather writes them over it, so nothing in it
+// is read: every kernel asks this itself.
+__device__ __forceinline__ bool scratch_is_free(const ExtendArgs& a) {
+  int64_t koff, total;
+  key_rows(a, 0, &koff, &total);
+  return uniform(total) <= a.ws_rows - a.scratch_rows;
+}
+
+// The plan. Items are the 128-row blocks of every sequence, the keys of all
+// blocks of one sequence cut at the same multiples of a chunk of at most KC
+// steps. KC is the best of 32 candidates, one per lane -- multiples of a CU's
+// equal share of all steps, fractions of the longest sequence, no cut -- by an
+// estimate: steps per CU, plus an item's start and end, plus the partials'
+// traffic. Longer chunks go first; a sequence's items are ordered so that the
+// same chunk of its blocks lands on one XCD (blocks go to the 8 XCDs
+// round-robin), whose L2 then serves its key rows. The block's latency is the
+// gather's where there is little to gather, so every step is spread over
+// lanes (a first version with one thread per sequence took 20 us).
+template <int D, int R>
+__device__ void extend_plan(const ExtendArgs& a) {
+  constexpr int KT = D == 256 ? 64 : 32;
+  constexpr int kCands = 32, kShares = 16;
+  __shared__ unsigned long long s_work, s_keys, s_n[kCands], s_slots[kCands];
+  __shared__ int s_longest, s_mx[kCands];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const ExtScratch x = ext_scratch(a.scratch, a.max_items, a.max_slots);
+  if (tid == 0) s_work = 0, s_keys = 0, s_longest = 0;
+  if (tid < kCands) s_n[tid] = 0, s_slots[tid] = 0, s_mx[tid] = 0;
+  __syncthreads();
+  struct Shape {
+    int64_t prefix, rows, keys;
+    int blocks, steps;  // blocks of rows; steps of the last one
+  };
+  auto shape = [&](int b) {
+    const int64_t q = a.qo_indptr[b + 1] - a.qo_indptr[b];
+    Shape s;
+    s.prefix = a.prefix_lens[b];
+    s.keys = s.prefix + q;
+    s.rows = q > 0 ? q * a.H : 0;
+    s.blocks = (int)((s.rows + kExtRows - 1) / kExtRows);
+    s.steps = s.blocks ? (int)((s.keys + KT - 1) / KT) : 0;
+    return s;
+  };
+  // rows 0 .. r of a sequence see keys below this many steps
+  auto steps_of = [&](const Shape& s, int64_t r) {
+    r = min(r, s.rows - 1);
+    const int64_t t = s.rows < (1ll << 31) ? (int64_t)((uint32_t)r / (uint32_t)a.H) : r / a.H;
+    return (int)((s.prefix + t) / KT) + 1;
+  };
+  {
+    int64_t work = 0, keys = 0;
+    int longest = 0;
+    for (int b = tid; b < a.B; b += blockDim.x) {
+      const Shape s = shape(b);
+      keys += s.keys;
+      if (s.blocks) work += (int64_t)s.blocks * (steps_of(s, kExtRows - 1) + s.steps) / 2;
+      longest = max(longest, s.steps);
+    }
+    if (wave * 64 < a.B) {
+      work = wave_sum64(work);
+      keys = wave_sum64(keys);
+      if (lane == 0) atomicAdd(&s_work, (unsigned long long)work), atomicAdd(&s_keys, (unsigned long long)keys);
+      atomicMax(&s_longest, longest);
+    }
+  }
+  __syncthreads();
+  const int longest = s_longest;
+  const float work = (float)s_work, share = work / a.cus;
+  // candidate c's KC, and the chunks of a sequence for it: count, steps of each
+  auto chunk_of = [&](int c) {
+    const int kc = c < kShares ? (int)fminf(ceilf(share * __builtin_amdgcn_exp2f(0.2f * (c - 9))), 1.0e9f)
+                               : (longest + (c - kShares + 1)) / (c - kShares + 2);
+    return c == kCands - 1 ? (1 << 30) : max(kExtMinSteps, kc);
+  };
+  auto cut = [](int steps, int kc, int& n, int& len) {
+    n = (int)(((uint32_t)steps + (uint32_t)kc - 1) / (uint32_t)kc);
+    len = n > 1 ? (int)(((uint32_t)steps + (uint32_t)n - 1) / (uint32_t)n) : steps;
+  };
+  {
+    const int c = tid % kCands, kc = chunk_of(c);
+    unsigned long long n_all = 0, slots = 0;
+    int mx = 0;
+    for (int b = tid / kCands; b < a.B; b += blockDim.x / kCands) {
+      const Shape s = shape(b);
+      if (s.blocks == 0) continue;
+      int n, len;
+      cut(s.steps, kc, n, len);
+      n_all += (unsigned long long)s.blocks * n;
+      if (n > 1) slots += (unsigned long long)s.blocks * n;
+      mx = max(mx, len);
+    }
+    if (tid / kCands < a.B) {
+      atomicAdd(&s_n[c], n_all);
+      atomicAdd(&s_slots[c], slots);
+      atomicMax(&s_mx[c], mx);
+    }
+  }
+  __syncthreads();
+  if ((int64_t)s_keys > a.ws_rows - a.scratch_rows) return;  // key rows lie in the scratch: nothing is written there
+  // chunks longer than the stated bound: the launch's blocks go without a plan
+  if (s_n[kCands - 1] > (unsigned long long)a.max_items) {
+    if (tid == 0) x.head->items = -1, x.head->merges = 0;
+    return;
+  }
+  int pick, mx;
+  {
+    constexpr float kItem = 5.f;                       // an item's start and end, in steps
+    constexpr float kSlot = D == 512 ? 0.065f : 0.033f;  // a partial written and merged
+    const int c = lane % kCands;
+    const unsigned long long n = s_n[c], sl = s_slots[c];
+    const int m = s_mx[c];
+    float t = n <= (unsigned long long)a.cus ? m + kItem : (work + n * kItem) / a.cus + 0.5f * m;
+    t += kSlot * sl + (sl ? 4.f : 0.f);
+    if (sl > (unsigned long long)a.max_slots || n > (unsigned long long)a.max_items) t = 3.0e38f;
+    pick = c;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {
+      const float t2 = __shfl_xor(t, o);
+      const int p2 = __shfl_xor(pick, o);
+      if (t2 < t || (t2 == t && p2 > pick)) t = t2, pick = p2;
+    }
+    mx = s_mx[pick];
+  }
+  const int kc = chunk_of(pick);
+  // A sequence's items, partials and merges start behind those of the
+  // sequences before it, the ones with long chunks first; each is written by
+  // one wave, or by several where there are fewer sequences than waves.
+  const int waves = blockDim.x / 64, share_w = a.B < waves ? waves / a.B : 1;
+  for (int b = wave / share_w; b < a.B; b += waves / share_w) {
+    int64_t items = 0, slots = 0, merges = 0, koff = 0;  // of the sequences before b (koff: in batch order)
+    int n, len;
+    const Shape s = shape(b);
+    cut(s.steps, kc, n, len);
+    const bool late = 4 * len < 3 * mx;
+    for (int i = lane; i < a.B; i += 64) {
+      const Shape si = shape(i);
+      int ni, li;
+      cut(si.steps, kc, ni, li);
+      const bool late_i = 4 * li < 3 * mx;
+      const bool before = late_i == late ? i < b : late;
+      if (before) {
+        items += (int64_t)si.blocks * ni;
+        if (ni > 1) slots += (int64_t)si.blocks * ni, merges += si.blocks;
+      }
+      if (i < b) koff += si.keys;
+    }
+    const int base = (int)wave_sum64(items), slot = (int)wave_sum64(slots), mrg = (int)wave_sum64(merges);
+    koff = wave_sum64(koff);
+    const int32_t qo0 = a.qo_indptr[b];
+    const int sub = wave % share_w;
+    for (int j = lane + 64 * sub; j < s.blocks * n; j += 64 * share_w) {
+      // item j: chunks in groups of 8 (fewer at the end), blocks in turn within a group
+      const int group = j / (8 * s.blocks), width = min(8, n - 8 * group), k = j - 8 * s.blocks * group;
+      const int c = 8 * group + k % width, blk = s.blocks - 1 - k / width;  // later blocks first
+      ExtItem it;
+      it.r0 = (int64_t)blk * kExtRows;
+      it.nrows = s.rows;
+      it.koff = koff;
+      it.qo0 = qo0;
+      it.prefix = (int32_t)s.prefix;
+      const int end = steps_of(s, it.r0 + kExtRows - 1);  // the block's own steps
+      it.s0 = min(c * len, end);
+      it.s1 = min((c + 1) * len, end);
+      it.slot = end > len ? slot + blk * n + c : -1;
+      x.items[base + j] = it;
+    }
+    if (n > 1)
+      for (int blk = lane + 64 * sub; blk < s.blocks; blk += 64 * share_w) {
+        ExtMerge m;
+        m.r0 = (int64_t)blk * kExtRows;
+        m.nrows = s.rows;
+        m.qo0 = qo0;
+        m.slot0 = slot + blk * n;
+        m.n = (steps_of(s, m.r0 + kExtRows - 1) + len - 1) / len;
+        x.merges[mrg + blk] = m;
+      }
+  }
+  if (wave == waves - 1) {
+    int64_t merges = 0;
+    for (int i = lane; i < a.B; i += 64) {
+      const Shape si = shape(i);
+      int ni, li;
+      cut(si.steps, kc, ni, li);
+      if (ni > 1) merges += si.blocks;
+    }
+    merges = wave_sum64(merges);
+    if (lane == 0) x.head->items = (int)s_n[pick], x.head->merges = (int)merges;
+  }
 }
 
 // Key rows of sequence blockIdx.x as fp16 (one thread per 16-byte chunk, rows
 // strided over blockIdx.y): chunk rows from k_chunk, prefix rows from the BF16
 // window (t < P or t >= L - W of the extended length L) or the INT2 row
-// ((code - zero) * scale rounded to bf16), rope from rope_buf.
+// ((code - zero) * scale rounded to bf16), rope from rope_buf. With scratch,
+// block (0, 0) makes the plan instead.
 template <int D, int R>
 __global__ __launch_bounds__(256) void extend_gather_kernel(ExtendArgs a) {
   constexpr int DR = D + R, CPR = DR / 8, NG = D / 128;
+  int y = blockIdx.y, ny = gridDim.y;
+  if (a.scratch) {
+    if (y == 0) {
+      if (blockIdx.x == 0) extend_plan<D, R>(a);
+      return;
+    }
+    --y, --ny;
+  }
   const int b = blockIdx.x;
   const int64_t qo0 = a.qo_indptr[b];
   const int64_t Tq = a.qo_indptr[b + 1] - qo0;
@@ -125,11 +404,12 @@ __global__ __launch_bounds__(256) void extend_gather_kernel(ExtendArgs a) {
   const int64_t req = a.req_idx[b];
   const bool ring = req >= 0 && req < a.max_reqs;
   const int P = ring ? a.P : 0, W = ring ? a.W : 0;
-  const int64_t koff = key_offset(a, b);
+  int64_t koff, total;
+  key_rows(a, b, &koff, &total);
   const int64_t kv0 = a.kv_indptr[b];
   const int pmask = (1 << a.page_shift) - 1;
   const int64_t n = min(L, a.ws_rows - koff) * CPR;
-  for (int64_t e = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.y * blockDim.x) {
+  for (int64_t e = (int64_t)y * blockDim.x + threadIdx.x; e < n; e += (int64_t)ny * blockDim.x) {
     const int64_t t = e / CPR;
     const int c = (int)(e - t * CPR);
     u32x4 v;
@@ -166,10 +446,10 @@ __global__ __launch_bounds__(256) void extend_gather_kernel(ExtendArgs a) {
 // work sits behind MFMAs, in whose shadow it is free: a 32x32x16 MFMA alone
 // takes 14 to 15 ns, with six VALU operations behind it 16.
 // Measured, before -> after: 4 x 2048 queries over 14336 keys, 40 heads, D =
-// 256: 5.42 -> 4.47 ms (1.22 PFLOP/s, 3108 cycles per 64 keys and wave, of
+// 256: 5.42 -> 4.52 ms (1.21 PFLOP/s, 3108 cycles per 64 keys and wave, of
 // which 2176 are MFMAs, at 1.62 GHz: the clock falls with the matrix cores'
-// power); six ragged chunks, 16 heads, D = 512: 1.04 -> 0.43 ms; 96 queries
-// over 12345 keys: 0.89 -> 0.58 ms.
+// power); six ragged chunks, 16 heads, D = 512: 1.06 -> 0.44 ms; 96 queries
+// over 12345 keys: 0.89 -> 0.58 ms (both with whole sequences per block).
 //
 // A lane holds one query row (column la32 of the MFMAs): its scores, its
 // reference, its sum and its outputs, so nothing crosses lanes but the two
@@ -189,34 +469,93 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   define_acc32_macros();
   extern __shared__ __attribute__((aligned(16))) uint8_t s_buf[];
 
-  const int b = blockIdx.x;
-  const int64_t qo0 = a.qo_indptr[b];
-  const int64_t Tq = a.qo_indptr[b + 1] - qo0;
-  // heavier blocks (later tokens) first
-  const int64_t r0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * BM;
-  const int64_t nrows = Tq * a.H;
-  if (r0 >= nrows) return;
-  const int64_t prefix = a.prefix_lens[b];
-  const int64_t L = prefix + Tq;
-  const int64_t koff = key_offset(a, b);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, la32 = lane & 31;
-  if (koff + L > a.ws_rows) {
-    // the sequence's key rows did not fit the workspace: its outputs are NaN
-    for (int64_t e = tid; e < (int64_t)BM * D; e += 64 * G::WAVES) {
-      const int64_t r = r0 + e / D;
-      if (r < nrows) a.out[(qo0 + r / a.H) * a.o_st + (r % a.H) * a.o_sh + e % D] = 0x7FC0;
-    }
-    return;
+
+  // ---- the work item: from the plan, or block (sequence, rows) with all keys ---
+  ExtScratch x{};
+  ExtItem it;
+  bool planned = a.scratch != nullptr;
+  if (planned) {
+    x = ext_scratch(a.scratch, a.max_items, a.max_slots);
+    const int items = x.head->items;
+    it = x.items[blockIdx.x];  // (within the array, whether planned or not)
+    planned = scratch_is_free(a) && items >= 0;
+    if (planned && ((int)blockIdx.x >= items || it.s0 >= it.s1)) return;
   }
-  // last query token of the block -> keys 0 .. prefix + t_last
-  const int64_t t_last = min(nrows - 1, r0 + BM - 1) / a.H;
-  const int kend = (int)(prefix + t_last + 1);
+  if (!planned) {
+    // heavier blocks (later tokens) first
+    const int b = blockIdx.x % a.B, y = a.row_blocks - 1 - blockIdx.x / a.B;
+    if (y < 0) return;
+    it.qo0 = a.qo_indptr[b];
+    const int64_t Tq = a.qo_indptr[b + 1] - it.qo0;
+    it.r0 = (int64_t)y * BM;
+    it.nrows = Tq * a.H;
+    if (it.r0 >= it.nrows) return;
+    it.prefix = (int)a.prefix_lens[b];
+    int64_t total;
+    key_rows(a, b, &it.koff, &total);
+    if (it.koff + it.prefix + Tq > a.ws_rows) {
+      // the sequence's key rows did not fit the workspace: its outputs are NaN
+      for (int64_t e = tid; e < (int64_t)BM * D; e += 64 * G::WAVES) {
+        const int64_t r = it.r0 + e / D;
+        if (r < it.nrows) a.out[(it.qo0 + r / a.H) * a.o_st + (r % a.H) * a.o_sh + e % D] = 0x7FC0;
+      }
+      return;
+    }
+    it.s0 = 0;
+    it.s1 = 1 << 30;
+    it.slot = -1;
+  }
+  // (the same on every lane, kept in scalar registers)
+  const int64_t r0 = uniform(it.r0), nrows = uniform(it.nrows), qo0 = uniform(it.qo0), prefix = uniform(it.prefix);
+  const int s0 = uniform(it.s0), s1 = uniform(it.s1), slot = uniform(it.slot);
+  // the block's first and last query token, within the sequence; keys are
+  // counted from the item's first one on
+  const int64_t t_first = uniform(r0 / a.H), t_last = uniform(min(nrows - 1, r0 + BM - 1) / a.H);
+  const int key0 = s0 * KT;
+  const int64_t koff = uniform(it.koff) + key0;
+  const int kend = (int)min(prefix + t_last + 1, (int64_t)s1 * KT) - key0;
   const int n = (kend + KT - 1) / KT;  // steps
 
-  // ---- tile copies: this wave's rows of a tile, 16-byte chunk 64 j + lane ------
+  // ---- query rows of this wave ------------------------------------------------
+  // the lane's row of the sequence (whether there is one), token and head
+  struct Row {
+    bool ok;
+    int64_t t;
+    int h;
+  };
+  auto row_of = [&](int lane32) {
+    const int rest = (int)(r0 - t_first * a.H) + RW * wave + lane32;  // from the first token's head 0
+    Row r{r0 + RW * wave + lane32 < nrows, t_first, 0};
+    if (r.ok) r.t += rest / a.H, r.h = rest % a.H;
+    return r;
+  };
+  // They are copied to LDS as whole rows (like a key tile, into ring buffers
+  // without a tile yet) and read back as Q^T fragments: read from memory in
+  // the fragments' layout each load would touch 32 rows, which took most of a
+  // 20,000-cycle start.
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)s_buf;
+  constexpr int kQBuf = D == 512 ? 0 : 2;  // the last 128 rows' worth of buffers
+  int qp;                                  // causal limit of the lane's row (-2^30: no row)
+  {
+    const Row r = row_of(la32);
+    qp = r.ok ? (int)(prefix + r.t) - key0 : -(1 << 30);
+    const int64_t mine = reinterpret_cast<int64_t>(a.q + (qo0 + r.t) * a.q_st + r.h * a.q_sh);
+#pragma unroll
+    for (int j = 0; j < RW * CPR / 64; ++j) {
+      const int ci = 64 * j + lane, row = ci / CPR, pc = ci - row * CPR;
+      const uint64_t src = (uint64_t)__shfl(mine, row) + 16 * (pc ^ ext_sw<D>(row));
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                   ::"s"(lds0 + kQBuf * G::TILE + RW * RB * wave + 1024 * j), "v"(src)
+                   : "memory", "m0");
+    }
+  }
+  const float c2 = a.sm_scale * kLog2e;
+  const int qfirst = (int)(prefix + t_first) - key0;  // causal limit of the block's first row
+
+  // ---- tile copies: this wave's rows of a tile, 16-byte chunk 64 j + lane ------
   // byte offset of the chunk from kBias bytes before the wave's first row, less
   // the 1024 (j % 4) that the copy's own offset adds (kBias keeps the
   // unsigned offsets from wrapping, also when clamp_rows moves them to row 0)
@@ -227,9 +566,7 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
     const int ci = 64 * j + lane, row = ci / CPR, pc = ci - row * CPR;
     doff[j] = kBias + row * RB + 16 * (pc ^ ext_sw<D>(G::WROWS * wave + row)) - 1024 * (j % 4);
   }
-  const uint64_t keys_v = reinterpret_cast<uint64_t>(a.ws) + (uint64_t)koff * RB - kBias;
-  const uint64_t keys = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)keys_v) |
-                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(keys_v >> 32)) << 32;
+  const uint64_t keys = reinterpret_cast<uint64_t>(a.ws) + (uint64_t)koff * RB - kBias;
   // Third p of the copies of tile i. Rows past the block's last key read that
   // key again: they are masked (clamp_rows(i) comes before the parts). In
   // place of tiles past the last one that one is copied again, to buffers that
@@ -254,28 +591,15 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
     else
       copy_to_lds(src, doff[8], dst);
   };
-#pragma unroll
-  for (int t = 0; t < 3; ++t) {
+  auto first_tile = [&](int t) {
     clamp_rows(t);
 #pragma unroll
     for (int p = 0; p < 3; ++p) copy_part(t, p);
+  };
+  if constexpr (kQBuf == 2) {
+    first_tile(0);
+    first_tile(1);
   }
-
-  // ---- query rows of this wave: Q^T fragments (fp16) and causal limits --------
-  u32x4 qf[KSQ];
-  int qp;  // causal limit of the lane's row (-1: no row)
-  {
-    const int64_t r = r0 + RW * wave + la32;
-    const bool ok = r < nrows;
-    const int64_t t = ok ? r / a.H : 0, h = ok ? r % a.H : 0;
-    qp = ok ? (int)(prefix + t) : -1;
-    const uint16_t* qr = a.q + (qo0 + t) * a.q_st + h * a.q_sh + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < KSQ; ++ks)
-      qf[ks] = ok ? bf16x8_to_f16x8(gload<u32x4>(qr + 16 * ks)) : u32x4{0u, 0u, 0u, 0u};
-  }
-  const float c2 = a.sm_scale * kLog2e;
-  const int qfirst = (int)(prefix + r0 / a.H);  // causal limit of the block's first row
 
   // ---- LDS read addresses: a few lane bases plus immediate offsets ------------
   // score operand of K-step ks: row la32 of the unit's 32 keys, chunk 2 ks + g
@@ -303,6 +627,26 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   auto kread = [&](const uint8_t* kb, int ks) {
     return *reinterpret_cast<const u32x4*>(kb + kbase[ks % KB] + 32 * KB * (ks / KB));
   };
+  // ---- Q^T fragments (fp16), then the first tiles -----------------------------
+  if constexpr (kQBuf == 2)
+    asm volatile("s_waitcnt vmcnt(18)" ::: "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  u32x4 qf[KSQ];
+#pragma unroll
+  for (int ks = 0; ks < KSQ; ++ks) qf[ks] = kread(s_buf + kQBuf * G::TILE + RW * RB * wave, ks);
+#pragma unroll
+  for (int ks = 0; ks < KSQ; ++ks) {
+    qf[ks] = bf16x8_to_f16x8(qf[ks]) & keep_mask(qp >= -(1 << 29));
+    asm volatile("" : "+v"(qf[ks])::"memory");
+  }
+  __builtin_amdgcn_s_barrier();  // every wave has its fragments: the buffers are free
+  asm volatile("" ::: "memory");
+  if constexpr (kQBuf == 0) {
+    first_tile(0);
+    first_tile(1);
+  }
+  first_tile(2);
   auto vread = [&](const uint8_t* vb, int m, int nd) {
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -419,10 +763,10 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   };
   // keys past a row's causal limit (only in units that reach past the block's
   // first row): -inf, so that a row without any key in the unit adds nothing
-  auto mask = [&](f32x16& S, int key0) {
-    if (__builtin_expect(key0 + 31 > qfirst, 0)) {
+  auto mask = [&](f32x16& S, int key) {
+    if (__builtin_expect(key + 31 > qfirst, 0)) {
       asm volatile("");  // a branch, not selects in every unit
-      const int lim = qp < 0 ? -1 : qp - key0 - 4 * g;
+      const int lim = qp - key - 4 * g;
 #pragma unroll
       for (int j = 0; j < 16; ++j) S[j] = 8 * (j / 4) + j % 4 <= lim ? S[j] : -__builtin_inff();
     }
@@ -436,7 +780,9 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   float mx, f, mn, t0, t1;
   uint64_t need;
   auto softmax_slice = [&](const f32x16& S, u32x4 (&p)[2], int k, int slots) {
-    constexpr int kFirst = 6, kOps = 48;
+    // (at D = 512 the first half's probabilities take the place of those that
+    // the first half of the output MFMAs has used)
+    constexpr int kFirst = D == 512 ? 16 : 6, kOps = 48;
     if (k >= 1 && k <= 4) {
 #pragma unroll
       for (int e = 4 * (k - 1); e < 4 * k; ++e) mx = e == 0 ? S[0] : fmaxf(mx, S[e]);
@@ -535,7 +881,7 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
     // i the matrix cores run S_i, then O += V_{i-1} P_{i-1} while the VALU
     // turns S_i into P_i.
     f32x16 S;
-    u32x4 P[2], pn[2];
+    u32x4 P[2];
 #pragma unroll
     for (int k = 0; k < kAhead; ++k) kfetch(buf(0), 2 * k);
     score_phase(S, buf(0), buf(0), nothing);
@@ -564,6 +910,7 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
         for (int j = 0; j < 16; ++j) S[j] = -__builtin_inff();
       }
       __builtin_amdgcn_sched_barrier(0);
+      u32x4 pn[2];
       output_phase(P, vb, buf(i + 1), true, [&](int k) { softmax_slice(S, pn, k, kAllV); }, meet);
 #pragma unroll
       for (int m = 0; m < 2; ++m) P[m] = pn[m];
@@ -575,11 +922,30 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- normalise and store -----------------------------------------------------
+  // the lane's place again: kept since the start, it would take registers
+  // from the loop, and a spilled one's reload would wait for the stores
+  int lane_now;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_now));
+  const int ge = lane_now >> 5;
   const float l = add_over_halves(l_run);
   const float inv = l > 0.f ? 1.0f / l : 0.f;
-  const int64_t r = r0 + RW * wave + la32;
-  const bool ok = r < nrows;
-  uint16_t* const dst = a.out + (qo0 + (ok ? r / a.H : 0)) * a.o_st + (ok ? r % a.H : 0) * a.o_sh;
+  if (slot >= 0) {
+    // a partial: FP32, 16 bytes per lane in the accumulators' order (whole
+    // kilobytes per store), and the rows' LSE (log2 domain)
+    f32x4* const po = reinterpret_cast<f32x4*>(x.o) + ((int64_t)slot * G::WAVES + wave) * ND * 4 * 64 + lane_now;
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        po[(4 * nd + q) * 64] = f32x4{O[nd][4 * q] * inv, O[nd][4 * q + 1] * inv, O[nd][4 * q + 2] * inv,
+                                      O[nd][4 * q + 3] * inv};
+    if (ge == 0)
+      x.lse[(int64_t)slot * BM + RW * wave + lane_now] = l == 0.f ? kExtNoRef : m_ref + __log2f(l);
+    return;
+  }
+  const Row r = row_of(lane_now & 31);
+  const bool ok = r.ok;
+  uint16_t* const dst = a.out + (qo0 + r.t) * a.o_st + r.h * a.o_sh + 4 * ge;
 #pragma unroll
   for (int nd = 0; nd < ND; ++nd) {
     uint32_t w[4][2];  // columns 32 nd + 8 q + 4 g + (0..3)
@@ -594,38 +960,144 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
       for (int p = 0; p < 2; ++p) {
         const auto x = __builtin_amdgcn_permlane32_swap(w[2 * p][0], w[2 * p + 1][0], false, false);
         const auto y = __builtin_amdgcn_permlane32_swap(w[2 * p][1], w[2 * p + 1][1], false, false);
-        if (ok) *reinterpret_cast<u32x4*>(dst + 32 * nd + 16 * p + 8 * g) = u32x4{x[0], y[0], x[1], y[1]};
+        if (ok) *reinterpret_cast<u32x4*>(dst + 32 * nd + 16 * p + 4 * ge) = u32x4{x[0], y[0], x[1], y[1]};
       }
     } else if (ok) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-          dst[32 * nd + 8 * q + 4 * g + 2 * k] = (uint16_t)w[q][k];
-          dst[32 * nd + 8 * q + 4 * g + 2 * k + 1] = (uint16_t)(w[q][k] >> 16);
+          dst[32 * nd + 8 * q + 2 * k] = (uint16_t)w[q][k];
+          dst[32 * nd + 8 * q + 2 * k + 1] = (uint16_t)(w[q][k] >> 16);
         }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Merge of a plan's partials: out = sum_c 2^(lse_c - M) O_c / sum_c 2^(lse_c - M)
+// in FP32, to bf16. A thread takes four columns of a row; what it reads of a
+// partial is 16 bytes of a whole kilobyte per wave.
+// ---------------------------------------------------------------------------
+template <int D, int R>
+__global__ __launch_bounds__(256) void extend_merge_kernel(ExtendArgs a) {
+  using G = ExtGeo<D, R>;
+  constexpr int ND = G::ND, PARTS = D / 8;  // 256-thread parts of a block of rows
+  const ExtScratch x = ext_scratch(a.scratch, a.max_items, a.max_slots);
+  const int entries = (a.max_slots + 1) / 2;
+  const bool free = scratch_is_free(a);
+  for (int u = blockIdx.x; u < entries * PARTS; u += gridDim.x) {
+    // (the entry is read with the count, not after it)
+    const ExtMerge m = x.merges[u / PARTS];
+    if (!free || u >= x.head->merges * PARTS) return;
+    if (m.n < 2) continue;
+    const int e = (u % PARTS) * 256 + threadIdx.x;
+    const int lane = e & 63, q = (e >> 6) & 3, nd = (e >> 8) % ND, w = e / (256 * ND);
+    const int row = G::RW * w + (lane & 31);
+    if (m.r0 + row >= m.nrows) continue;
+    const float* lse = x.lse + (int64_t)m.slot0 * G::BM + row;
+    const f32x4* po = reinterpret_cast<const f32x4*>(x.o) + (int64_t)m.slot0 * G::BM * D / 4 + e;
+    float M = kExtNoRef, den = 0.f;
+    for (int c = 0; c < m.n; ++c) M = fmaxf(M, lse[(int64_t)c * G::BM]);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int c = 0; c < m.n; ++c) {
+      const float wt = __builtin_amdgcn_exp2f(lse[(int64_t)c * G::BM] - M);
+      den += wt;
+      acc += wt * po[(int64_t)c * G::BM * D / 4];
+    }
+    const float inv = 1.f / den;
+    const int64_t t = (m.r0 + row) / a.H, h = (m.r0 + row) % a.H;
+    uint16_t* dst = a.out + (m.qo0 + t) * a.o_st + h * a.o_sh + 32 * nd + 8 * q + 4 * (lane >> 5);
+    const u32x2 v = {pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv)};
+    if (a.o_vec) {
+      *reinterpret_cast<u32x2*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[i] = (uint16_t)(v[i / 2] >> (16 * (i % 2)));
     }
   }
 }
 
 }  // namespace rolaq
 
-hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& args, int D, int R, int max_q_len, hipStream_t stream) {
+namespace {
+
+struct ExtPlanSize {
+  int row_blocks;  // blocks of query rows of the longest possible chunk
+  int items, slots;
+  int64_t rows;    // workspace rows of the scratch, 0: no plan
+};
+
+// What a plan may need at most, from what the host knows: the chunk lengths'
+// bound and the sum of all key rows.
+ExtPlanSize extend_plan_size(int B, int H, int D, int R, int max_q_len, int64_t key_rows, int num_cus) {
+  using namespace rolaq;
+  ExtPlanSize p{};
+  const int64_t kt = D == 256 ? 64 : 32;
+  const int64_t rb = ((int64_t)max_q_len * H + kExtRows - 1) / kExtRows;
+  p.row_blocks = (int)rb;
+  // A plan pays where some sequence has many steps: its block of the gather
+  // launch, the merge launch and the partials take about as long as 12 steps
+  // (one sequence of 250 keys: 36 us with a plan, 28 without; 2000 keys: 41
+  // and 72). The longest one is taken to be no longer than twice the mean.
+  // With a block for every CU anyway it can only shorten the end, by half of
+  // that sequence's steps at most (5 x 550 queries over 80 keys, 20 heads: 57
+  // us with a plan, 51 without).
+  const int64_t longest = std::min(key_rows, 2 * ((key_rows + B - 1) / std::max(B, 1)));
+  if (longest < (rb * B < num_cus ? 24 : 64) * kt) return p;
+  // Slots: at most two per CU (a plan of more would only add partials), and no
+  // more than chunks of the least length make
+  const int64_t chunks = ((key_rows + kt - 1) / kt + kExtMinSteps - 1) / kExtMinSteps;
+  const int64_t slots = std::min<int64_t>(2 * (int64_t)num_cus, rb * B * chunks);
+  if (slots < 2 || chunks < 2 || rb * B > (1 << 20)) return p;
+  p.slots = (int)slots;
+  p.items = (int)(rb * B + slots);
+  const ExtScratch x = ext_scratch(nullptr, p.items, p.slots);
+  const int64_t bytes = reinterpret_cast<intptr_t>(x.o) + (int64_t)p.slots * kExtRows * D * 4;
+  p.rows = (bytes + 2 * (D + R) - 1) / (2 * (D + R));
+  return p;
+}
+
+}  // namespace
+
+int64_t rolaq_extend_plan_rows(int B, int H, int D, int R, int max_q_len, int64_t key_rows, int num_cus) {
+  return extend_plan_size(B, H, D, R, max_q_len, key_rows, num_cus).rows;
+}
+
+hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& args, int D, int R, int max_q_len, int64_t key_rows,
+                               int num_cus, hipStream_t stream) {
   using namespace rolaq;
   ExtendArgs a = args;
   // 16-byte output stores where the rows allow them
   a.o_vec = (reinterpret_cast<uintptr_t>(a.out) % 16) == 0 && a.o_st % 8 == 0 && a.o_sh % 8 == 0;
+  const ExtPlanSize p = extend_plan_size(a.B, a.H, D, R, max_q_len, key_rows, num_cus);
+  a.row_blocks = p.row_blocks;
+  a.cus = num_cus;
+  int64_t blocks = (int64_t)p.row_blocks * a.B;
+  if (p.rows > 0 && a.ws_rows - key_rows >= p.rows) {
+    a.scratch = reinterpret_cast<uint8_t*>(a.ws + (a.ws_rows - p.rows) * (D + R));
+    a.scratch_rows = p.rows;
+    a.max_items = p.items;
+    a.max_slots = p.slots;
+    blocks = p.items;
+  }
+  // gather: about 16 rows per block, 64 blocks per sequence at least (their
+  // lengths may differ) and no more than 2048 in all
+  const int64_t gy = std::min<int64_t>(std::max<int64_t>(64, 2048 / a.B), std::max<int64_t>(1, (key_rows + 15) / 16));
 #define ROLAQ_EXT(DD, RR)                                                                               \
   if (D == DD && R == RR) {                                                                             \
     using G = ExtGeo<DD, RR>;                                                                           \
-    const int64_t rows = (int64_t)max_q_len * a.H;                                                      \
-    const dim3 grid((unsigned)a.B, (unsigned)((rows + G::BM - 1) / G::BM));                             \
+    static_assert(G::BM == kExtRows, "rows per item");                                                  \
     const int lds = G::NBUF * G::TILE;                                                                  \
     const hipError_t e = hipFuncSetAttribute((const void*)extend_kernel<DD, RR>,                        \
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);          \
     if (e != hipSuccess) return e;                                                                      \
-    hipLaunchKernelGGL((extend_gather_kernel<DD, RR>), dim3((unsigned)a.B, 64), dim3(256), 0, stream, a); \
-    hipLaunchKernelGGL((extend_kernel<DD, RR>), grid, dim3(64 * G::WAVES), lds, stream, a);             \
+    hipLaunchKernelGGL((extend_gather_kernel<DD, RR>), dim3((unsigned)a.B, (unsigned)(gy + (a.scratch ? 1 : 0))), \
+                       dim3(256), 0, stream, a);                                                        \
+    hipLaunchKernelGGL((extend_kernel<DD, RR>), dim3((unsigned)blocks), dim3(64 * G::WAVES), lds, stream, a); \
+    if (a.scratch)                                                                                      \
+      hipLaunchKernelGGL((extend_merge_kernel<DD, RR>), dim3(16 * (unsigned)num_cus), dim3(256), 0, stream, a); \
     return hipGetLastError();                                                                           \
   }
   ROLAQ_EXT(256, 32)

@@ -93,7 +93,13 @@ struct ExtendArgs {
   int64_t ws_rows;
   uint16_t* out;            // [T, H, D] bf16, strides (o_st, o_sh)
   int64_t o_st, o_sh;
-  int o_vec;                // output rows allow 16-byte stores (set by the launcher)
+  // set by the launcher
+  int o_vec;                // output rows allow 16-byte stores
+  int row_blocks;           // blocks of query rows of a chunk of the largest length
+  int cus;
+  uint8_t* scratch;         // the end of the workspace: the plan and its partials, or null
+  int64_t scratch_rows;     // workspace rows it takes
+  int max_items, max_slots;
 };
 
 struct AssembleArgs {
@@ -133,5 +139,8 @@ hipError_t rolaq_launch_pack_bf16_aux(const uint16_t* x, int64_t xs, const int64
 hipError_t rolaq_launch_prepare_splits(const int32_t* splits, int32_t* quant, int32_t* merge, int64_t n,
                                        hipStream_t stream);
 hipError_t rolaq_launch_writer(const rolaq::WriterArgs& a, int D, int num_cus, hipStream_t stream);
-hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& a, int D, int R, int max_q_len, hipStream_t stream);
+hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& a, int D, int R, int max_q_len, int64_t key_rows, int num_cus,
+                               hipStream_t stream);
+// Workspace rows past the key rows with which the extend launch splits keys.
+int64_t rolaq_extend_plan_rows(int B, int H, int D, int R, int max_q_len, int64_t key_rows, int num_cus);
 hipError_t rolaq_launch_assemble(const rolaq::AssembleArgs& a, int D, hipStream_t stream);

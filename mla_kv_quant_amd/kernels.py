@@ -302,6 +302,16 @@ def decode_merge(attn_logits: torch.Tensor, attn_lse: torch.Tensor, num_kv_split
     return out
 
 
+def extend_scratch_rows(B: int, H: int, D: int, R: int, max_q_len: int, key_rows: int) -> int:
+    """Workspace rows past the key rows with which :func:`extend_fwd` splits
+    keys over compute units (0: it would not)."""
+    if key_rows < 24 * 32:  # too few for any split
+        return 0
+    rows = ctypes.c_int64(0)
+    _lib.check(_lib.load().rolaq_extend_scratch_rows(B, H, D, R, int(max_q_len), int(key_rows), ctypes.byref(rows)))
+    return rows.value
+
+
 def extend_fwd(q: torch.Tensor, k_chunk: torch.Tensor, qo_indptr: torch.Tensor, kv_indptr: torch.Tensor,
                kv_indices: torch.Tensor, prefix_lens: torch.Tensor, req_idx: torch.Tensor, codes: torch.Tensor,
                params: torch.Tensor, rope_buf: torch.Tensor, hp_c: torch.Tensor, max_q_len: int,
@@ -316,7 +326,8 @@ def extend_fwd(q: torch.Tensor, k_chunk: torch.Tensor, qo_indptr: torch.Tensor, 
     count); read back from the device when not given (one host sync).
     ``workspace``: 16-bit ``[rows, D + R]`` scratch (bf16 or fp16 storage;
     fp16 values are written into it) with ``rows >= key_rows``, allocated
-    here when not given; a shorter one raises ``ValueError``."""
+    here when not given; a shorter one raises ``ValueError``. With
+    :func:`extend_scratch_rows` more rows the call may split keys."""
     dev = q.device
     _need(q, "q", torch.bfloat16, dev, 3)
     T, H, DR = q.shape
@@ -350,7 +361,8 @@ def extend_fwd(q: torch.Tensor, k_chunk: torch.Tensor, qo_indptr: torch.Tensor, 
     if key_rows is None:
         key_rows = int(prefix_lens[:B].sum().item()) + int(qo_indptr[B].item()) - int(qo_indptr[0].item())
     if workspace is None:
-        workspace = torch.empty(max(int(key_rows), 1), DR, dtype=torch.float16, device=dev)
+        extra = extend_scratch_rows(B, H, D, R, max_q_len, key_rows)
+        workspace = torch.empty(max(int(key_rows) + extra, 1), DR, dtype=torch.float16, device=dev)
     if workspace.dtype not in (torch.bfloat16, torch.float16) or workspace.device != dev or workspace.dim() != 2:
         raise TypeError("workspace must be a 2-D bf16 or fp16 tensor on the query's device")
     _contig(workspace, "workspace")

@@ -349,3 +349,55 @@ def test_extend_at_the_edges_of_rows_and_tiles(D, R, H):
         ref, _ = attention.extend(pool, q[s:e, :, :D], q[s:e, :, D:], kc[s:e, :D], kc[s:e, D:], slots[b],
                                   prefixes[b], int(reqs[b]), P, W, sm, D, dtype=torch.float64)
         torch.testing.assert_close(outs[0][s:e].double().cpu(), ref, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("D,R,H", [(512, 64, 16), (256, 32, 40)])
+@pytest.mark.parametrize("prefixes,chunks", [
+    ([6000], [9]),                           # one sequence, one or three blocks of rows: many chunks each
+    ([3000, 0, 40, 5000], [1, 300, 30, 64]),  # cut and uncut sequences, a fresh one (causal: blocks of unequal keys)
+    ([2050, 2047, 2048], [17, 16, 16]),       # lengths around the steps' multiples
+    ([800] * 70, [2] * 70),                   # more sequences than the lanes of a wave
+], ids=["one", "mixed", "edges", "many"])
+def test_extend_with_split_keys_matches_unsplit(D, R, H, prefixes, chunks):
+    """A workspace with room for a plan splits keys; the result is that of a
+    workspace without it (whole sequences per block) up to FP32 summation order
+    and the fp16 probabilities' other references: 2^-11 per probability, so
+    outputs of unit variance agree within the readers' bar, and sampled
+    sequences match the oracle at it. A workspace whose spare rows the key rows
+    turn out to need (key_rows understated) gives the unsplit bits."""
+    P, W, page = 4, 16, 16
+    sm = 1.0 / math.sqrt(96 if D == 256 else 192)
+    pool, slots, pages, reqs, rot = build_pool(prefixes, D, R, P, W, page, seed=41)
+    gp = pool_to_gpu(pool)
+    T, B = sum(chunks), len(prefixes)
+    q = synth.make_normal((T, H, D + R), 42, std=2.0 / (sm * math.sqrt(D + R)))
+    kc = torch.cat([rotated_latent(T, D, 3, 43, rot), synth.make_normal((T, R), 44)], 1)
+    qo = np.concatenate([[0], np.cumsum(chunks)]).astype(np.int32)
+    indptr, indices = index_lists(slots, pages, page)
+    rows = sum(prefixes) + T
+    spare = kernels.extend_scratch_rows(B, H, D, R, max(chunks), rows)
+    assert spare > 0
+
+    def run(ws_rows, key_rows):
+        out = torch.full((T, H, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ws = torch.empty(ws_rows, D + R, dtype=torch.float16, device=DEV).fill_(float("nan"))
+        kernels.extend_fwd(q.to(DEV), kc.to(DEV), torch.from_numpy(qo).to(DEV), indptr, indices,
+                           torch.tensor(prefixes, device=DEV), torch.tensor(reqs, dtype=torch.int64, device=DEV),
+                           gp["codes"], gp["params"], gp["rope"], gp["hp"], max(chunks), out, sm, P, W, page,
+                           workspace=ws, key_rows=key_rows)
+        torch.cuda.synchronize()
+        return out
+
+    whole, split = run(rows, rows), run(rows + spare, rows)
+    assert torch.isfinite(split.float()).all()
+    torch.testing.assert_close(split.float(), whole.float(), rtol=RTOL, atol=ATOL)
+    assert not torch.equal(split, whole) or B == 70  # keys were split
+    assert torch.equal(split, run(rows + spare + 999, rows))
+    # one row short of the truth: a plan would need the key rows' last place
+    short = kernels.extend_scratch_rows(B, H, D, R, max(chunks), rows - 1)
+    assert torch.equal(run(rows - 1 + short, rows - 1), whole)
+    for b in sorted({0, B // 2, B - 1}):
+        s, e = qo[b], qo[b + 1]
+        ref, _ = attention.extend(pool, q[s:e, :, :D], q[s:e, :, D:], kc[s:e, :D], kc[s:e, D:], slots[b],
+                                  prefixes[b], int(reqs[b]), P, W, sm, D, dtype=torch.float64)
+        torch.testing.assert_close(split[s:e].double().cpu(), ref, rtol=RTOL, atol=ATOL)
