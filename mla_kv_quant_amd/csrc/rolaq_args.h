@@ -61,6 +61,7 @@ struct WriterArgs {
   int32_t* row_of_slot;
   int32_t* owner_of_row;
   int nstripes;
+  int tile_wave, tile_stripe;  // first tile of wave w of stripe s: w tile_wave + s tile_stripe (set by the launcher)
   int pe_vec;  // k_pe rows copied as dword pairs (set by the launcher)
   // kv_a_layernorm fused in front of the rotation: x is the pre-norm kv_a
   // row, gamma the norm weight [D] (bf16), or null for no norm; y [n, ys]

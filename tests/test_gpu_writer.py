@@ -255,3 +255,52 @@ def test_row_local_batching_is_exact(D, R):
     assert torch.equal(pools[0].hp_row_of_slot, pools[1].hp_row_of_slot)
     assert torch.equal(pools[0].hp_owner_of_row, pools[1].hp_owner_of_row)
     assert int((pools[0].hp_row_of_slot >= 0).sum()) == sum(min(L, P + W) for L in lengths)
+
+
+@pytest.mark.parametrize("norm", [False, True], ids=["plain", "norm"])
+@pytest.mark.parametrize("D,R", [(512, 64), (256, 32)])
+@pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 1023, 4097, 32767, 40961])
+def test_write_does_not_depend_on_the_launch_size(D, R, n, norm):
+    """The launch's size picks how rows are shared out (rows per wave, tiles per
+    block); a row's bytes must not follow it: one launch against slices of 5,
+    64 and 700 rows in turn, in every buffer, window rows and normalized rows
+    included, bit for bit (a row's sums run in one order everywhere)."""
+    from mla_kv_quant_amd import kernels
+
+    P, W, max_reqs, size = 4, 16, 3, n + 70
+    g = torch.Generator().manual_seed(n + D)
+    loc = (torch.randperm(size, generator=g)[:n] + 1).to(DEV)
+    x = synth.make_kv_a(n, D, 7, device=DEV) if norm else synth.make_latent(n, D, 5, seed=7, device=DEV)
+    pe = synth.make_normal((n, R), 8, device=DEV)
+    pos = torch.arange(n, device=DEV)
+    seq = torch.full((n,), n, device=DEV)
+    req = torch.ones(n, dtype=torch.int64, device=DEV)
+    rt = synth.make_rotation(D, 9).to(torch.bfloat16).t().contiguous().to(DEV)
+    gamma = synth.make_norm_weight(D, 10, device=DEV)
+
+    def write(slices):
+        hp_rows = 1 + max_reqs * (P + W)
+        b = {"codes": torch.zeros(size + 1, D // 4, dtype=torch.uint8, device=DEV),
+             "params": torch.zeros(size + 1, D // 128, 2, device=DEV),
+             "rope": torch.zeros(size + 1, R, dtype=torch.bfloat16, device=DEV),
+             "hp": torch.zeros(hp_rows, D, dtype=torch.bfloat16, device=DEV),
+             "row": torch.full((size + 1,), -1, dtype=torch.int32, device=DEV),
+             "owner": torch.zeros(hp_rows, dtype=torch.int32, device=DEV)}
+        y = torch.zeros(n, D, dtype=torch.bfloat16, device=DEV)
+        for s in slices:
+            tail = (b["codes"], b["params"], b["rope"], b["hp"], b["row"], b["owner"], P, W, max_reqs, 0.98, 1.16)
+            if norm:
+                kernels.norm_write_rows(x[s], gamma, 1e-6, y[s], pe[s], rt, loc[s], seq[s], pos[s], req[s], *tail)
+            else:
+                kernels.write_rows(x[s], pe[s], rt, loc[s], seq[s], pos[s], req[s], *tail)
+        torch.cuda.synchronize()
+        return dict(b, y=y)
+
+    cuts, k = [], 0
+    while k < n:
+        for m in (5, 64, 700):
+            cuts.append(slice(k, min(k + m, n)))
+            k = min(k + m, n)
+    whole, parts = write([slice(0, n)]), write([c for c in cuts if c.start < c.stop])
+    for name in whole:
+        assert torch.equal(whole[name].view(torch.uint8), parts[name].view(torch.uint8)), name
