@@ -19,6 +19,7 @@
 #include "rolaq_common.h"
 #include "rolaq_args.h"
 
+#include <algorithm>
 #include <cstddef>
 #include <type_traits>
 
@@ -112,6 +113,103 @@ struct WriterGeo {
   static constexpr int LDS_BYTES = 128 * STRIDE;
   static constexpr int LDS_NORM_BYTES = LDS_BYTES + 2 * D;  // + the norm weight
 };
+
+// The code thresholds -t, 0, t as midpoints (FP64) and tie rules.
+struct CodeTests {
+  double mu_lo, mu_zero, mu_hi;
+  bool incl_lo, incl_hi;
+};
+__device__ __forceinline__ CodeTests code_tests(float thr) {
+  return CodeTests{below_midpoint(-thr), below_midpoint(0.0f), below_midpoint(thr), threshold_inclusive(-thr),
+                   threshold_inclusive(thr)};
+}
+
+// Everything stored for group g of one row, whose rotated values acc(mb)[i]
+// = column 32 gq + 16 (mb / 4) + 4 (mb % 4) + i lie with its four lanes gq (gr:
+// the same number, for the rope piece): statistics, codes, parameters, the
+// window row, rope columns and the ownership maps. acc is overwritten. Both
+// writers end here, so a row's bytes do not depend on which one ran.
+template <int D, typename Acc>
+__device__ __forceinline__ void store_row(const WriterArgs& a, Acc acc, int64_t row, int64_t sl, int32_t p, int32_t sq,
+                                          int32_t rq, u32x2 pe, int g, int gq, int gr, const CodeTests& t) {
+  constexpr int NG = D / 128;
+  // rope columns [16 g, 16 g + 16) of the row, four per lane
+  const bool live = row < a.n;
+  // window bookkeeping (mla_fused_writer.py:36-51)
+  const bool keep = live && ((p < a.P) || (p >= sq - a.W)) && rq < a.max_reqs && rq >= 0 && sl > 0;
+  const int32_t inner = p < a.P ? p : a.P + (p - a.P > 0 ? p - a.P : 0) % (a.W > 0 ? a.W : 1);
+  const int64_t ring = 1 + (int64_t)rq * (a.P + a.W) + inner;
+  if (keep) {
+    // bf16 of the rotated FP32 row (columns 32gq..32gq+31 of group g)
+    uint16_t* hrow = a.hp + ring * D + 128 * g + 32 * gq;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const f32x4 u = acc(2 * h), v = acc(2 * h + 1);
+      const u32x4 pk = {pack_bf16(u[0], u[1]), pack_bf16(u[2], u[3]), pack_bf16(v[0], v[1]),
+                        pack_bf16(v[2], v[3])};
+      *reinterpret_cast<u32x4*>(hrow + 8 * h) = pk;
+    }
+  }
+  // Lloyd statistics over the row's 128 group columns (4 lanes)
+  float s = 0.f;
+#pragma unroll
+  for (int mb = 0; mb < 8; ++mb) s += (acc(mb)[0] + acc(mb)[1]) + (acc(mb)[2] + acc(mb)[3]);
+  s = sum_over_rows(s);
+  const float mean = s * (1.0f / 128.0f);
+  float q = 0.f;
+#pragma unroll
+  for (int mb = 0; mb < 8; ++mb)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      acc(mb)[i] -= mean;
+      q = fmaf(acc(mb)[i], acc(mb)[i], q);
+    }
+  q = sum_over_rows(q);
+  const float std_ = sqrtf(q * (1.0f / 128.0f) + 1e-08f);
+  // code = #{-t, 0, t <= normalized}, normalized = (x - mean) / std, the
+  // correctly rounded FP32 quotient (oscar.py:135-140): compared through
+  // the row's exact thresholds on y = x - mean (no division per element).
+  // Its two bits: high = (y >= y0), low = the parity of the three tests.
+  const double sd = (double)std_;
+  const float ylo = y_threshold(sd, t.mu_lo, t.incl_lo), y0 = y_threshold(sd, t.mu_zero, true),
+              yhi = y_threshold(sd, t.mu_hi, t.incl_hi);
+  uint32_t word[2] = {0u, 0u};
+#pragma unroll
+  for (int wi = 0; wi < 2; ++wi)
+#pragma unroll
+    for (int e = 15; e >= 0; --e) {  // Horner, element e at bits 2e, 2e + 1
+      const float y = acc(4 * wi + e / 4)[e % 4];
+      const uint64_t hi = __builtin_amdgcn_ballot_w64(y >= y0);
+      const uint64_t lo = __builtin_amdgcn_ballot_w64(y >= ylo) ^ hi ^ __builtin_amdgcn_ballot_w64(y >= yhi);
+      word[wi] = twice_plus_bit(twice_plus_bit(word[wi], hi), lo);
+    }
+  if (live) {
+    // words 2gq, 2gq+1 of group g: row words 8g + 2gq, 8g + 2gq + 1
+    *reinterpret_cast<u32x2*>(a.codes + sl * (D / 4) + 4 * (8 * g + 2 * gq)) = u32x2{word[0], word[1]};
+    if (gq == 0) {
+      const float scale = a.kscale * std_;
+      const float zero = kZeroOffset - mean / scale;
+      *reinterpret_cast<f32x2*>(a.params + sl * 2 * NG + 2 * g) = f32x2{scale, zero};
+    }
+    if (sl > 0) {
+      if (a.pe_vec) {
+        // the rope pool's base read again from the kernel arguments here
+        // (a scalar load), not held in a register that would be spilled
+        // (as a global pointer: through a generic one the store is a flat
+        // store, which the next LDS waits would also wait for)
+        typedef __attribute__((address_space(1))) u32x2 g_u32x2;
+        uint16_t* const rope = kernarg_field<uint16_t*>(offsetof(WriterArgs, rope));
+        *(g_u32x2*)(rope + sl * a.R + 16 * g + 4 * gr) = pe;
+      } else if (g == 0) {
+        for (int r = gq; r < a.R; r += 4) a.rope[sl * a.R + r] = a.k_pe[row * a.pe_s0 + r * a.pe_s1];
+      }
+      if (g == 0 && gq == 0) {
+        a.row_of_slot[sl] = keep ? int32_t(ring) : -1;
+        if (keep) a.owner_of_row[ring] = int32_t(sl);
+      }
+    }
+  }
+}
 
 // Block = one quantization group g x a stripe of 64-row tiles. The block's
 // R_g^T slice stays in LDS; its eight waves each own whole tiles and never
@@ -344,10 +442,7 @@ __global__ __launch_bounds__(64 * kWriterWaves, 1) void writer_kernel(WriterArgs
     int lane_now;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_now));
     const int lr = lane_now & 15, gr = lane_now >> 4;
-    // the code thresholds -t, 0, t as midpoints (FP64) and tie rules
-    const float thr = a.thr;
-    const double mu_lo = below_midpoint(-thr), mu_hi = below_midpoint(thr), mu_zero = below_midpoint(0.0f);
-    const bool incl_lo = threshold_inclusive(-thr), incl_hi = threshold_inclusive(thr);
+    const CodeTests t3 = code_tests(a.thr);
     int64_t slot[4];
     int32_t seq[4], pos[4], req[4];
     u32x2 pes[4];
@@ -367,86 +462,116 @@ __global__ __launch_bounds__(64 * kWriterWaves, 1) void writer_kernel(WriterArgs
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       __builtin_amdgcn_sched_barrier(0);
-      const int64_t row = row0 + 16 * nb + lr;
-      // rope columns [16 g, 16 g + 16) of the row, four per lane
-      const u32x2 pe = pes[nb];
-      const bool live = row < a.n;
-      const int64_t sl = slot[nb];
-      // window bookkeeping (mla_fused_writer.py:36-51)
-      const int32_t p = pos[nb], sq = seq[nb], rq = req[nb];
-      const bool keep = live && ((p < a.P) || (p >= sq - a.W)) && rq < a.max_reqs && rq >= 0 && sl > 0;
-      const int32_t inner = p < a.P ? p : a.P + (p - a.P > 0 ? p - a.P : 0) % (a.W > 0 ? a.W : 1);
-      const int64_t ring = 1 + (int64_t)rq * (a.P + a.W) + inner;
-      if (keep) {
-        // bf16 of the rotated FP32 row (columns 32gq..32gq+31 of group g)
-        uint16_t* hrow = a.hp + ring * D + 128 * g + 32 * gq;
+      store_row<D>(a, [&](int mb) -> f32x4& { return acc[mb][nb]; }, row0 + 16 * nb + lr, slot[nb], pos[nb], seq[nb],
+                   req[nb], pes[nb], g, gq, gr, t3);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows (a decode step's batch, short prompts). A block is one group of one
+// 16-row tile: each of its eight waves rotates to 16 of the group's 128 columns
+// with its 16 rows of R_eff^T straight from L2 into registers (one round trip
+// for all K-steps, while writer_kernel first fills 128 KB of LDS and then
+// streams the latent two K-steps at a time), the latent tile is shared
+// through LDS, and one wave ends with all of a row's columns in writer_kernel's
+// lane order. What bounds it is latency: the launch, one round trip to memory,
+// three barriers and one row's epilogue chain. Same products, same order of
+// every sum as writer_kernel: the same bytes. us by launch, before -> after:
+// D = 512: 1 row 13.2 -> 7.4, 1024 rows 14.3 -> 8.1; with the norm 21.6 -> 8.0 and
+// 22.9 -> 8.8; D = 256, 1 row: 10.1 -> 5.3, with the norm 14.3 -> 5.7.
+// ---------------------------------------------------------------------------
+template <int D, bool NORM>
+__global__ __launch_bounds__(64 * kWriterWaves, 1) void writer_few_kernel(WriterArgs a) {
+  constexpr int NG = D / 128, KS = D / 32, KW = KS / kWriterWaves;  // K-steps, and those that a wave loads
+  static_assert(KS % kWriterWaves == 0, "each wave loads whole K-steps");
+  __shared__ u32x4 s_x[KS * 64];           // latent operands, MFMA layout
+  __shared__ f32x4 s_c[kWriterWaves * 64];  // rotated values, by wave
+  __shared__ float s_ss[NORM ? KS * 64 : 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int gq = lane >> 4, la = lane & 15;
+  // (consecutive blocks take the groups in turn: with 2 or 4 of them the blocks
+  // of one XCD share one or two groups' rows of R in its L2)
+  const int g = blockIdx.x % NG;
+  const int64_t ntiles = (a.n + 15) / 16;
+  const CodeTests t3 = code_tests(a.thr);
+  const int32_t* seq32 = reinterpret_cast<const int32_t*>(a.seq_lens);
+  const int32_t* pos32 = reinterpret_cast<const int32_t*>(a.positions ? a.positions : a.seq_lens);
+  const int32_t pos_adj = a.positions ? 0 : -1;
+  const int32_t* req32 = reinterpret_cast<const int32_t*>(a.req_idx);
+
+  // operands: K-steps KW wave .. of the first tile's rows, then this wave's
+  // columns 16 wave + (0..15) of the group (rows of R_eff^T)
+  int64_t t = blockIdx.x / NG;
+  u32x4 xr[KW], gm[KW], ra[KS];
+  auto load_x = [&](int64_t tile) {
+    const uint16_t* x = a.x + min(tile * 16 + la, a.n - 1) * a.xs + 8 * gq;
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const f32x4 u = acc[2 * h][nb], v = acc[2 * h + 1][nb];
-          const u32x4 pk = {pack_bf16(u[0], u[1]), pack_bf16(u[2], u[3]), pack_bf16(v[0], v[1]),
-                            pack_bf16(v[2], v[3])};
-          *reinterpret_cast<u32x4*>(hrow + 8 * h) = pk;
-        }
+    for (int k = 0; k < KW; ++k) xr[k] = gload<u32x4>(x + 32 * (KW * wave + k));
+  };
+  load_x(t);
+  if constexpr (NORM) {
+#pragma unroll
+    for (int k = 0; k < KW; ++k) gm[k] = gload<u32x4>(a.gamma + 32 * (KW * wave + k) + 8 * gq);
+  }
+  {
+    const uint16_t* r = a.rt + (int64_t)(128 * g + writer_col(16 * wave + la)) * D + 8 * gq;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) ra[k] = gload<u32x4>(r + 32 * k);
+  }
+
+  for (; t < ntiles; t += a.nstripes) {
+    const int64_t row = t * 16 + la, rc = min(row, a.n - 1);
+    // the row's metadata, on the wave that needs it
+    int64_t slot = 0;
+    int32_t seq = 0, pos = 0, req = -1;
+    u32x2 pe = {0u, 0u};
+    if (wave == 0) {
+      if (a.pe_vec) pe = *reinterpret_cast<const u32x2*>(a.k_pe + rc * a.pe_s0 + 16 * g + 4 * gq);
+      slot = a.loc[rc];
+      seq = seq32[2 * rc];
+      pos = pos32[2 * rc] + pos_adj;
+      // a request index that does not fit 32 bits is outside [0, max_reqs)
+      const int32_t rlo = req32[2 * rc], rhi = req32[2 * rc + 1];
+      req = rhi == (rlo >> 31) ? rlo : -1;
+    }
+    if constexpr (NORM) {
+      // the row's sum of squares: eight columns per K-step and lane, the
+      // K-steps in order, then the row's four lanes
+#pragma unroll
+      for (int k = 0; k < KW; ++k) s_ss[(KW * wave + k) * 64 + lane] = sumsq8(xr[k]);
+      __syncthreads();
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) ss += s_ss[k * 64 + lane];
+      const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+      ss = __uint_as_float(u[0]) + __uint_as_float(u[1]);
+      const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+      ss = __uint_as_float(v[0]) + __uint_as_float(v[1]);
+      const float rinv = 1.0f / sqrtf(ss * (1.0f / D) + a.eps);
+#pragma unroll
+      for (int k = 0; k < KW; ++k) {
+        xr[k] = rms_apply8(xr[k], rinv, gm[k]);
+        const int ks = KW * wave + k;
+        if (a.y != nullptr && ks % NG == g && row < a.n)
+          *reinterpret_cast<u32x4*>(a.y + row * a.ys + 32 * ks + 8 * gq) = xr[k];
       }
-      // Lloyd statistics over the row's 128 group columns (4 lanes)
-      float s = 0.f;
+    }
 #pragma unroll
-      for (int mb = 0; mb < 8; ++mb) s += (acc[mb][nb][0] + acc[mb][nb][1]) + (acc[mb][nb][2] + acc[mb][nb][3]);
-      s = sum_over_rows(s);
-      const float mean = s * (1.0f / 128.0f);
-      float q = 0.f;
+    for (int k = 0; k < KW; ++k) s_x[(KW * wave + k) * 64 + lane] = xr[k];
+    __syncthreads();
+    if (t + a.nstripes < ntiles) load_x(t + a.nstripes);
+    f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int mb = 0; mb < 8; ++mb)
+    for (int k = 0; k < KS; ++k) c = mfma16x16x32(ra[k], s_x[k * 64 + lane], c);
+    s_c[wave * 64 + lane] = c;
+    __syncthreads();
+    if (wave == 0) {
+      f32x4 acc[kWriterWaves];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[mb][nb][i] -= mean;
-          q = fmaf(acc[mb][nb][i], acc[mb][nb][i], q);
-        }
-      q = sum_over_rows(q);
-      const float std_ = sqrtf(q * (1.0f / 128.0f) + 1e-08f);
-      // code = #{-t, 0, t <= normalized}, normalized = (x - mean) / std, the
-      // correctly rounded FP32 quotient (oscar.py:135-140): compared through
-      // the row's exact thresholds on y = x - mean (no division per element).
-      // Its two bits: high = (y >= y0), low = the parity of the three tests.
-      const double sd = (double)std_;
-      const float ylo = y_threshold(sd, mu_lo, incl_lo), y0 = y_threshold(sd, mu_zero, true),
-                  yhi = y_threshold(sd, mu_hi, incl_hi);
-      uint32_t word[2] = {0u, 0u};
-#pragma unroll
-      for (int wi = 0; wi < 2; ++wi)
-#pragma unroll
-        for (int e = 15; e >= 0; --e) {  // Horner, element e at bits 2e, 2e + 1
-          const float y = acc[4 * wi + e / 4][nb][e % 4];
-          const uint64_t hi = __builtin_amdgcn_ballot_w64(y >= y0);
-          const uint64_t lo = __builtin_amdgcn_ballot_w64(y >= ylo) ^ hi ^ __builtin_amdgcn_ballot_w64(y >= yhi);
-          word[wi] = twice_plus_bit(twice_plus_bit(word[wi], hi), lo);
-        }
-      if (live) {
-        // words 2gq, 2gq+1 of group g: row words 8g + 2gq, 8g + 2gq + 1
-        *reinterpret_cast<u32x2*>(a.codes + sl * (D / 4) + 4 * (8 * g + 2 * gq)) = u32x2{word[0], word[1]};
-        if (gq == 0) {
-          const float scale = a.kscale * std_;
-          const float zero = kZeroOffset - mean / scale;
-          *reinterpret_cast<f32x2*>(a.params + sl * 2 * NG + 2 * g) = f32x2{scale, zero};
-        }
-        if (sl > 0) {
-          if (a.pe_vec) {
-            // the rope pool's base read again from the kernel arguments here
-            // (a scalar load), not held in a register that would be spilled
-            // (as a global pointer: through a generic one the store is a flat
-            // store, which the next LDS waits would also wait for)
-            typedef __attribute__((address_space(1))) u32x2 g_u32x2;
-            uint16_t* const rope = kernarg_field<uint16_t*>(offsetof(WriterArgs, rope));
-            *(g_u32x2*)(rope + sl * a.R + 16 * g + 4 * gr) = pe;
-          } else if (g == 0) {
-            for (int r = gq; r < a.R; r += 4) a.rope[sl * a.R + r] = a.k_pe[row * a.pe_s0 + r * a.pe_s1];
-          }
-          if (g == 0 && gq == 0) {
-            a.row_of_slot[sl] = keep ? int32_t(ring) : -1;
-            if (keep) a.owner_of_row[ring] = int32_t(sl);
-          }
-        }
-      }
+      for (int mb = 0; mb < kWriterWaves; ++mb) acc[mb] = s_c[mb * 64 + lane];
+      store_row<D>(a, [&](int mb) -> f32x4& { return acc[mb]; }, row, slot, pos, seq, req, pe, g, gq, gq, t3);
     }
   }
 }
@@ -455,6 +580,8 @@ __global__ __launch_bounds__(64 * kWriterWaves, 1) void writer_kernel(WriterArgs
 static_assert(std::is_same<decltype(&writer_kernel<512, false>), void (*)(WriterArgs)>::value &&
                   std::is_same<decltype(&writer_kernel<256, true>), void (*)(WriterArgs)>::value,
               "writer_kernel's only argument must be WriterArgs (read at kernel-argument offset 0)");
+static_assert(std::is_same<decltype(&writer_few_kernel<512, false>), void (*)(WriterArgs)>::value,
+              "writer_few_kernel's only argument must be WriterArgs (read at kernel-argument offset 0)");
 
 }  // namespace rolaq
 
@@ -482,6 +609,28 @@ hipError_t rolaq_launch_writer(const rolaq::WriterArgs& args_in, int D, int num_
   // rope copy as 8-byte pieces: 16 columns per group, 8-byte aligned rows
   a.pe_vec = a.pe_s1 == 1 && a.R == 16 * NG && (a.pe_s0 % 4) == 0 &&
              (reinterpret_cast<uintptr_t>(a.k_pe) % 8) == 0 && (reinterpret_cast<uintptr_t>(a.rope) % 8) == 0;
+  // Few rows: 16-row tiles over CUs / NG stripes, while a stripe has at most
+  // three of them (five with the norm, which the other kernel pays for with a
+  // pass of its own). us, this kernel / the other, at one pass, at the line and
+  // past it -- D = 512: 1024 rows 8.1 / 14.3, 3000 12.7 / 14.7, 4096 15.3 / 15.0;
+  // with the norm 8.8 / 22.9, 5120 20.5 / 24.3, 8192 29.7 / 26.7; D = 256: 2048
+  // 5.8 / 11.1, 6000 9.9 / 11.3, 8192 11.9 / 11.5; with the norm 6.3 / 15.5, 8192
+  // 13.5 / 16.1, 16384 23.2 / 17.3.
+  const int64_t few_stripes = std::max(num_cus / NG, 1), tiles16 = (a.n + 15) / 16;
+  if (tiles16 <= few_stripes * (a.gamma ? 5 : 3)) {
+    a.nstripes = (int)std::min(tiles16, few_stripes);
+    const dim3 few((unsigned)(a.nstripes * NG));
+#define ROLAQ_FEW(DD, NORM)                                                                    \
+    if (D == DD && (a.gamma != nullptr) == NORM) {                                             \
+      hipLaunchKernelGGL((writer_few_kernel<DD, NORM>), few, dim3(64 * kWriterWaves), 0, stream, a); \
+      return hipGetLastError();                                                                \
+    }
+    ROLAQ_FEW(512, false)
+    ROLAQ_FEW(256, false)
+    ROLAQ_FEW(512, true)
+    ROLAQ_FEW(256, true)
+#undef ROLAQ_FEW
+  }
   const dim3 grid((unsigned)(stripes * NG)), block(64 * kWriterWaves);
 #define ROLAQ_WRITER(DD, NORM, LDS)                                                                         \
   if (D == DD && (a.gamma != nullptr) == NORM) {                                                           \

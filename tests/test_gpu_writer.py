@@ -259,7 +259,7 @@ def test_row_local_batching_is_exact(D, R):
 
 @pytest.mark.parametrize("norm", [False, True], ids=["plain", "norm"])
 @pytest.mark.parametrize("D,R", [(512, 64), (256, 32)])
-@pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 1023, 4097, 32767, 40961])
+@pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 1023, 1040, 3073, 5121, 6145, 10241, 32767, 40961])
 def test_write_does_not_depend_on_the_launch_size(D, R, n, norm):
     """The launch's size picks how rows are shared out (rows per wave, tiles per
     block); a row's bytes must not follow it: one launch against slices of 5,
