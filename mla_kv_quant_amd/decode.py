@@ -38,12 +38,12 @@ def packed_mla_decode_gf_fwd(q, o, pool, layer_id, kv_indptr, kv_indices, num_kv
         if P + W:
             raise ValueError("req_pool_indices is required when the BF16 window is enabled")
         req_pool_indices = torch.zeros(B, dtype=torch.int64, device=q.device)
-    req = req_pool_indices.reshape(-1)
+    req = req_pool_indices if req_pool_indices.ndim == 1 else req_pool_indices.reshape(-1)
     if req.dtype != torch.int64:
         req = req.to(torch.int64)
     sl = None
     if seq_lens is not None:
-        sl = seq_lens.reshape(-1)
+        sl = seq_lens if seq_lens.ndim == 1 else seq_lens.reshape(-1)
         if sl.dtype != torch.int64:
             sl = sl.to(torch.int64)
     return kernels.decode_fwd(q, pool.c_codes[li], pool.c_params[li], pool.rope_buf[li], pool.hp_c[li],

@@ -37,10 +37,10 @@ def packed_mla_extend_fwd(q, k, o, pool, layer_id, qo_indptr, kv_indptr, kv_indi
     li = layer_id - pool.start_layer
     if k.dim() == 3:
         k = k.reshape(k.shape[0], k.shape[-1])
-    pl = prefix_lens.reshape(-1)
+    pl = prefix_lens if prefix_lens.ndim == 1 else prefix_lens.reshape(-1)
     if pl.dtype != torch.int64:
         pl = pl.to(torch.int64)
-    req = req_pool_indices.reshape(-1)
+    req = req_pool_indices if req_pool_indices.ndim == 1 else req_pool_indices.reshape(-1)
     if req.dtype != torch.int64:
         req = req.to(torch.int64)
     B = qo_indptr.numel() - 1

@@ -18,11 +18,19 @@ GROUP_SIZE = 128
 
 
 def _p(t: torch.Tensor | None):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return None if t is None else t.data_ptr()
+
+
+# The current stream's handle by device index: what
+# ``torch.cuda.current_stream(device).cuda_stream`` returns, without building
+# the Stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype, device: torch.device, ndim: int | None = None):
@@ -39,6 +47,24 @@ def _need(t: torch.Tensor, name: str, dtype: torch.dtype, device: torch.device, 
 def _contig(t: torch.Tensor, name: str):
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
+
+
+# A decode step calls these functions a few times per layer, and their checks
+# were most of a call's host time (the 13 tensors of a write one by one: 17 us
+# a call, more than the kernel): a whole argument list is compared in one
+# expression per tensor, and only one that fails it is looked at again for
+# its message.
+_Tensor = torch.Tensor
+
+
+def _need_all(device, specs):
+    """``specs``: (tensor, name, dtype, ndim) of contiguous tensors on ``device``."""
+    for t, name, dtype, ndim in specs:
+        if isinstance(t, _Tensor) and t.dtype is dtype and t.device == device and t.ndim == ndim \
+                and t.is_contiguous():
+            continue
+        _need(t, name, dtype, device, ndim)
+        _contig(t, name)
 
 
 def scatter_pack_rows(x: torch.Tensor, slots: torch.Tensor, codes: torch.Tensor, params: torch.Tensor,
@@ -75,25 +101,18 @@ def _check_writer(latent, k_pe, rotation_t, loc, seq_lens, positions, req_idx, c
         _contig(rotation_t, "rotation_t")
         if tuple(rotation_t.shape) != (D, D):
             raise ValueError("rotation_t must be [D, D]")
-    for name, t in (("loc", loc), ("seq_lens", seq_lens), ("req_idx", req_idx)):
-        _need(t, name, torch.int64, dev, 1)
-        _contig(t, name)
-        if t.numel() != n:
-            raise ValueError(f"{name} must have {n} entries")
+    i64, i32 = torch.int64, torch.int32
+    _need_all(dev, ((loc, "loc", i64, 1), (seq_lens, "seq_lens", i64, 1), (req_idx, "req_idx", i64, 1)))
+    if loc.shape[0] != n or seq_lens.shape[0] != n or req_idx.shape[0] != n:
+        raise ValueError(f"loc, seq_lens and req_idx must have {n} entries")
     if positions is not None:
-        _need(positions, "positions", torch.int64, dev, 1)
-        _contig(positions, "positions")
-        if positions.numel() != n:
+        _need_all(dev, ((positions, "positions", i64, 1),))
+        if positions.shape[0] != n:
             raise ValueError("positions must have n entries")
-    _need(codes, "codes", torch.uint8, dev, 2)
-    _need(params, "params", torch.float32, dev, 3)
-    _need(rope_buf, "rope_buf", torch.bfloat16, dev, 2)
-    _need(hp_c, "hp_c", torch.bfloat16, dev, 2)
-    _need(row_of_slot, "row_of_slot", torch.int32, dev, 1)
-    _need(owner_of_row, "owner_of_row", torch.int32, dev, 1)
-    for name, t in (("codes", codes), ("params", params), ("rope_buf", rope_buf), ("hp_c", hp_c),
-                    ("row_of_slot", row_of_slot), ("owner_of_row", owner_of_row)):
-        _contig(t, name)
+    bf16 = torch.bfloat16
+    _need_all(dev, ((codes, "codes", torch.uint8, 2), (params, "params", torch.float32, 3),
+                    (rope_buf, "rope_buf", bf16, 2), (hp_c, "hp_c", bf16, 2), (row_of_slot, "row_of_slot", i32, 1),
+                    (owner_of_row, "owner_of_row", i32, 1)))
     if codes.shape[1] != D // 4 or tuple(params.shape[1:]) != (D // GROUP_SIZE, 2) or rope_buf.shape[1] != R \
             or hp_c.shape[1] != D:
         raise ValueError("cache buffers do not match (D, R)")
@@ -179,21 +198,13 @@ def _decode_check(q, codes, params, rope_buf, hp_c, kv_indptr, kv_indices, seq_l
     R = DR - D
     if q.stride(2) != 1:
         raise ValueError("q must be contiguous in its last dim")
-    _need(codes, "codes", torch.uint8, dev, 2)
-    _need(params, "params", torch.float32, dev, 3)
-    _need(rope_buf, "rope_buf", torch.bfloat16, dev, 2)
-    _need(hp_c, "hp_c", torch.bfloat16, dev, 2)
-    for name, t in (("codes", codes), ("params", params), ("rope_buf", rope_buf), ("hp_c", hp_c)):
-        _contig(t, name)
+    bf16, i32, i64 = torch.bfloat16, torch.int32, torch.int64
+    _need_all(dev, ((codes, "codes", torch.uint8, 2), (params, "params", torch.float32, 3),
+                    (rope_buf, "rope_buf", bf16, 2), (hp_c, "hp_c", bf16, 2)))
     if rope_buf.shape[1] != R or hp_c.shape[1] != D or tuple(params.shape[1:]) != (D // GROUP_SIZE, 2):
         raise ValueError("cache buffers do not match q's (D, R)")
-    _need(kv_indptr, "kv_indptr", torch.int32, dev, 1)
-    _need(kv_indices, "kv_indices", torch.int32, dev, 1)
-    _need(req_idx, "req_idx", torch.int64, dev, 1)
-    _need(num_kv_splits, "num_kv_splits", torch.int32, dev, 1)
-    for name, t in (("kv_indptr", kv_indptr), ("kv_indices", kv_indices), ("req_idx", req_idx),
-                    ("num_kv_splits", num_kv_splits)):
-        _contig(t, name)
+    _need_all(dev, ((kv_indptr, "kv_indptr", i32, 1), (kv_indices, "kv_indices", i32, 1), (req_idx, "req_idx", i64, 1),
+                    (num_kv_splits, "num_kv_splits", i32, 1)))
     if kv_indptr.numel() < B + 1 or req_idx.numel() < B or num_kv_splits.numel() < B:
         raise ValueError("index tensors are shorter than the batch")
     if seq_lens is not None:
@@ -338,19 +349,13 @@ def extend_fwd(q: torch.Tensor, k_chunk: torch.Tensor, qo_indptr: torch.Tensor, 
     _need(k_chunk, "k_chunk", torch.bfloat16, dev, 2)
     if k_chunk.shape[0] < T or k_chunk.shape[1] != DR or k_chunk.stride(1) != 1:
         raise ValueError("k_chunk must be [T, D + R] with a contiguous last dim")
-    _need(codes, "codes", torch.uint8, dev, 2)
-    _need(params, "params", torch.float32, dev, 3)
-    _need(rope_buf, "rope_buf", torch.bfloat16, dev, 2)
-    _need(hp_c, "hp_c", torch.bfloat16, dev, 2)
-    for name, t in (("codes", codes), ("params", params), ("rope_buf", rope_buf), ("hp_c", hp_c)):
-        _contig(t, name)
+    bf16, i32, i64 = torch.bfloat16, torch.int32, torch.int64
+    _need_all(dev, ((codes, "codes", torch.uint8, 2), (params, "params", torch.float32, 3),
+                    (rope_buf, "rope_buf", bf16, 2), (hp_c, "hp_c", bf16, 2)))
     if rope_buf.shape[1] != R or hp_c.shape[1] != D or tuple(params.shape[1:]) != (D // GROUP_SIZE, 2):
         raise ValueError("cache buffers do not match q's (D, R)")
-    for name, t, dt in (("qo_indptr", qo_indptr, torch.int32), ("kv_indptr", kv_indptr, torch.int32),
-                        ("kv_indices", kv_indices, torch.int32), ("prefix_lens", prefix_lens, torch.int64),
-                        ("req_idx", req_idx, torch.int64)):
-        _need(t, name, dt, dev, 1)
-        _contig(t, name)
+    _need_all(dev, ((qo_indptr, "qo_indptr", i32, 1), (kv_indptr, "kv_indptr", i32, 1), (kv_indices, "kv_indices", i32, 1),
+                    (prefix_lens, "prefix_lens", i64, 1), (req_idx, "req_idx", i64, 1)))
     B = qo_indptr.numel() - 1
     if B < 0 or kv_indptr.numel() < B + 1 or prefix_lens.numel() < B or req_idx.numel() < B:
         raise ValueError("index tensors are shorter than the batch")
@@ -385,11 +390,10 @@ def assemble_rows(slots: torch.Tensor, codes: torch.Tensor, params: torch.Tensor
     _contig(slots, "slots")
     D = codes.shape[1] * 4
     R = rope_buf.shape[1]
-    for name, t, dt in (("codes", codes, torch.uint8), ("params", params, torch.float32),
-                        ("rope_buf", rope_buf, torch.bfloat16), ("hp_c", hp_c, torch.bfloat16),
-                        ("row_of_slot", row_of_slot, torch.int32), ("owner_of_row", owner_of_row, torch.int32)):
-        _need(t, name, dt, dev)
-        _contig(t, name)
+    _need_all(dev, ((codes, "codes", torch.uint8, codes.ndim), (params, "params", torch.float32, params.ndim),
+                    (rope_buf, "rope_buf", torch.bfloat16, rope_buf.ndim), (hp_c, "hp_c", torch.bfloat16, hp_c.ndim),
+                    (row_of_slot, "row_of_slot", torch.int32, row_of_slot.ndim),
+                    (owner_of_row, "owner_of_row", torch.int32, owner_of_row.ndim)))
     if hp_c.shape[1] != D or tuple(params.shape[1:]) != (D // GROUP_SIZE, 2):
         raise ValueError("cache buffers do not match")
     if rotation is not None:

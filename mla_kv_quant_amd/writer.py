@@ -19,8 +19,14 @@ SUPPORTED_DIMS = {(512, 64), (256, 32)}
 
 
 def _as_int64(t: torch.Tensor) -> torch.Tensor:
-    t = t.reshape(-1)
+    if t.ndim != 1:
+        t = t.reshape(-1)
     return t if t.dtype == torch.int64 and t.is_contiguous() else t.to(torch.int64).contiguous()
+
+
+def _rows(t: torch.Tensor, width: int) -> torch.Tensor:
+    """``t`` as ``[n, width]`` (itself where it is: a view costs more than the test)."""
+    return t if t.ndim == 2 and t.shape[1] == width else t.reshape(-1, width)
 
 
 def _write_rotation(pool, layer_id: int, r: torch.Tensor | None):
@@ -85,10 +91,10 @@ def try_fast_decode_store(pool, layer_id, loc, c_kv, k_pe) -> bool:
         frames.setdefault(layer_id, id(r))
     loc64 = _as_int64(loc)
     pool._write_loc = loc64
-    x = c_kv.reshape(-1, pool.kv_lora_rank)
+    x = _rows(c_kv, pool.kv_lora_rank)
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
-    pe = k_pe.reshape(-1, pool.qk_rope_head_dim)
+    pe = _rows(k_pe, pool.qk_rope_head_dim)
     params = pool._rolaq_quantizers[li]
     t, g = (params[0], params[1]) if params is not None else (LM_THRESHOLD, LM_GAIN)
     kernels.write_rows(
@@ -109,10 +115,10 @@ def write_prefill(pool, layer_id, loc, c_kv, k_pe, positions, seq_lens, req_pool
     li = layer_id - pool.start_layer
     r = pool.latent_rotation(layer_id, local=True)
     rt = _write_rotation(pool, layer_id, r)
-    x = c_kv.reshape(-1, pool.kv_lora_rank)
+    x = _rows(c_kv, pool.kv_lora_rank)
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
-    pe = k_pe.reshape(-1, pool.qk_rope_head_dim)
+    pe = _rows(k_pe, pool.qk_rope_head_dim)
     params = pool._rolaq_quantizers[li]
     t, g = (params[0], params[1]) if params is not None else (LM_THRESHOLD, LM_GAIN)
     kernels.write_rows(
@@ -144,12 +150,12 @@ def try_fast_norm_decode_store(pool, layer_id, loc, kv_a, k_pe, norm_weight, eps
         rt = _identity_rotation(pool, kv_a.device)
     loc64 = _as_int64(loc)
     pool._write_loc = loc64
-    x = kv_a.reshape(-1, pool.kv_lora_rank)
+    x = _rows(kv_a, pool.kv_lora_rank)
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
     t, g = _quantizer(pool, li)
     kernels.norm_write_rows(
-        x, norm_weight, float(eps), latent_out, k_pe.reshape(-1, pool.qk_rope_head_dim), rt, loc64,
+        x, norm_weight, float(eps), latent_out, _rows(k_pe, pool.qk_rope_head_dim), rt, loc64,
         _as_int64(meta["seq_lens"]), None, _as_int64(meta["req_pool_indices"]), pool.c_codes[li],
         pool.c_params[li], pool.rope_buf[li], pool.hp_c[li], pool.hp_row_of_slot, pool.hp_owner_of_row,
         pool._win_p, pool._win_r, pool._max_reqs, t, g)
@@ -165,12 +171,12 @@ def norm_write_prefill(pool, layer_id, loc, kv_a, k_pe, positions, seq_lens, req
     rt = _write_rotation(pool, layer_id, r)
     if rt is None:
         rt = _identity_rotation(pool, kv_a.device)
-    x = kv_a.reshape(-1, pool.kv_lora_rank)
+    x = _rows(kv_a, pool.kv_lora_rank)
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
     t, g = _quantizer(pool, li)
     kernels.norm_write_rows(
-        x, norm_weight, float(eps), latent_out, k_pe.reshape(-1, pool.qk_rope_head_dim), rt, _as_int64(loc),
+        x, norm_weight, float(eps), latent_out, _rows(k_pe, pool.qk_rope_head_dim), rt, _as_int64(loc),
         _as_int64(seq_lens), _as_int64(positions), _as_int64(req_pool_indices), pool.c_codes[li],
         pool.c_params[li], pool.rope_buf[li], pool.hp_c[li], pool.hp_row_of_slot, pool.hp_owner_of_row,
         pool._win_p, pool._win_r, pool._max_reqs, t, g)
