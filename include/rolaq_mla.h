@@ -135,18 +135,22 @@ int rolaq_prepare_gf_splits(const int32_t* splits, int32_t* quant, int32_t* merg
  * disabled, deployment/serve.py:149).
  * num_kv_splits: int32 [B] requested splits ns_b (1 <= ns_b <= max_kv_splits);
  * request b uses ns'_b = min(ns_b, cap) splits, cap as rolaq_decode_split_cap
- * returns it (about one working block per compute unit: more splits only
- * add partials to write and merge, and SGLang reads only the merged output;
- * the output does not depend on the split count beyond FP32 summation order).
+ * returns it, or, where the batch's requests together ask for more than one
+ * working block per compute unit, a share of the units by its length (more
+ * splits only add partials to write and merge, and SGLang reads only the merged
+ * output; the output does not depend on the split count beyond FP32 summation
+ * order).
  * Positions P <= t < L_b - W and the window rows are split over
- * nq_b = max(ns'_b - 1, 1) splits (the window rows go with split 0); the
+ * nq_b <= max(ns'_b - 1, 1) splits (the window rows go with split 0); the
  * reference's separate window split has no partial of its own here.
  * attn_logits (fp32, 16-byte aligned, at least B * H * (max_kv_splits + 1) * D
  * floats) and attn_lse (fp32, at least B * H * (max_kv_splits + 1)) are
- * scratch: the call uses their first B * H * S1c * D and B * H * S1c floats as
- * [B, H, S1c, D] and [B, H, S1c], S1c = min(cap - 1, max_kv_splits) + 1, and
- * writes partials (normalised output, natural-log LSE; empty splits 0 / -1e4)
- * to slots 0 .. nq_b - 1 of each (b, h). The merged output goes to out: bf16
+ * scratch: the call uses their first B * H * S1c * D and B * H * S1c floats,
+ * S1c = min(cap - 1, max_kv_splits) + 1. attn_lse is [B, H, S1c]: the natural-log
+ * LSE of splits 0 .. nq_b - 1, -1e4 for empty and for unused ones up to
+ * ns'_b - 1, and the call's own bookkeeping in slot S1c - 1. attn_logits is
+ * [B, H, S1c, D] (normalised output, empty splits 0) where every split asked for
+ * is used; else the requests' [H, nq_b, D] lie one after another. The merged output goes to out: bf16
  * [B, H, D] with strides (out_stride_b, out_stride_h), in the rotated frame.
  * Supported shapes: (D, R) = (512, 64) or (256, 32), 1 <= H <= 128; window
  * P + W <= 32. Latent values (query, stored levels, window rows) are carried
@@ -185,8 +189,10 @@ int rolaq_decode_fwd_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride
 
 /*
  * The split cap of rolaq_decode_fwd and rolaq_decode_fwd_noalloc on the
- * current device: ceil(CUs / (B * head blocks)) + 1, at most max_kv_splits
- * (a head block is 16 heads at D = 512 and up to 48 at D = 256), written to
+ * current device, at most max_kv_splits: each + 1, each = ceil(CUs / (B * head
+ * blocks)) (a head block is 16 heads at D = 512 and up to 48 at D = 256), for
+ * one request, for more than 256 and where each = 1; otherwise one request may
+ * have min(4 * each, 64, CUs / head blocks - B + 1) + 1 if that is more. Written to
  * *cap. Host only: no launch, no synchronisation. No counterpart in the
  * reference, whose stage 1 runs every requested split.
  */

@@ -269,14 +269,21 @@ int decode_args(const char* who, const void* q, int64_t q_stride_b, int64_t q_st
   return ROLAQ_OK;
 }
 
-// The split count the fused decode uses at most: enough quantized splits for
-// one working block per compute unit over the batch's (sequence, head block)
-// pairs, plus the window split, and never more than the caller's maximum.
-// Every request then takes min(its num_kv_splits, this); the merged output
-// does not depend on the split count (up to FP32 summation order).
+// The most splits the fused decode gives one request. `each` quantized splits
+// give every compute unit a working block over the batch's (sequence, head
+// block) pairs; the units are shared by the requests' lengths (share_blocks in
+// decode.hip), up to four times `each` for one request. Past 64 splits the
+// merge costs what the share gives (four requests of 26000 .. 65536 tokens, 20
+// heads at D = 256: 53.8 us with 64 each, 55.3 us shared), so up to four
+// requests have `each` as they are. Plus the window split, and never more than
+// the caller's maximum. The merged output does not depend on the split count
+// (up to FP32 summation order).
 int fused_split_cap(int B, int H, int D, int max_kv_splits) {
   const int64_t units = int64_t(B) * rolaq_decode_head_blocks(D, H);
-  const int64_t quant = (cu_count() + units - 1) / units;
+  const int64_t each = (cu_count() + units - 1) / units;
+  const int64_t blocks = cu_count() / rolaq_decode_head_blocks(D, H);
+  const bool share = B > 1 && B < blocks && B <= rolaq::kShareRequests;
+  const int64_t quant = share ? std::max<int64_t>(each, std::min<int64_t>({4 * each, 64, blocks - B + 1})) : each;
   const int64_t cap = (quant < 1 ? 1 : quant) + 1;
   return cap < max_kv_splits ? int(cap) : max_kv_splits;
 }
@@ -292,6 +299,13 @@ void fused_layout(rolaq::DecodeArgs* a, int B, int H, int D, int max_kv_splits) 
   a->split_cap = fused_split_cap(B, H, D, max_kv_splits);
   a->neutral = 0;
   a->S1 = std::max(std::min(a->split_cap - 1, max_kv_splits), 1) + 1;
+  // one block per CU, shared out by the requests' lengths on the device, where
+  // there are several requests and more than one split to give
+  const int64_t blocks = cu_count() / rolaq_decode_head_blocks(D, H);
+  const int64_t most = int64_t(B) * (a->S1 - 1);  // what the requests can ask for
+  const bool share = B > 1 && B < blocks && B <= rolaq::kShareRequests && a->S1 > 2;
+  a->blocks = share && most > blocks && blocks < 4096 ? int(blocks) : 0;
+  a->blocks_each = a->blocks / B;
 }
 
 }  // namespace

@@ -174,11 +174,153 @@ __device__ void write_neutral(const DecodeArgs& a, int b, int h0, int nh, int sp
   if ((int)threadIdx.x < nh) a.lse[((int64_t)b * a.H + h0 + threadIdx.x) * a.S1 + split] = kNeutralLse;
 }
 
+// Inclusive scan of v over the wave (DPP: rows of 16, then the rows' totals);
+// lane 63 holds the sum.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int add_dpp(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_scan(int v) {
+  v = add_dpp<0x111, 0xF>(v);  // row_shr 1, 2, 4, 8
+  v = add_dpp<0x112, 0xF>(v);
+  v = add_dpp<0x114, 0xF>(v);
+  v = add_dpp<0x118, 0xF>(v);
+  v = add_dpp<0x142, 0xA>(v);  // lane 15 of rows 0 and 2 to rows 1 and 3
+  return add_dpp<0x143, 0xC>(v);  // lane 31 to rows 2 and 3
+}
+__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_scan(v), 63); }
+
+// Units of a sequence of L tokens (the window tile, when there is one, and the
+// 32-token tiles of the INT2 positions), as stage 1 cuts them.
+__device__ __forceinline__ int units_of(int L, int P, int W) {
+  const int lo = min(P, L), hi = max(L - W, lo);
+  const int tiles = hi > lo ? (hi + kTile - 1) / kTile - lo / kTile : 0;
+  return tiles + (L > 0 && P + W > 0 ? 1 : 0);
+}
+
+// The fused call's blocks shared out over the batch. Every block finds its
+// (sequence, split) itself, from all requests' lengths, a lane each. Each
+// request gets its requested splits if they all fit the launch's blocks;
+// otherwise as many as leave every block at most m units (tiles), with about
+// the smallest m for which the blocks suffice. Equal lengths get equal counts.
+// With equal counts for all, the launch waits for the longest request's blocks:
+// stage 1 of 16 requests of 1024 .. 16384 tokens took 27 us, now 21; of 128
+// requests of 2048 .. 8192, 69.8 us, now 63.7 (a whole decode: 71 -> 65.5 us a
+// layer); 32 requests of 16384 are where they were (46.5 us a layer).
+struct Share {
+  int b = 0, split = 0, nq = 1;
+  int first = 0;        // blocks before the request's
+  bool any = false;     // this block has a split at all
+  bool packed = false;  // not every requested split fits a block
+  int L = 0, kv0 = 0, req = 0;
+  bool ring = false;
+};
+template <int NC>  // chunks of 64 requests
+__device__ __forceinline__ Share share_blocks(const DecodeArgs& a, int p, int lane) {
+  int ns[NC], k0[NC], k1[NC];
+  int64_t req[NC], sl[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {  // one round trip for all
+    const int i = min(64 * c + lane, a.B - 1);
+    ns[c] = gload<int32_t>(a.num_kv_splits + i);
+    k0[c] = gload<int32_t>(a.kv_indptr + i);
+    k1[c] = gload<int32_t>(a.kv_indptr + i + 1);
+    req[c] = gload<int64_t>(a.req_idx + i);
+    sl[c] = gload<int64_t>((a.seq_lens ? a.seq_lens : a.req_idx) + i);
+  }
+  int L[NC], ring[NC], asked[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    L[c] = a.seq_lens ? (int)sl[c] : k1[c] - k0[c];
+    ring[c] = req[c] >= 0 && req[c] < a.max_reqs ? 1 : 0;
+    asked[c] = min(max(min(ns[c], a.split_cap) - 1, 1), a.S1 - 1);
+  }
+  const int T = a.blocks;
+  Share r;
+  // Equal requests (the lanes past the batch hold the last one's): T / B
+  // blocks each, without the search. A split of every request, then the next.
+  const int L0 = __builtin_amdgcn_readfirstlane(L[0]), ring0 = __builtin_amdgcn_readfirstlane(ring[0]);
+  const int asked0 = __builtin_amdgcn_readfirstlane(asked[0]);
+  int differ = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) differ |= (L[c] ^ L0) | (ring[c] ^ ring0) | (asked[c] ^ asked0);
+  if (__builtin_amdgcn_ballot_w64(differ != 0) == 0) {
+    r.nq = min(asked0, a.blocks_each);
+    r.packed = asked0 > a.blocks_each;
+    r.split = (int)((uint32_t)p / (uint32_t)a.B);
+    r.b = p - r.split * a.B;
+    r.any = r.split < r.nq;
+    r.first = r.b * r.nq;
+  } else {
+    int units[NC], give[NC], n_asked = 0, n_units = 0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const bool in = 64 * c + lane < a.B;
+      // (2^22 units are 2^27 tokens: sums of all requests stay in 32 bits)
+      units[c] = in ? min(units_of(L[c], ring[c] ? a.P : 0, ring[c] ? a.W : 0), 1 << 22) : 0;
+      give[c] = asked[c] = in ? asked[c] : 0;
+      n_asked += asked[c];
+      n_units += units[c];
+    }
+    r.packed = wave_total(n_asked) > T;
+    if (r.packed) {
+      const int all_units = wave_total(n_units);
+      const float inv_t = __builtin_amdgcn_rcpf((float)T);
+      float m = fmaxf(ceilf((float)all_units * inv_t - 1.0e-3f), 1.f);
+      for (int it = 0;; ++it) {
+        const float inv = __builtin_amdgcn_rcpf(m);
+        int n = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          // (a hair less than the quotient: an exact multiple must not round up)
+          give[c] = min(max((int)ceilf((float)units[c] * inv - 1.0e-3f), 1), asked[c]);
+          n += give[c];
+        }
+        n = wave_total(n);
+        if (n <= T || it == 7) break;
+        m = fmaxf(m + 1.f, ceilf(m * (float)n * inv_t));
+        // at m_end a block of each request's own and T - B more (T > B) suffice
+        if (it >= 4) {
+          const float m_end = (float)(all_units / (T - a.B) + 1);
+          m = it == 6 ? m_end : fminf(m, m_end);
+        }
+      }
+    }
+    // block p's request: the first one whose running count passes p
+    int before = 0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (!r.any) {
+        const int scan = wave_scan(give[c]) + before;
+        const uint64_t past = __builtin_amdgcn_ballot_w64(scan > p);
+        if (past) {
+          const int l = __builtin_ctzll(past);
+          r.any = true;
+          r.b = 64 * c + l;
+          r.nq = __builtin_amdgcn_readlane(give[c], l);
+          r.first = __builtin_amdgcn_readlane(scan, l) - r.nq;
+          r.split = p - r.first;
+        }
+        before = __builtin_amdgcn_readlane(scan, 63);
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (NC == 1 || r.b >> 6 == c) {
+      const int l = r.b & 63;
+      r.L = __builtin_amdgcn_readlane(L[c], l);
+      r.kv0 = __builtin_amdgcn_readlane(k0[c], l);
+      r.ring = __builtin_amdgcn_readlane(ring[c], l) != 0;
+      r.req = __builtin_amdgcn_readlane((int)req[c], l);
+    }
+  return r;
+}
+
 // ---------------------------------------------------------------------------
 // Stage 1. HG head groups of 16 per block (their query operands and output
 // accumulators live in one wave); D = 512 uses HG = 1.
 // ---------------------------------------------------------------------------
-template <int D, int R, int HG>
+template <int D, int R, int HG, int NC>
 __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   using G = DGeo<D, R>;
   constexpr int KL = G::KL, KR = G::KR, CB = G::CB, CV = G::CV, WPL = G::WPL, ROWB = G::ROWB, NB = G::NB;
@@ -197,7 +339,7 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   asm volatile("" ::"s"(a.q), "s"(a.q_sb), "s"(a.q_sh), "s"(a.codes), "s"(a.params), "s"(a.rope), "s"(a.hp),
                "s"(a.kv_indptr), "s"(a.kv_indices), "s"(a.page_shift), "s"(a.seq_lens), "s"(a.req_idx),
                "s"(a.num_kv_splits), "s"(a.split_cap), "s"(a.S1), "s"(a.max_reqs), "s"(a.H), "s"(a.P),
-               "s"(a.W), "s"(a.sm_scale), "s"(gridDim.x), "s"(gridDim.y));
+               "s"(a.W), "s"(a.sm_scale), "s"(a.logits), "s"(a.lse), "s"(gridDim.x), "s"(gridDim.y));
 
   // ---- which (sequence, head block, split) ------------------------------------
   const int nhb = ((a.H + 15) / 16 + HG - 1) / HG;
@@ -209,34 +351,56 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   const int nblk = gridDim.x * gridDim.y;
   if (nhb > 1 && nblk % kXcds == 0) lin = (lin % kXcds) * (nblk / kXcds) + lin / kXcds;
   const int hb = nhb > 1 ? lin % nhb : 0;
-  const int split = nhb > 1 ? (lin / nhb) % (int)gridDim.y : (int)blockIdx.y;
-  const int b = nhb > 1 ? (lin / nhb) / (int)gridDim.y : (int)blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, la = lane & 15, gq = lane >> 4;
+  int split = nhb > 1 ? (lin / nhb) % (int)gridDim.y : (int)blockIdx.y;
+  int b = nhb > 1 ? (lin / nhb) / (int)gridDim.y : (int)blockIdx.x;
+  Share sh;
+  if constexpr (NC > 0) {
+    sh = share_blocks<NC>(a, nhb > 1 ? lin / nhb : lin, lane);
+    if (!sh.any) return;
+    b = sh.b;
+    split = sh.split;
+  }
   const int h0 = 16 * HG * hb;
   const int nh = min(16 * HG, a.H - h0);  // heads of this block
-  const int tid = threadIdx.x, lane = tid & 63, la = lane & 15, gq = lane >> 4;
   const int gl = lane_group<D>(gq), s0 = lane_word0<D>(gq);
 
   // The sequence's metadata: five loads issued together and waited for once
   // (the split test below would otherwise wait for its own load first), then
   // the query's loads, which the first tile needs only after two more round
-  // trips (page lookups, tile data).
-  const int ns_req = a.num_kv_splits[b];
-  const int kv0 = a.kv_indptr[b], kv1 = a.kv_indptr[b + 1];
-  const int64_t req = a.req_idx[b];
-  const int64_t slv = (a.seq_lens ? a.seq_lens : a.req_idx)[b];  // no branch before the loads
-  u32x4 qB[HG][KL], qR[HG][KR];
-#pragma unroll
-  for (int hg = 0; hg < HG; ++hg) {
-    const uint16_t* qh = a.q + b * a.q_sb + (int64_t)min(h0 + 16 * hg + la, a.H - 1) * a.q_sh;
-#pragma unroll
-    for (int j = 0; j < KL; ++j) qB[hg][j] = gload<u32x4>(qh + 128 * gl + 16 * (s0 + j / 2) + 8 * (j & 1));
-#pragma unroll
-    for (int kr = 0; kr < KR; ++kr) qR[hg][kr] = gload<u32x4>(qh + D + 32 * kr + 8 * gq);
+  // trips (page lookups, tile data). With NC > 0 the metadata is here already:
+  // the query's loads then go out behind the page lookups (loads return in
+  // order) and are waited for behind the first tile's.
+  int ns_req, kv0, kv1;
+  int64_t req, slv;
+  if constexpr (NC == 0) {
+    ns_req = a.num_kv_splits[b];
+    kv0 = a.kv_indptr[b], kv1 = a.kv_indptr[b + 1];
+    req = a.req_idx[b];
+    slv = (a.seq_lens ? a.seq_lens : a.req_idx)[b];  // no branch before the loads
   }
-  asm volatile("" ::"v"(ns_req), "v"(kv0), "v"(kv1), "v"(req), "v"(slv));
-  const int ns = min(ns_req, a.split_cap);
-  const int L = a.seq_lens ? (int)slv : kv1 - kv0;
-  const int nq = min(max(ns - 1, 1), a.S1 - 1);
+  u32x4 qB[HG][KL], qR[HG][KR];
+  auto load_q = [&]() {
+#pragma unroll
+    for (int hg = 0; hg < HG; ++hg) {
+      const uint16_t* qh = a.q + b * a.q_sb + (int64_t)min(h0 + 16 * hg + la, a.H - 1) * a.q_sh;
+#pragma unroll
+      for (int j = 0; j < KL; ++j) qB[hg][j] = gload<u32x4>(qh + 128 * gl + 16 * (s0 + j / 2) + 8 * (j & 1));
+#pragma unroll
+      for (int kr = 0; kr < KR; ++kr) qR[hg][kr] = gload<u32x4>(qh + D + 32 * kr + 8 * gq);
+    }
+  };
+  if constexpr (NC == 0) load_q();
+  int L, nq;
+  bool has_ring;
+  if constexpr (NC > 0) {
+    L = sh.L, nq = sh.nq, kv0 = sh.kv0, req = sh.req, has_ring = sh.ring;
+  } else {
+    asm volatile("" ::"v"(ns_req), "v"(kv0), "v"(kv1), "v"(req), "v"(slv));
+    L = a.seq_lens ? (int)slv : kv1 - kv0;
+    nq = min(max(min(ns_req, a.split_cap) - 1, 1), a.S1 - 1);
+    has_ring = req >= 0 && req < a.max_reqs;
+  }
   if (split > nq) return;
   if (split == nq) {
     if (a.neutral) write_neutral(a, b, h0, nh, split, D);
@@ -245,7 +409,6 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
 
   // a request without ring rows (index outside [0, max_reqs)) has no window:
   // the writer stored none for it, so every position is read from its codes
-  const bool has_ring = req >= 0 && req < a.max_reqs;
   const int P = has_ring ? a.P : 0, W = has_ring ? a.W : 0;
   const int lo = min(P, L), hi = max(L - W, lo);          // INT2 positions [lo, hi)
   const int n_sink = lo, rec_lo = max(L - W, n_sink);
@@ -640,11 +803,14 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     lookup(min(1, nl), pgn);
     window_pages();
     window_rows();
+    if constexpr (NC > 0) load_q();
     __builtin_amdgcn_sched_barrier(0);
-    setup();
+    if constexpr (NC == 0) setup();
     __builtin_amdgcn_sched_barrier(0);
     window_rope();
     load(0, pgc, dn);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NC > 0) setup();
     __builtin_amdgcn_sched_barrier(0);
     window_tile();
     first = false;
@@ -652,9 +818,13 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     lookup(0, pgc);
     lookup(min(1, nl), pgn);
     __builtin_amdgcn_sched_barrier(0);
-    setup();
+    if constexpr (NC > 0) load_q();
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NC == 0) setup();
     __builtin_amdgcn_sched_barrier(0);
     load(0, pgc, dn);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NC > 0) setup();
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -760,7 +930,12 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
       }
     }
     if (hh < nh) {
-      float* const row = a.logits + (((int64_t)b * a.H + h0 + hh) * a.S1 + split) * D;
+      // shared blocks: the request's partials of a head together, the requests one
+      // after another (at S1 slots a head, most of them unused, the merge read and
+      // the L2 wrote back 2 us slower)
+      const int64_t r0 = NC > 0 && sh.packed ? (int64_t)sh.first * a.H + (h0 + hh) * nq
+                                             : ((int64_t)b * a.H + h0 + hh) * a.S1;
+      float* const row = a.logits + (r0 + split) * D;
 #pragma unroll
       for (int k = 0; k < KL / 4; ++k) {
         const int j = tt % KL, gqo = (16 / KL) * k + tt / KL;
@@ -774,56 +949,87 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     }
     if (hg + 1 < HG) __syncthreads();  // before the next head group reuses the buffers
   }
+  // for the merge, in the LSE slot that no partial has: the request's count and
+  // where its partials lie
+  if (NC > 0 && split == 0 && tid < nh)
+    a.lse[((int64_t)b * a.H + h0 + tid) * a.S1 + a.S1 - 1] =
+        __builtin_bit_cast(float, (sh.packed ? (sh.first + 1) << 12 : 0) | nq);
 }
 
 // ---------------------------------------------------------------------------
 // Stage 2: LSE merge of the partials -> bf16 output: the nq quantized splits'
 // partials and, when stage 1 wrote it (neutral = 1), the window split's
 // neutral one. The LSEs and partials of up to kBatch splits are loaded
-// together (one round trip after the split count), then merged online.
+// together (one round trip after the split count), then merged online; by
+// groups of kGroup, so that few splits issue few loads: with the last split's
+// loads repeated up to a full batch, decode of 64 x 16384 tokens (40 heads,
+// four splits) took 58.6 us a layer where it takes 58.1.
 // ---------------------------------------------------------------------------
 template <int D>
 __global__ __launch_bounds__(128) void decode_stage2(const float* __restrict__ logits,
-                                                     const float* __restrict__ lse,
+                                                     float* __restrict__ lse,
                                                      const int32_t* __restrict__ num_kv_splits,
-                                                     int split_cap, int neutral, int H, int S1, uint16_t* out,
+                                                     int split_cap, int neutral, int shared, int H, int S1,
+                                                     uint16_t* out,
                                                      int64_t o_sb, int64_t o_sh) {
   constexpr int FPT = D / 128;
-  constexpr int kBatch = 16;
+  constexpr int kBatch = D == 256 ? 32 : 16, kGroup = 4;  // (64 registers of partials)
   typedef float fv __attribute__((ext_vector_type(FPT)));
   const int b = blockIdx.x / H, h = blockIdx.x % H;
-  const int nq = min(max(min(num_kv_splits[b], split_cap) - 1, 1), S1 - 1);
-  const int np = nq + neutral;  // partials to merge (1 <= np <= S1)
   const int64_t row = ((int64_t)b * H + h) * S1;
+  const int ns = num_kv_splits[b];
+  const int last = __builtin_bit_cast(int, lse[row + S1 - 1]);
+  asm volatile("" ::"s"(ns), "s"(last), "s"(logits), "s"(split_cap), "s"(neutral), "s"(shared), "s"(out), "s"(o_sb),
+               "s"(o_sh));  // one wait for all
+  const int asked = min(max(min(ns, split_cap) - 1, 1), S1 - 1) + neutral;
+  // partials to merge (1 <= np <= S1) and their first row, by stage 1's code
+  // where it shared out its blocks (shared = 1)
+  const int code = shared ? last : asked;
+  const int np = shared ? min(max(code & 0xFFF, 1), S1 - 1) : asked;
+  const int64_t part = shared && code >> 12 ? (int64_t)((code >> 12) - 1) * H + h * np : row;
   float M = -3.0e38f, den = 0.f;
   fv acc = {};
   for (int s0 = 0; s0 < np; s0 += kBatch) {
     float ls[kBatch];
     fv v[kBatch];
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      const int s = min(s0 + i, np - 1);
-      ls[i] = lse[row + s];
-      v[i] = *reinterpret_cast<const fv*>(logits + (row + s) * D + threadIdx.x * FPT);
-    }
+    for (int g = 0; g < kBatch; g += kGroup)
+      if (s0 + g < np) {
+#pragma unroll
+        for (int i = g; i < g + kGroup; ++i) {
+          const int s = min(s0 + i, np - 1);
+          ls[i] = lse[row + s];
+          v[i] = *reinterpret_cast<const fv*>(logits + (part + s) * D + threadIdx.x * FPT);
+        }
+      }
     float mb = M;
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) mb = s0 + i < np ? fmaxf(mb, ls[i]) : mb;
+    for (int g = 0; g < kBatch; g += kGroup)
+      if (s0 + g < np) {
+#pragma unroll
+        for (int i = g; i < g + kGroup; ++i) mb = s0 + i < np ? fmaxf(mb, ls[i]) : mb;
+      }
     const float c = __builtin_amdgcn_exp2f((M - mb) * kLog2e);  // 0 on the first batch
     den *= c;
     acc *= c;
     M = mb;
 #pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      const float w = s0 + i < np ? __builtin_amdgcn_exp2f((ls[i] - M) * kLog2e) : 0.f;
-      den += w;
-      acc += w * v[i];
-    }
+    for (int g = 0; g < kBatch; g += kGroup)
+      if (s0 + g < np) {
+#pragma unroll
+        for (int i = g; i < g + kGroup; ++i) {
+          const float w = s0 + i < np ? __builtin_amdgcn_exp2f((ls[i] - M) * kLog2e) : 0.f;
+          den += w;
+          acc += w * v[i];
+        }
+      }
   }
   const float inv = 1.f / den;
   uint16_t* dst = out + b * o_sb + h * o_sh + threadIdx.x * FPT;
 #pragma unroll
   for (int i = 0; i < FPT; ++i) dst[i] = float_to_bf16(acc[i] * inv);
+  // splits asked for beyond the request's share hold no key
+  for (int s = np + threadIdx.x; s < asked; s += 128) lse[row + s] = kNeutralLse;
 }
 
 }  // namespace rolaq
@@ -851,9 +1057,14 @@ hipError_t rolaq_launch_decode(const rolaq::DecodeArgs& a, int D, int R, int max
   // quantized splits, then (neutral = 1) the window split's neutral partial
   const int nq_max = std::max(std::min(a.split_cap - 1, max_splits), 1);
   const int rows = nq_max + (a.neutral ? 1 : 0);
-  const dim3 grid(a.B * nhb, rows), block(kThreads);
-#define ROLAQ_S1(DD, RR, GG) \
-  if (D == DD && R == RR && HG == GG) hipLaunchKernelGGL((decode_stage1<DD, RR, GG>), grid, block, 0, stream, a);
+  // (a.blocks: blocks per head block that the requests share by their lengths)
+  const dim3 grid = a.blocks ? dim3(a.blocks * nhb) : dim3(a.B * nhb, rows), block(kThreads);
+#define ROLAQ_S1(DD, RR, GG)                                                                         \
+  if (D == DD && R == RR && HG == GG) {                                                              \
+    if (!a.blocks) hipLaunchKernelGGL((decode_stage1<DD, RR, GG, 0>), grid, block, 0, stream, a);    \
+    else if (a.B <= 64) hipLaunchKernelGGL((decode_stage1<DD, RR, GG, 1>), grid, block, 0, stream, a); \
+    else hipLaunchKernelGGL((decode_stage1<DD, RR, GG, kShareRequests / 64>), grid, block, 0, stream, a); \
+  }
   if (stages & kStagePartials) {
     ROLAQ_S1(512, 64, 1)
     else ROLAQ_S1(256, 32, 1)
@@ -865,10 +1076,10 @@ hipError_t rolaq_launch_decode(const rolaq::DecodeArgs& a, int D, int R, int max
   if (stages & kStageMerge) {
     if (D == 512)
       hipLaunchKernelGGL((decode_stage2<512>), dim3(a.B * a.H), dim3(128), 0, stream, a.logits, a.lse,
-                         a.num_kv_splits, a.split_cap, a.neutral, a.H, a.S1, out, o_sb, o_sh);
+                         a.num_kv_splits, a.split_cap, a.neutral, a.blocks ? 1 : 0, a.H, a.S1, out, o_sb, o_sh);
     else if (D == 256)
       hipLaunchKernelGGL((decode_stage2<256>), dim3(a.B * a.H), dim3(128), 0, stream, a.logits, a.lse,
-                         a.num_kv_splits, a.split_cap, a.neutral, a.H, a.S1, out, o_sb, o_sh);
+                         a.num_kv_splits, a.split_cap, a.neutral, a.blocks ? 1 : 0, a.H, a.S1, out, o_sb, o_sh);
     else
       return hipErrorInvalidValue;
   }

@@ -5,6 +5,8 @@
 
 namespace rolaq {
 
+constexpr int kShareRequests = 256;  // the most requests whose lengths decode's blocks are shared by
+
 struct DecodeArgs {
   const uint16_t* q;
   int64_t q_sb, q_sh;
@@ -21,6 +23,8 @@ struct DecodeArgs {
   int split_cap;  // request b uses min(num_kv_splits[b], split_cap) splits
   int neutral;    // 1: split nq carries the window split's neutral partial; 0: no such partial (fused call)
   int S1;        // max_kv_splits + 1
+  int blocks;    // > 0: blocks per head block, shared by the requests by their lengths (fused call); 0: equal rows
+  int blocks_each;  // blocks / B
   int max_reqs;  // requests with ring rows; req_idx outside [0, max_reqs) reads no window rows
   int B, H, P, W;
   float sm_scale;

@@ -256,9 +256,9 @@ def decode_fwd(q: torch.Tensor, codes: torch.Tensor, params: torch.Tensor, rope_
 
     ``max_reqs``: requests with ring rows in ``hp_c`` (default: as many as its
     rows hold); a ``req_idx`` outside ``[0, max_reqs)`` reads no window rows.
-    Request ``b`` uses ``min(num_kv_splits[b], decode_split_cap(...))`` splits
-    (about one working block per compute unit); the partials in
-    ``attn_logits``/``attn_lse`` follow that count."""
+    Request ``b`` uses at most ``min(num_kv_splits[b], decode_split_cap(...))``
+    splits, by its length where the batch asks for more than one working block
+    per compute unit; ``attn_logits``/``attn_lse`` are scratch."""
     B, H, D, R = _decode_check(q, codes, params, rope_buf, hp_c, kv_indptr, kv_indices, seq_lens, req_idx,
                                num_kv_splits, max_kv_splits, attn_logits, attn_lse)
     _out_check(out, B, H, D, q.device)
@@ -273,8 +273,8 @@ def decode_fwd(q: torch.Tensor, codes: torch.Tensor, params: torch.Tensor, rope_
 
 def decode_split_cap(B: int, H: int, D: int, max_kv_splits: int) -> int:
     """The most splits :func:`decode_fwd` gives one request on the current
-    device: enough quantized splits for one working block per compute unit
-    over the batch, plus the window split, at most ``max_kv_splits``."""
+    device (a batch shares one working block per compute unit by its lengths),
+    the window split included, at most ``max_kv_splits``."""
     cap = ctypes.c_int(0)
     _lib.check(_lib.load().rolaq_decode_split_cap(int(B), int(H), int(D), int(max_kv_splits), ctypes.byref(cap)))
     return cap.value

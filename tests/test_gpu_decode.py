@@ -365,3 +365,41 @@ def test_output_independent_of_page_layout(D, R, H):
     for out, lse in results[1:]:
         assert torch.equal(out, results[0][0])
         assert torch.equal(lse.nan_to_num(0.0), results[0][1].nan_to_num(0.0))
+
+
+@pytest.mark.parametrize("D,R,H,lengths,ns", [
+    (512, 64, 16, [4000, 17] + [33 + 61 * i for i in range(14)], 129),   # 16 requests, one much longer
+    (512, 64, 16, [0, 5, 9000, 0, 40, 31], 129),                          # empty, window-only and one long request
+    (512, 64, 16, [300 + 7 * i for i in range(70)], 33),                  # more than 64 requests
+    (512, 64, 16, [64 + (97 * i) % 900 for i in range(250)], 3),          # nearly as many requests as compute units
+    (256, 32, 40, [700] * 24, 129),                                       # equal lengths that do not divide the CUs
+    (256, 32, 64, [1500, 90, 700, 2100] * 3, 65),                         # two head blocks
+    (512, 64, 128, [600, 2500, 37, 1100, 900], 40),                       # eight head blocks
+], ids=["one_long", "empties", "b70", "b250", "equal24", "h64", "h128"])
+def test_blocks_shared_by_length(D, R, H, lengths, ns):
+    """More splits asked for than compute units: every request's share follows
+    its length. Output and merged LSE against the oracle, the counts stage 1
+    left (last LSE slot of a head) fit one block per CU, and no block has more
+    units than m = total / (blocks - requests) + 1, at which sum(ceil(U_b / m))
+    <= total / m + requests <= blocks, or than all splits asked for leave it."""
+    P, W = 4, 16
+    sm = 1 / math.sqrt(192 if D == 512 else 96)
+    B = len(lengths)
+    gp, slots, pages, reqs = gpu_written_pool(lengths, D, R, P, W, 64, seed=71)
+    q = make_queries(B, H, D, R, sm, seed=73)
+    out, _, lse = run_decode(gp, q, slots, pages, lengths, reqs, 64, [ns] * B, ns, P, W, sm)
+    sample = sorted(set([0, 1, 2, B // 2, B - 1]) - {b for b in range(B) if lengths[b] == 0})
+    check_against_oracle(gpu_pool_to_oracle(gp), q, out, lse, slots, lengths, reqs, [ns] * B, P, W, sm, D,
+                         batch_index=sample, max_splits=ns)
+    assert (out[[b for b in range(B) if lengths[b] == 0]] == 0).all()
+    last = max(min(kernels.decode_split_cap(B, H, D, ns) - 1, ns), 1)
+    used = lse[:, :, last].contiguous().view(torch.int32) & 0xFFF
+    assert (used == used[:, :1]).all() and (used >= 1).all()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = cus // (-(-H // 16) if D == 512 else -(-H // 48))
+    units = torch.tensor([0 if L == 0 else 1 + (max(-(-(L - W) // 32), 0) if L > P + W else 0) for L in lengths])
+    assert used[:, 0].sum() <= blocks
+    per_block = torch.ceil(units / used[:, 0])
+    m = int(units.sum()) // (blocks - B) + 2  # (one more: the rounding of 1/m)
+    asked = min(ns, kernels.decode_split_cap(B, H, D, ns)) - 1
+    assert (per_block <= torch.clamp(torch.ceil(units / asked), min=m)).all()
