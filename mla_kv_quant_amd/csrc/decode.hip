@@ -204,9 +204,11 @@ __device__ __forceinline__ int units_of(int L, int P, int W) {
 // otherwise as many as leave every block at most m units (tiles), with about
 // the smallest m for which the blocks suffice. Equal lengths get equal counts.
 // With equal counts for all, the launch waits for the longest request's blocks:
-// stage 1 of 16 requests of 1024 .. 16384 tokens took 27 us, now 21; of 128
-// requests of 2048 .. 8192, 69.8 us, now 63.7 (a whole decode: 71 -> 65.5 us a
-// layer); 32 requests of 16384 are where they were (46.5 us a layer).
+// a decode of 16 requests of 1024 .. 16384 tokens (16 heads, D = 512) took 26.4 us
+// a layer, now 23.1; of 128 requests of 2048 .. 8192, 71.6, now 62.2. Equal ones
+// have the partition they had; the metadata through lanes costs the launch
+// nothing that the query's loads (load_q) do not give back: 16 requests of 4096
+// tokens 21.1 us a layer with and without the sharing, 32 of 16384 50.7 and 50.6.
 struct Share {
   int b = 0, split = 0, nq = 1;
   int first = 0;        // blocks before the request's
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   // the query's loads, which the first tile needs only after two more round
   // trips (page lookups, tile data). With NC > 0 the metadata is here already:
   // the query's loads then go out behind the page lookups (loads return in
-  // order) and are waited for behind the first tile's.
+  // order).
   int ns_req, kv0, kv1;
   int64_t req, slv;
   if constexpr (NC == 0) {
@@ -380,7 +382,33 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     slv = (a.seq_lens ? a.seq_lens : a.req_idx)[b];  // no branch before the loads
   }
   u32x4 qB[HG][KL], qR[HG][KR];
+  // Shared blocks at D = 512 read the heads' rows whole, each wave for itself,
+  // and bring them into the operands' layout through its LDS buffer (setup). In
+  // the operands' layout a load touches 64 lines; behind the metadata and beside
+  // the page lookups those loads kept the CU's texture path busy for 4600 cycles,
+  // with the first tile and the window's rows waiting behind them. Load j < KL
+  // holds head j, the last KR the 16 heads' rope.
+  // With the window wave's order below, us a layer, 16 heads, D = 512: 8 requests
+  // of 4096 tokens 20.9 -> 19.7 (19.8 at the unshared split count), 16 22.2 -> 21.0
+  // (21.2), 64 31.3 -> 30.3 (30.5); 16 of 1024 .. 16384 24.0 -> 23.2, 128 of 2048 ..
+  // 8192 62.7 -> 61.5. At D = 256 three head groups go through LDS, or a load has
+  // half the lines: 16 x 4096, 40 heads 24.3, in the operands' layout 23.4.
+  constexpr bool kWholeRows = NC > 0 && D == 512;
+  constexpr int QROW = 2 * (D + R) + 16;  // LDS bytes of a head's row (padded)
+  const int hr = lane / (4 * KR), cr = lane % (4 * KR);  // the lane's head and chunk in a rope load
   auto load_q = [&]() {
+    if constexpr (kWholeRows) {
+#pragma unroll
+      for (int hg = 0; hg < HG; ++hg) {
+        const uint16_t* const qg = a.q + b * a.q_sb + (int64_t)(h0 + 16 * hg) * a.q_sh;
+        const int last = a.H - 1 - h0 - 16 * hg;  // heads past the last one read that again (and are masked)
+#pragma unroll
+        for (int j = 0; j < KL; ++j) qB[hg][j] = gload<u32x4>(qg + min(j, last) * a.q_sh + 8 * lane);
+#pragma unroll
+        for (int kr = 0; kr < KR; ++kr) qR[hg][kr] = gload<u32x4>(qg + min(16 / KR * kr + hr, last) * a.q_sh + D + 8 * cr);
+      }
+      return;
+    }
 #pragma unroll
     for (int hg = 0; hg < HG; ++hg) {
       const uint16_t* qh = a.q + b * a.q_sb + (int64_t)min(h0 + 16 * hg + la, a.H - 1) * a.q_sh;
@@ -475,15 +503,18 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb) wpg[mb] = page_of(win_pos(min(16 * mb + la, nw - 1)));
   };
-  auto window_rows = [&]() {
+  const uint16_t* wrow[2];
+  auto window_row_bases = [&]() {
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb) {
       const int pos = win_pos(min(16 * mb + la, nw - 1));
       const int inner = pos < P ? pos : P + (pos - P) % max(W, 1);
-      const uint16_t* row = a.hp + (1 + req * (P + W) + inner) * D + 128 * gl + 16 * s0;
-#pragma unroll
-      for (int j = 0; j < KL; ++j) wc[mb][j] = gload<u32x4>(row + 16 * (j / 2) + 8 * (j & 1));
+      wrow[mb] = a.hp + (1 + req * (P + W) + inner) * D + 128 * gl + 16 * s0;
     }
+  };
+  auto window_rows = [&](int j) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) wc[mb][j] = gload<u32x4>(wrow[mb] + 16 * (j / 2) + 8 * (j & 1));
   };
   auto window_rope = [&]() {
 #pragma unroll
@@ -764,11 +795,16 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   // block holding unit 0) has a prologue of its own: the window's ring rows go
   // out with the page lookups, its rope rows ahead of the first tile's loads,
   // and the window tile is computed before the paths join, where the loads
-  // in flight are the same (the first tile's) on both.
-  auto setup = [&]() {
+  // in flight are the same (the first tile's) on both. With shared blocks this
+  // wave is the launch's last: half of its ring rows go out between the set-up's
+  // conversions (all of them at once held up the rope rows behind 2000 cycles of
+  // the texture path), the first tile's loads behind the set-up (they have the
+  // window tile's time to land), and its buffer is left as it is (the window
+  // tile writes all of it).
+  auto setup = [&](auto fill, auto between) {
     // this wave's buffer starts as zeros (see the pending-output rule below),
-    // the softmax state, and the query operands (their loads went out with
-    // the metadata, ahead of the page lookups)
+    // the softmax state, and the query operands (unless blocks are shared,
+    // their loads went out with the metadata, ahead of the page lookups)
 #pragma unroll
     for (int hg = 0; hg < HG; ++hg) {
 #pragma unroll
@@ -777,13 +813,35 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
       l_lane[hg] = 0.f;
       Ph[hg] = u32x4{0u, 0u, 0u, 0u};
     }
+    if constexpr (kWholeRows) {
+      // whole rows to operands (one wave's LDS operations run in order)
+      static_assert(KL == 16 && 16 * QROW <= G::WBUF, "a head group's rows in the wave's buffer");
 #pragma unroll
-    for (int k = 0; k < G::WBUF / 1024; ++k) lds_store128(wbuf + 1024 * k + 16 * lane, u32x4{0u, 0u, 0u, 0u});
+      for (int hg = 0; hg < HG; ++hg) {
+#pragma unroll
+        for (int j = 0; j < KL; ++j) lds_store128(wbuf + QROW * j + 16 * lane, qB[hg][j]);
+#pragma unroll
+        for (int kr = 0; kr < KR; ++kr) lds_store128(wbuf + QROW * (16 / KR * kr + hr) + 2 * D + 16 * cr, qR[hg][kr]);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < KL; ++j) qB[hg][j] = lds_load128(wbuf + QROW * la + 16 * (16 * gl + 2 * (s0 + j / 2) + (j & 1)));
+#pragma unroll
+        for (int kr = 0; kr < KR; ++kr) qR[hg][kr] = lds_load128(wbuf + QROW * la + 16 * (D / 8 + 4 * kr + gq));
+        asm volatile("" ::: "memory");
+      }
+    }
+    if constexpr (fill()) {
+#pragma unroll
+      for (int k = 0; k < G::WBUF / 1024; ++k) lds_store128(wbuf + 1024 * k + 16 * lane, u32x4{0u, 0u, 0u, 0u});
+    }
 #pragma unroll
     for (int hg = 0; hg < HG; ++hg) {
       const bool hv = h0 + 16 * hg + la < a.H;
 #pragma unroll
-      for (int j = 0; j < KL; ++j) qB[hg][j] = bf16x8_to_f16x8(pi_permute(qB[hg][j])) & keep_mask(hv);
+      for (int j = 0; j < KL; ++j) {
+        qB[hg][j] = bf16x8_to_f16x8(pi_permute(qB[hg][j])) & keep_mask(hv);
+        if (hg == 0) between(j);
+      }
 #pragma unroll
       for (int kr = 0; kr < KR; ++kr) qR[hg][kr] &= keep_mask(hv);
     }
@@ -798,19 +856,32 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     }
   };
   bool first = true;
+  auto nothing = [](int) {};
   if (win_mine) {
     lookup(0, pgc);
     lookup(min(1, nl), pgn);
     window_pages();
-    window_rows();
-    if constexpr (NC > 0) load_q();
+    if constexpr (NC > 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_q();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    window_row_bases();
+#pragma unroll
+    for (int j = 0; j < (NC == 0 ? KL : KL / 2); ++j) window_rows(j);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (NC == 0) setup();
+    if constexpr (NC == 0) setup(std::true_type{}, nothing);
     __builtin_amdgcn_sched_barrier(0);
     window_rope();
+    if constexpr (NC > 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      setup(std::false_type{}, [&](int j) {
+        if (j >= KL / 2) window_rows(j);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    }
     load(0, pgc, dn);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (NC > 0) setup();
     __builtin_amdgcn_sched_barrier(0);
     window_tile();
     first = false;
@@ -820,11 +891,11 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (NC > 0) load_q();
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (NC == 0) setup();
+    if constexpr (NC == 0) setup(std::true_type{}, nothing);
     __builtin_amdgcn_sched_barrier(0);
     load(0, pgc, dn);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (NC > 0) setup();
+    if constexpr (NC > 0) setup(std::true_type{}, nothing);
   }
   __builtin_amdgcn_sched_barrier(0);
 

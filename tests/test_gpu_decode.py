@@ -403,3 +403,30 @@ def test_blocks_shared_by_length(D, R, H, lengths, ns):
     m = int(units.sum()) // (blocks - B) + 2  # (one more: the rounding of 1/m)
     asked = min(ns, kernels.decode_split_cap(B, H, D, ns)) - 1
     assert (per_block <= torch.clamp(torch.ceil(units / asked), min=m)).all()
+
+
+@pytest.mark.parametrize("D,R,heads", [(512, 64, [1, 15, 16, 17, 33]), (256, 32, [1, 2, 15, 17, 33, 40, 47, 48, 49, 64, 97])])
+def test_shared_blocks_read_every_head_of_a_strided_query(D, R, heads):
+    """Shared blocks at D = 512 read the query in whole rows, past the last head
+    that one again: head counts around a group of 16 and a block's three groups,
+    equal and ragged lengths, head rows further apart than D + R and in a batch of
+    another stride. Against the same call at a split count that does not share
+    (the operands' own layout), the readers' bar; the same bits as with a
+    contiguous query."""
+    P, W, page = 4, 16, 16
+    sm = 1 / math.sqrt(192 if D == 512 else 96)
+    for lengths in ([700] * 9, [1500, 40, 900, 3, 60, 333, 21, 800, 64]):
+        B = len(lengths)
+        gp, slots, pages, reqs = gpu_written_pool(lengths, D, R, P, W, page, seed=5)
+        for H in heads:
+            q = make_queries(B, H, D, R, sm, seed=H)
+            wide = torch.full((B + 1, H + 2, D + R + 24), float("nan"), dtype=torch.bfloat16, device=DEV)
+            wide[:B, :H, :D + R] = q.to(DEV)
+            assert kernels.decode_split_cap(B, H, D, 200) - 1 > torch.cuda.get_device_properties(0).multi_processor_count // (
+                B * -(-H // (16 if D == 512 else 48)))  # more asked for than a block per unit: shared
+            args = (slots, pages, lengths, reqs, page)
+            out, _, _ = run_decode(gp, q, *args, [200] * B, 200, P, W, sm)
+            strided, _, _ = run_decode(gp, wide[:B, :H, :D + R], *args, [200] * B, 200, P, W, sm)
+            plain, _, _ = run_decode(gp, q, *args, [3] * B, 3, P, W, sm)
+            assert torch.equal(out, strided), H
+            torch.testing.assert_close(out, plain, rtol=RTOL, atol=ATOL)
