@@ -166,13 +166,16 @@ __device__ __forceinline__ int64_t add_dpp(int64_t v) {
   const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xF, false);
   return v + (int64_t)((uint64_t)hi << 32 | lo);
 }
-__device__ __forceinline__ int64_t wave_sum64(int64_t v) {
+__device__ __forceinline__ int64_t wave_scan64(int64_t v) {  // inclusive; lane 63 has the sum
   v = add_dpp<0x111, 0xF>(v);  // row_shr 1, 2, 4, 8: lane 15 of a row has its total
   v = add_dpp<0x112, 0xF>(v);
   v = add_dpp<0x114, 0xF>(v);
   v = add_dpp<0x118, 0xF>(v);
   v = add_dpp<0x142, 0xA>(v);  // lane 15 of rows 0 and 2 to rows 1 and 3
-  v = add_dpp<0x143, 0xC>(v);  // lane 31 to rows 2 and 3
+  return add_dpp<0x143, 0xC>(v);  // lane 31 to rows 2 and 3
+}
+__device__ __forceinline__ int64_t wave_sum64(int64_t v) {
+  v = wave_scan64(v);
   const uint32_t lo = __builtin_amdgcn_readlane((int)v, 63), hi = __builtin_amdgcn_readlane((int)(v >> 32), 63);
   return (int64_t)((uint64_t)hi << 32 | lo);
 }
@@ -207,13 +210,18 @@ __device__ __forceinline__ bool scratch_is_free(const ExtendArgs& a) {
 // same chunk of its blocks lands on one XCD (blocks go to the 8 XCDs
 // round-robin), whose L2 then serves its key rows. The block's latency is the
 // gather's where there is little to gather, so every step is spread over
-// lanes (a first version with one thread per sequence took 20 us).
+// lanes (a first version with one thread per sequence took 20 us), and its cost
+// grows with the batch as the gather's does: lengths are read once per stage of
+// kStage sequences, places come from scans (with every sequence counting those
+// before it, 1000 chunks of 4 queries over 2500 keys took 2990 us, 2430 without
+// a plan, now 2400; 4000 of one over 1200 keys 23900, 7700 and 7740).
 template <int D, int R>
 __device__ void extend_plan(const ExtendArgs& a) {
   constexpr int KT = D == 256 ? 64 : 32;
-  constexpr int kCands = 32, kShares = 16;
+  constexpr int kCands = 32, kShares = 16, kStage = 512;
   __shared__ unsigned long long s_work, s_keys, s_n[kCands], s_slots[kCands];
   __shared__ int s_longest, s_mx[kCands];
+  __shared__ int s_seq[kStage][2];  // blocks and steps of a stage's sequences
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const ExtScratch x = ext_scratch(a.scratch, a.max_items, a.max_slots);
   if (tid == 0) s_work = 0, s_keys = 0, s_longest = 0;
@@ -244,6 +252,7 @@ __device__ void extend_plan(const ExtendArgs& a) {
     int longest = 0;
     for (int b = tid; b < a.B; b += blockDim.x) {
       const Shape s = shape(b);
+      if (b < kStage) s_seq[b][0] = s.blocks, s_seq[b][1] = s.steps;
       keys += s.keys;
       if (s.blocks) work += (int64_t)s.blocks * (steps_of(s, kExtRows - 1) + s.steps) / 2;
       longest = max(longest, s.steps);
@@ -272,14 +281,24 @@ __device__ void extend_plan(const ExtendArgs& a) {
     const int c = tid % kCands, kc = chunk_of(c);
     unsigned long long n_all = 0, slots = 0;
     int mx = 0;
-    for (int b = tid / kCands; b < a.B; b += blockDim.x / kCands) {
-      const Shape s = shape(b);
-      if (s.blocks == 0) continue;
-      int n, len;
-      cut(s.steps, kc, n, len);
-      n_all += (unsigned long long)s.blocks * n;
-      if (n > 1) slots += (unsigned long long)s.blocks * n;
-      mx = max(mx, len);
+    for (int b0 = 0; b0 < a.B; b0 += kStage) {
+      const int m = min(kStage, a.B - b0);
+      if (b0 > 0) {
+        __syncthreads();
+        for (int i = tid; i < m; i += blockDim.x) {
+          const Shape s = shape(b0 + i);
+          s_seq[i][0] = s.blocks, s_seq[i][1] = s.steps;
+        }
+        __syncthreads();
+      }
+      for (int i = tid / kCands; i < m; i += blockDim.x / kCands) {
+        const int blocks = s_seq[i][0];
+        int n, len;
+        cut(s_seq[i][1], kc, n, len);
+        n_all += (unsigned long long)blocks * n;  // (a sequence without blocks has no steps: n = 0)
+        if (n > 1) slots += (unsigned long long)blocks * n;
+        mx = max(mx, len);
+      }
     }
     if (tid / kCands < a.B) {
       atomicAdd(&s_n[c], n_all);
@@ -314,69 +333,105 @@ __device__ void extend_plan(const ExtendArgs& a) {
     mx = s_mx[pick];
   }
   const int kc = chunk_of(pick);
-  // A sequence's items, partials and merges start behind those of the
-  // sequences before it, the ones with long chunks first; each is written by
-  // one wave, or by several where there are fewer sequences than waves.
-  const int waves = blockDim.x / 64, share_w = a.B < waves ? waves / a.B : 1;
-  for (int b = wave / share_w; b < a.B; b += waves / share_w) {
-    int64_t items = 0, slots = 0, merges = 0, koff = 0;  // of the sequences before b (koff: in batch order)
-    int n, len;
-    const Shape s = shape(b);
-    cut(s.steps, kc, n, len);
-    const bool late = 4 * len < 3 * mx;
-    for (int i = lane; i < a.B; i += 64) {
-      const Shape si = shape(i);
-      int ni, li;
-      cut(si.steps, kc, ni, li);
-      const bool late_i = 4 * li < 3 * mx;
-      const bool before = late_i == late ? i < b : late;
-      if (before) {
-        items += (int64_t)si.blocks * ni;
-        if (ni > 1) slots += (int64_t)si.blocks * ni, merges += si.blocks;
-      }
-      if (i < b) koff += si.keys;
+  // A sequence's items start behind those of the sequences before it, the ones
+  // with long chunks first; its partials, merges and key rows in batch order. A
+  // wave, or a group of waves where there are fewer, takes the sequences of a
+  // range 64 at a time, a lane each: scans give the places, and the 64 sequences'
+  // items are written an item per lane, which finds its sequence in the scan.
+  struct Places {
+    int64_t early, late, marks, keys;  // items by class, merges << 32 | partials, key rows
+  };
+  struct Seq {
+    Shape s;
+    int n, len, items;
+    bool late;
+  };
+  auto sequence = [&](int b) {
+    Seq q{};
+    if (b < a.B) {
+      q.s = shape(b);
+      cut(q.s.steps, kc, q.n, q.len);
+      q.items = q.s.blocks * q.n;
+      q.late = 4 * (int64_t)q.len < 3 * (int64_t)mx;
     }
-    const int base = (int)wave_sum64(items), slot = (int)wave_sum64(slots), mrg = (int)wave_sum64(merges);
-    koff = wave_sum64(koff);
-    const int32_t qo0 = a.qo_indptr[b];
-    const int sub = wave % share_w;
-    for (int j = lane + 64 * sub; j < s.blocks * n; j += 64 * share_w) {
+    return q;
+  };
+  auto places = [](const Seq& q) {
+    return Places{q.late ? 0 : q.items, q.late ? q.items : 0,
+                  q.n > 1 ? (int64_t)q.s.blocks << 32 | q.items : 0, q.s.keys};
+  };
+  const int waves = blockDim.x / 64, chunks = (a.B + 63) / 64, groups = min(waves, chunks), per = waves / groups;
+  const int group = min(wave / per, groups - 1), sub = wave - group * per;
+  const int c0 = chunks * group / groups, c1 = chunks * (group + 1) / groups;
+  __shared__ Places s_range[4];
+  Places at{0, 0, 0, 0}, all{0, 0, 0, 0};
+  {
+    Places mine{0, 0, 0, 0};
+    for (int c = c0; c < c1; ++c) {
+      const Places p = places(sequence(64 * c + lane));
+      mine.early += p.early, mine.late += p.late, mine.marks += p.marks, mine.keys += p.keys;
+    }
+    mine.early = wave_sum64(mine.early), mine.late = wave_sum64(mine.late);
+    mine.marks = wave_sum64(mine.marks), mine.keys = wave_sum64(mine.keys);
+    if (groups == 1) {
+      all = mine;
+    } else {
+      if (lane == 0 && sub == 0) s_range[group] = mine;
+      __syncthreads();
+      for (int g = 0; g < groups; ++g) {
+        const Places p = s_range[g];
+        if (g < group) at.early += p.early, at.late += p.late, at.marks += p.marks, at.keys += p.keys;
+        all.early += p.early, all.marks += p.marks;
+      }
+    }
+  }
+  if (tid == 0) x.head->items = (int)s_n[pick], x.head->merges = (int)(all.marks >> 32);
+  if (sub >= per) return;  // (waves that divide into no group)
+  at.late += all.early;
+  for (int c = c0; c < c1; ++c) {
+    const int b = 64 * c + lane;
+    const Seq q = sequence(b);
+    const Places mine = places(q);
+    const Places incl{wave_scan64(mine.early), wave_scan64(mine.late), wave_scan64(mine.marks), wave_scan64(mine.keys)};
+    const int upto = (int)(incl.early + incl.late);  // the items up to this sequence's last
+    const int base = (int)(q.late ? at.late + incl.late : at.early + incl.early) - q.items;
+    const int64_t marks = at.marks + incl.marks - mine.marks;
+    const int slot0 = (int)(uint32_t)marks, merge0 = (int)(marks >> 32);
+    const int64_t koff = at.keys + incl.keys - q.s.keys;
+    const int qo0 = b < a.B ? a.qo_indptr[b] : 0;
+    const int total = __shfl(upto, 63), live = min(64, a.B - 64 * c);
+    const int top = live > 1 ? 1 << (31 - __clz(live - 1)) : 0;
+    for (int j0 = 64 * sub; j0 < total; j0 += 64 * per) {
+      const int jj = min(j0 + lane, total - 1);
+      int l = 0;  // the sequences whose items all come before item jj
+      for (int step = top; step > 0; step >>= 1)
+        if (__shfl(upto, l + step - 1) <= jj) l += step;
+      const int items = __shfl(q.items, l), j = jj - (__shfl(upto, l) - items);
+      Shape s;
+      s.prefix = __shfl(q.s.prefix, l), s.rows = __shfl(q.s.rows, l), s.blocks = __shfl(q.s.blocks, l);
+      const int n = __shfl(q.n, l), len = __shfl(q.len, l), first = __shfl(base, l), slot = __shfl(slot0, l);
+      const int merge = __shfl(merge0, l);
       // item j: chunks in groups of 8 (fewer at the end), blocks in turn within a group
-      const int group = j / (8 * s.blocks), width = min(8, n - 8 * group), k = j - 8 * s.blocks * group;
-      const int c = 8 * group + k % width, blk = s.blocks - 1 - k / width;  // later blocks first
+      const int eight = j / (8 * s.blocks), width = min(8, n - 8 * eight), k = j - 8 * s.blocks * eight;
+      const int chunk = 8 * eight + k % width, blk = s.blocks - 1 - k / width;  // later blocks first
       ExtItem it;
       it.r0 = (int64_t)blk * kExtRows;
       it.nrows = s.rows;
-      it.koff = koff;
-      it.qo0 = qo0;
+      it.koff = __shfl(koff, l);
+      it.qo0 = __shfl(qo0, l);
       it.prefix = (int32_t)s.prefix;
       const int end = steps_of(s, it.r0 + kExtRows - 1);  // the block's own steps
-      it.s0 = min(c * len, end);
-      it.s1 = min((c + 1) * len, end);
-      it.slot = end > len ? slot + blk * n + c : -1;
-      x.items[base + j] = it;
-    }
-    if (n > 1)
-      for (int blk = lane + 64 * sub; blk < s.blocks; blk += 64 * share_w) {
-        ExtMerge m;
-        m.r0 = (int64_t)blk * kExtRows;
-        m.nrows = s.rows;
-        m.qo0 = qo0;
-        m.slot0 = slot + blk * n;
-        m.n = (steps_of(s, m.r0 + kExtRows - 1) + len - 1) / len;
-        x.merges[mrg + blk] = m;
+      it.s0 = min(chunk * len, end);
+      it.s1 = min((chunk + 1) * len, end);
+      it.slot = end > len ? slot + blk * n + chunk : -1;
+      if (j0 + lane < total) {
+        x.items[first + j] = it;
+        if (n > 1 && chunk == 0)
+          x.merges[merge + blk] = ExtMerge{it.r0, s.rows, it.qo0, slot + blk * n, (end + len - 1) / len, 0};
       }
-  }
-  if (wave == waves - 1) {
-    int64_t merges = 0;
-    for (int i = lane; i < a.B; i += 64) {
-      const Shape si = shape(i);
-      int ni, li;
-      cut(si.steps, kc, ni, li);
-      if (ni > 1) merges += si.blocks;
     }
-    merges = wave_sum64(merges);
-    if (lane == 0) x.head->items = (int)s_n[pick], x.head->merges = (int)merges;
+    at.early += __shfl(incl.early, 63), at.late += __shfl(incl.late, 63);
+    at.marks += __shfl(incl.marks, 63), at.keys += __shfl(incl.keys, 63);
   }
 }
 

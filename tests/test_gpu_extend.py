@@ -401,3 +401,96 @@ def test_extend_with_split_keys_matches_unsplit(D, R, H, prefixes, chunks):
         ref, _ = attention.extend(pool, q[s:e, :, :D], q[s:e, :, D:], kc[s:e, :D], kc[s:e, D:], slots[b],
                                   prefixes[b], int(reqs[b]), P, W, sm, D, dtype=torch.float64)
         torch.testing.assert_close(split[s:e].double().cpu(), ref, rtol=RTOL, atol=ATOL)
+
+
+def _batch(B, seed, prefix, chunk, empty=0.0):
+    """Lengths of B sequences up to twice their means, a share of them without a chunk."""
+    r = np.random.default_rng(seed)
+    return ([int(v) for v in r.integers(0, 2 * prefix + 1, B)],
+            [0 if r.random() < empty else int(v) for v in r.integers(1, 2 * chunk + 1, B)])
+
+
+@pytest.mark.parametrize("D,H,prefixes,chunks", [
+    (512, 16, [9000, 50], [40, 300]),
+    (256, 40, [3000, 0, 7000], [5, 70, 33]),                # three sequences, four waves
+    (512, 16, *_batch(64, 1, 1300, 20)),                    # one chunk of lanes
+    (512, 16, *_batch(65, 2, 1300, 20, empty=0.3)),         # and one more sequence, some without a chunk
+    (256, 16, *_batch(130, 3, 2300, 6)),
+    (512, 16, *_batch(300, 4, 1700, 3, empty=0.2)),         # as many ranges as waves
+    (256, 8, *_batch(1200, 5, 2300, 2)),                    # more than two stages of lengths
+    (512, 16, [200] * 90 + [60000], [2] * 91),              # one long sequence behind many short ones
+], ids=["b2", "b3", "b64", "b65", "b130", "b300", "b1200", "long_last"])
+def test_extend_plan_covers_every_key_of_every_row_once(D, H, prefixes, chunks):
+    """The plan that the call left in the workspace's last rows, against its
+    rules: every block of 128 query rows has its keys cut into steps without gap
+    or overlap, partial slots are its own and consecutive, merges name them, and
+    places in the workspace are the running sums of the lengths. The output is
+    that of a workspace without a plan up to the readers' bar."""
+    R, P, W, page, pages = D // 8, 4, 16, 16, 64
+    B, T, KT = len(chunks), sum(chunks), 64 if D == 256 else 32
+    g = torch.Generator(device=DEV).manual_seed(B)
+    codes = torch.randint(0, 256, (pages * page, D // 4), dtype=torch.uint8, device=DEV, generator=g)
+    params = torch.tensor([1.1, 1.5], device=DEV).expand(pages * page, D // 128, 2).contiguous()
+    rope = torch.randn(pages * page, R, device=DEV, generator=g).bfloat16()
+    hp = torch.randn(1 + (B + 1) * (P + W), D, device=DEV, generator=g).bfloat16()
+    counts = [-(-n // page) for n in prefixes]
+    indptr = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32, device=DEV)
+    indices = torch.randint(0, pages, (max(sum(counts), 1),), dtype=torch.int32, device=DEV, generator=g)
+    sm = 1.0 / math.sqrt(96 if D == 256 else 192)
+    q = (torch.randn(T, H, D + R, device=DEV, generator=g) * (2.0 / (sm * math.sqrt(D + R)))).bfloat16()
+    kc = torch.randn(T, D + R, device=DEV, generator=g).bfloat16()
+    qo = torch.tensor(np.concatenate([[0], np.cumsum(chunks)]), dtype=torch.int32, device=DEV)
+    rows = sum(prefixes) + T
+    spare = kernels.extend_scratch_rows(B, H, D, R, max(chunks), rows)
+    assert spare > 0
+
+    def run(ws):
+        out = torch.full((T, H, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        kernels.extend_fwd(q, kc, qo, indptr, indices, torch.tensor(prefixes, device=DEV),
+                           torch.arange(1, B + 1, device=DEV), codes, params, rope, hp, max(chunks), out, sm, P, W,
+                           page, workspace=ws, key_rows=rows)
+        torch.cuda.synchronize()
+        return out
+
+    ws = torch.empty(rows + spare, D + R, dtype=torch.float16, device=DEV).fill_(float("nan"))
+    split = run(ws)
+    whole = run(torch.empty(rows, D + R, dtype=torch.float16, device=DEV))
+    torch.testing.assert_close(split.float(), whole.float(), rtol=RTOL, atol=ATOL)
+
+    plan = ws[rows:].cpu().numpy().view(np.uint8).reshape(-1)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = -(-max(chunks) * H // 128) * B
+    max_items = blocks + min(2 * cus, blocks * -(-(-(-rows // KT)) // 4))
+    n_items, n_merges = plan[:8].view(np.int32)
+    item = np.dtype([("r0", "<i8"), ("nrows", "<i8"), ("koff", "<i8"), ("qo0", "<i4"), ("prefix", "<i4"), ("s0", "<i4"),
+                     ("s1", "<i4"), ("slot", "<i4"), ("pad", "<i4", 5)])
+    merge = np.dtype([("r0", "<i8"), ("nrows", "<i8"), ("qo0", "<i4"), ("slot0", "<i4"), ("n", "<i4"), ("pad", "<i4")])
+    items = plan[256:256 + 64 * n_items].view(item)
+    merges = plan[256 + 64 * max_items:][:32 * n_merges].view(merge)
+    assert 0 < n_items <= max_items
+    koffs = np.concatenate([[0], np.cumsum(np.asarray(prefixes) + np.asarray(chunks))])
+    by_place = {}
+    for it in items:
+        by_place.setdefault((int(it["koff"]), int(it["r0"])), []).append(it)
+    by_merge = {(int(m["qo0"]), int(m["r0"])): m for m in merges}
+    used, n_blocks = set(), 0
+    for b in range(B):
+        for r0 in range(0, chunks[b] * H, 128):
+            n_blocks += 1
+            mine = sorted((it for it in by_place[(int(koffs[b]), r0)] if it["s0"] < it["s1"]), key=lambda it: it["s0"])
+            last_row = min(r0 + 127, chunks[b] * H - 1)
+            assert [it["s0"] for it in mine] == [0] + [it["s1"] for it in mine[:-1]]
+            assert mine[-1]["s1"] == (prefixes[b] + last_row // H) // KT + 1
+            assert all(it["nrows"] == chunks[b] * H and it["qo0"] == int(qo[b]) and it["prefix"] == prefixes[b] for it in mine)
+            slots = [int(it["slot"]) for it in mine]
+            if len(mine) == 1:
+                assert slots == [-1]
+                continue
+            m = by_merge[(int(qo[b]), r0)]
+            assert m["n"] == len(mine) and m["nrows"] == chunks[b] * H
+            assert slots == list(range(m["slot0"], m["slot0"] + len(mine)))
+            assert not used.intersection(slots) and max(slots) < 2 * cus
+            used.update(slots)
+    assert n_blocks == sum(-(-c * H // 128) for c in chunks)
+    assert len({(int(it["koff"]), int(it["r0"]), int(it["s0"])) for it in items if it["s0"] < it["s1"]}) == \
+        sum(it["s0"] < it["s1"] for it in items)
