@@ -58,9 +58,9 @@ _Tensor = torch.Tensor
 
 
 def _need_all(device, specs):
-    """``specs``: (tensor, name, dtype, ndim) of contiguous tensors on ``device``."""
+    """``specs``: (tensor, name, dtype, ndim or None) of contiguous tensors on ``device``."""
     for t, name, dtype, ndim in specs:
-        if isinstance(t, _Tensor) and t.dtype is dtype and t.device == device and t.ndim == ndim \
+        if isinstance(t, _Tensor) and t.dtype is dtype and t.device == device and (ndim is None or t.ndim == ndim) \
                 and t.is_contiguous():
             continue
         _need(t, name, dtype, device, ndim)
@@ -104,7 +104,8 @@ def _check_writer(latent, k_pe, rotation_t, loc, seq_lens, positions, req_idx, c
     i64, i32 = torch.int64, torch.int32
     _need_all(dev, ((loc, "loc", i64, 1), (seq_lens, "seq_lens", i64, 1), (req_idx, "req_idx", i64, 1)))
     if loc.shape[0] != n or seq_lens.shape[0] != n or req_idx.shape[0] != n:
-        raise ValueError(f"loc, seq_lens and req_idx must have {n} entries")
+        name = "loc" if loc.shape[0] != n else "seq_lens" if seq_lens.shape[0] != n else "req_idx"
+        raise ValueError(f"{name} must have {n} entries")
     if positions is not None:
         _need_all(dev, ((positions, "positions", i64, 1),))
         if positions.shape[0] != n:
@@ -390,10 +391,9 @@ def assemble_rows(slots: torch.Tensor, codes: torch.Tensor, params: torch.Tensor
     _contig(slots, "slots")
     D = codes.shape[1] * 4
     R = rope_buf.shape[1]
-    _need_all(dev, ((codes, "codes", torch.uint8, codes.ndim), (params, "params", torch.float32, params.ndim),
-                    (rope_buf, "rope_buf", torch.bfloat16, rope_buf.ndim), (hp_c, "hp_c", torch.bfloat16, hp_c.ndim),
-                    (row_of_slot, "row_of_slot", torch.int32, row_of_slot.ndim),
-                    (owner_of_row, "owner_of_row", torch.int32, owner_of_row.ndim)))
+    _need_all(dev, ((codes, "codes", torch.uint8, None), (params, "params", torch.float32, None),
+                    (rope_buf, "rope_buf", torch.bfloat16, None), (hp_c, "hp_c", torch.bfloat16, None),
+                    (row_of_slot, "row_of_slot", torch.int32, None), (owner_of_row, "owner_of_row", torch.int32, None)))
     if hp_c.shape[1] != D or tuple(params.shape[1:]) != (D // GROUP_SIZE, 2):
         raise ValueError("cache buffers do not match")
     if rotation is not None:
