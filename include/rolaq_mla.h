@@ -269,8 +269,11 @@ int rolaq_extend_fwd(const void* q, int64_t q_stride_t, int64_t q_stride_h, cons
 /*
  * Workspace rows past key_rows with which rolaq_extend_fwd splits keys on the
  * current device, written to *rows (0: it would not split). At most
- * 2 * compute units * 128 * D * 4 bytes of partials and a few hundred KB. Host
- * only: no launch, no synchronisation. No counterpart in the reference.
+ * 2 * compute units * (128 * (D + 1) * 4 + 96) bytes of partials, and 64 bytes
+ * for each block of 128 (token, head) query rows that B chunks of max_q_len
+ * tokens would have (more than 2^20 of them, 67 MB, are not split): 202 MB at
+ * D = 512 and 135 MB at D = 256 on 256 compute units. Host only: no launch, no
+ * synchronisation. No counterpart in the reference.
  */
 int rolaq_extend_scratch_rows(int B, int H, int D, int R, int max_q_len, int64_t key_rows, int64_t* rows);
 

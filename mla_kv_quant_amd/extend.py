@@ -32,7 +32,7 @@ def packed_mla_extend_fwd(q, k, o, pool, layer_id, qo_indptr, kv_indptr, kv_indi
     scratch with ``rows >= sum(prefix_lens) + T`` (with
     ``kernels.extend_scratch_rows`` more, keys can be split over compute
     units); when omitted the pool's own workspace is used (kept across layers
-    and calls, grown as needed).
+    and calls, replaced only by a batch of more key rows than any before).
     """
     li = layer_id - pool.start_layer
     if k.dim() == 3:
@@ -49,8 +49,7 @@ def packed_mla_extend_fwd(q, k, o, pool, layer_id, qo_indptr, kv_indptr, kv_indi
     else:
         key_rows = int(pl[:B].sum().item()) + int(q.shape[0])
     if workspace is None:
-        extra = kernels.extend_scratch_rows(B, q.shape[1], pool.kv_lora_rank, pool.qk_rope_head_dim, max_q_len, key_rows)
-        workspace = pool.extend_workspace(key_rows + extra)
+        workspace = pool.extend_workspace(key_rows)
     return kernels.extend_fwd(q, k, qo_indptr, kv_indptr, kv_indices, pl, req, pool.c_codes[li], pool.c_params[li],
                               pool.rope_buf[li], pool.hp_c[li], max_q_len, o, sm_scale, pool._win_p, pool._win_r,
                               page_size, max_reqs=pool._max_reqs, workspace=workspace, key_rows=key_rows)

@@ -314,14 +314,25 @@ def decode_merge(attn_logits: torch.Tensor, attn_lse: torch.Tensor, num_kv_split
     return out
 
 
+EXTEND_SPLIT_ROWS = 24 * 32  # fewer key rows are never split
+
+
 def extend_scratch_rows(B: int, H: int, D: int, R: int, max_q_len: int, key_rows: int) -> int:
     """Workspace rows past the key rows with which :func:`extend_fwd` splits
     keys over compute units (0: it would not)."""
-    if key_rows < 24 * 32:  # too few for any split
+    if key_rows < EXTEND_SPLIT_ROWS:
         return 0
     rows = ctypes.c_int64(0)
     _lib.check(_lib.load().rolaq_extend_scratch_rows(B, H, D, R, int(max_q_len), int(key_rows), ctypes.byref(rows)))
     return rows.value
+
+
+def extend_scratch_bound(D: int, R: int) -> int:
+    """The most that :func:`extend_scratch_rows` returns for any batch of
+    ``(D, R)`` on the current device (about 200 MB of rows at D = 512, 135 MB at
+    D = 256): the row blocks of the largest batch that is split, 2^20, and all
+    partial slots."""
+    return extend_scratch_rows(1, 128, D, R, 1 << 20, 1 << 40) if (D, R) in ((512, 64), (256, 32)) else 0
 
 
 def extend_fwd(q: torch.Tensor, k_chunk: torch.Tensor, qo_indptr: torch.Tensor, kv_indptr: torch.Tensor,
@@ -367,7 +378,9 @@ def extend_fwd(q: torch.Tensor, k_chunk: torch.Tensor, qo_indptr: torch.Tensor, 
     if key_rows is None:
         key_rows = int(prefix_lens[:B].sum().item()) + int(qo_indptr[B].item()) - int(qo_indptr[0].item())
     if workspace is None:
-        extra = extend_scratch_rows(B, H, D, R, max_q_len, key_rows)
+        # (a call that the library refuses is left to it)
+        taken = (D, R) in ((512, 64), (256, 32)) and 0 < H <= 4096 and max_q_len >= 0
+        extra = extend_scratch_rows(B, H, D, R, max_q_len, key_rows) if taken else 0
         workspace = torch.empty(max(int(key_rows) + extra, 1), DR, dtype=torch.float16, device=dev)
     if workspace.dtype not in (torch.bfloat16, torch.float16) or workspace.device != dev or workspace.dim() != 2:
         raise TypeError("workspace must be a 2-D bf16 or fp16 tensor on the query's device")

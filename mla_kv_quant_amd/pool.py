@@ -11,7 +11,7 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import GROUP_SIZE
+from .kernels import EXTEND_SPLIT_ROWS, GROUP_SIZE, extend_scratch_bound
 
 
 class PackedMLAPool:
@@ -62,8 +62,12 @@ class PackedMLAPool:
     def extend_workspace(self, rows: int) -> torch.Tensor:
         """The extend reader's scratch of at least ``rows`` key rows (fp16
         ``[rows, D + R]``): one buffer for every layer and call, reallocated
-        only when a batch needs more rows than it holds."""
+        only when a batch has more key rows than it holds. Behind the key rows
+        it has room to split any such batch's keys, so a batch of other shape
+        never replaces a buffer that a captured call reads."""
         need = max(int(rows), 1)
+        if need >= EXTEND_SPLIT_ROWS:
+            need += extend_scratch_bound(self.kv_lora_rank, self.qk_rope_head_dim)
         ws = self._extend_ws
         if ws is None or ws.shape[0] < need:
             ws = torch.empty(need, self.kv_lora_rank + self.qk_rope_head_dim, dtype=torch.float16,
