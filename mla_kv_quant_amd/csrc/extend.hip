@@ -541,7 +541,8 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   }
   if (!planned) {
     // heavier blocks (later tokens) first
-    const int b = blockIdx.x % a.B, y = a.row_blocks - 1 - blockIdx.x / a.B;
+    const int b = blockIdx.x % a.B;
+    const int y = a.row_blocks - 1 - (int)(blockIdx.x / a.B + blockIdx.y + gridDim.y * blockIdx.z);
     if (y < 0) return;
     it.qo0 = a.qo_indptr[b];
     const int64_t Tq = a.qo_indptr[b + 1] - it.qo0;
@@ -1129,13 +1130,16 @@ hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& args, int D, int R, int 
   const ExtPlanSize p = extend_plan_size(a.B, a.H, D, R, max_q_len, key_rows, num_cus);
   a.row_blocks = p.row_blocks;
   a.cus = num_cus;
-  int64_t blocks = (int64_t)p.row_blocks * a.B;
+  // the attend launch: an item per block, or (sequence, row block), the latter
+  // over two dimensions (in one, 2^24 blocks of 256 threads are too many to launch)
+  const unsigned ny = (unsigned)std::min(std::max(p.row_blocks, 1), 65535);
+  dim3 blocks((unsigned)a.B, ny, ((unsigned)p.row_blocks + ny - 1) / ny);
   if (p.rows > 0 && a.ws_rows - key_rows >= p.rows) {
     a.scratch = reinterpret_cast<uint8_t*>(a.ws + (a.ws_rows - p.rows) * (D + R));
     a.scratch_rows = p.rows;
     a.max_items = p.items;
     a.max_slots = p.slots;
-    blocks = p.items;
+    blocks = dim3((unsigned)p.items);
   }
   // gather: about 16 rows per block, 64 blocks per sequence at least (their
   // lengths may differ) and no more than 2048 in all
@@ -1150,7 +1154,7 @@ hipError_t rolaq_launch_extend(const rolaq::ExtendArgs& args, int D, int R, int 
     if (e != hipSuccess) return e;                                                                      \
     hipLaunchKernelGGL((extend_gather_kernel<DD, RR>), dim3((unsigned)a.B, (unsigned)(gy + (a.scratch ? 1 : 0))), \
                        dim3(256), 0, stream, a);                                                        \
-    hipLaunchKernelGGL((extend_kernel<DD, RR>), dim3((unsigned)blocks), dim3(64 * G::WAVES), lds, stream, a); \
+    hipLaunchKernelGGL((extend_kernel<DD, RR>), blocks, dim3(64 * G::WAVES), lds, stream, a);           \
     if (a.scratch)                                                                                      \
       hipLaunchKernelGGL((extend_merge_kernel<DD, RR>), dim3(16 * (unsigned)num_cus), dim3(256), 0, stream, a); \
     return hipGetLastError();                                                                           \

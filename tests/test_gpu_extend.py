@@ -494,3 +494,35 @@ def test_extend_plan_covers_every_key_of_every_row_once(D, H, prefixes, chunks):
     assert n_blocks == sum(-(-c * H // 128) for c in chunks)
     assert len({(int(it["koff"]), int(it["r0"]), int(it["s0"])) for it in items if it["s0"] < it["s1"]}) == \
         sum(it["s0"] < it["s1"] for it in items)
+
+
+@pytest.mark.parametrize("max_q_len", [8192, 70000], ids=["blocks_past_2_24", "row_blocks_past_2_16"])
+def test_extend_launches_more_blocks_than_one_dimension_holds(max_q_len):
+    """2048 sequences with a stated chunk length of up to 8192 tokens of 128
+    heads have 2^24 blocks of 256 threads, and a length of 70000 more row blocks
+    than a grid's second dimension: the call runs, and gives the bits that the
+    true length gives (the other blocks have no rows)."""
+    D, R, H, P, W, page = 256, 32, 128, 4, 16, 16
+    B = 2048 if max_q_len == 8192 else 3
+    prefixes, chunks = [(7 * i) % 40 for i in range(B)], [1 + i % 2 for i in range(B)]
+    sm = 1.0 / math.sqrt(96)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    T, pages = sum(chunks), 16
+    args = [torch.randint(0, 256, (pages * page, D // 4), dtype=torch.uint8, device=DEV, generator=g),
+            torch.tensor([1.1, 1.5], device=DEV).expand(pages * page, D // 128, 2).contiguous(),
+            torch.randn(pages * page, R, device=DEV, generator=g).bfloat16(),
+            torch.randn(1 + (B + 1) * (P + W), D, device=DEV, generator=g).bfloat16()]
+    counts = [-(-n // page) for n in prefixes]
+    indptr = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32, device=DEV)
+    indices = torch.randint(0, pages, (sum(counts),), dtype=torch.int32, device=DEV, generator=g)
+    q = torch.randn(T, H, D + R, device=DEV, generator=g).bfloat16()
+    kc = torch.randn(T, D + R, device=DEV, generator=g).bfloat16()
+    qo = torch.tensor(np.concatenate([[0], np.cumsum(chunks)]), dtype=torch.int32, device=DEV)
+    outs = []
+    for mq in (max(chunks), max_q_len):
+        outs.append(torch.full((T, H, D), float("nan"), dtype=torch.bfloat16, device=DEV))
+        kernels.extend_fwd(q, kc, qo, indptr, indices, torch.tensor(prefixes, device=DEV),
+                           torch.arange(1, B + 1, device=DEV), *args, mq, outs[-1], sm, P, W, page)
+    torch.cuda.synchronize()
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(outs[0], outs[1])
