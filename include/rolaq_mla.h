@@ -41,7 +41,11 @@ extern "C" {
 /* Message of the last error on the calling thread ("" if none). */
 const char* rolaq_last_error(void);
 
-/* ABI version of this library (bumped on any signature change). */
+/* ABI version of this library, bumped on any change of a signature or of a
+ * documented layout. 5: rolaq_decode_fwd shares blocks by the requests' lengths,
+ * its scratch holds partials packed by request and bookkeeping in the last LSE
+ * slot; rolaq_decode_split_cap returns the larger cap; rolaq_extend_scratch_rows
+ * is new. */
 int rolaq_abi_version(void);
 
 /*

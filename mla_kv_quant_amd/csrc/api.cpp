@@ -65,7 +65,7 @@ extern "C" {
 
 const char* rolaq_last_error(void) { return g_err; }
 
-int rolaq_abi_version(void) { return 4; }
+int rolaq_abi_version(void) { return 5; }
 
 int rolaq_scatter_pack_rows(const float* x, int64_t x_stride, const int32_t* slots, int64_t n, int D,
                             int group_size, float threshold, double gain, uint8_t* codes, float* params,

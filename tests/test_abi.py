@@ -30,7 +30,7 @@ def test_library_exports_every_declared_symbol():
         assert hasattr(lib, name), name
     # every declared symbol has a ctypes signature in the binding
     assert set(declared_symbols()) - {"rolaq_last_error"} <= set(_lib.SIGNATURES)
-    assert lib.rolaq_abi_version() == 4
+    assert lib.rolaq_abi_version() == 5
 
 
 def test_invalid_arguments_are_rejected_before_any_launch():
