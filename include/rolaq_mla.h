@@ -142,8 +142,10 @@ int rolaq_prepare_gf_splits(const int32_t* splits, int32_t* quant, int32_t* merg
  * returns it, or, where the batch's requests together ask for more than one
  * working block per compute unit, a share of the units by its length (more
  * splits only add partials to write and merge, and SGLang reads only the merged
- * output; the output does not depend on the split count beyond FP32 summation
- * order).
+ * output; beyond FP32 summation order and the rounding of the fp16 probabilities
+ * against each wave's own softmax reference, 2^-12 each, the output does not
+ * depend on the split count. With shared units a request's low-order bits
+ * therefore depend on the lengths of the others in the batch).
  * Positions P <= t < L_b - W and the window rows are split over
  * nq_b <= max(ns'_b - 1, 1) splits (the window rows go with split 0); the
  * reference's separate window split has no partial of its own here.
@@ -259,7 +261,10 @@ int rolaq_decode_merge(const float* attn_logits, const float* attn_lse, const in
  * returns lets the call split the keys of a block of query rows over several
  * compute units (FP32 partials and their merge, in the workspace's last rows):
  * short chunks over long prefixes and ragged batches are much faster with it.
- * The results differ by FP32 summation order only.
+ * The results differ in FP32 summation order and in the softmax reference, which
+ * each range of keys has of its own, so that the fp16 probabilities round
+ * differently (2^-12 each, as without a split). The split follows all sequences'
+ * lengths: a sequence's low-order bits depend on the batch that it is in.
  * Latent values are carried in fp16 as for rolaq_decode_fwd.
  */
 int rolaq_extend_fwd(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_chunk,
