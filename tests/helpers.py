@@ -133,20 +133,37 @@ def gpu_written_pool(lengths, D, R, P, W, page, seed, max_reqs=None, reqs=None, 
 
 
 def fused_splits(splits, H, D, max_splits):
-    """The split counts rolaq_decode_fwd uses for a batch that requests
-    ``splits``: each capped at the library's split cap for (B, H, D) on the
-    current device (whose partials the fused call writes)."""
+    """The most splits rolaq_decode_fwd gives the requests of a batch that asks
+    for ``splits``: each capped at the library's split cap for (B, H, D) on the
+    current device. Where the call shares its blocks by length a request may
+    have fewer; the LSE of the splits between is that of an empty one (-1e4)."""
     from mla_kv_quant_amd import kernels
     cap = kernels.decode_split_cap(len(splits), H, D, max_splits)
     return [min(int(ns), cap) for ns in splits]
 
 
+def fused_shares(B, H, D, max_splits):
+    """Whether rolaq_decode_fwd shares its blocks by length: several requests, at
+    most 256 and fewer than there are blocks (compute units over head blocks),
+    that can ask for more quantized splits than blocks, and for more than one
+    each."""
+    import torch
+    from mla_kv_quant_amd import kernels
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = cus // (-(-H // 16) if D == 512 else -(-H // 48))
+    most = max(min(kernels.decode_split_cap(B, H, D, max_splits) - 1, max_splits), 1)
+    return 1 < B < blocks and B <= 256 and most > 1 and B * most > blocks
+
+
 def fused_partials(logits, lse, B, H, D, max_splits):
     """The split partials a fused rolaq_decode_fwd call left in its scratch,
     in the standard ``[B, H, max_splits + 1, D]`` / ``[B, H, max_splits + 1]``
-    shape (slots past the fused call's stride are NaN). The fused call stores
-    them from the start of the buffers at a stride of S1c = min(cap - 1,
-    max_splits) + 1 slots per (sequence, head)."""
+    shape, NaN where the call left none. The LSEs lie at a stride of S1c =
+    min(cap - 1, max_splits) + 1 per (sequence, head), and so do the logits of a
+    call that does not share its blocks. One that does leaves in the last LSE slot
+    the request's count and, where its blocks did not suffice for every split
+    asked for, 1 + the blocks of the requests before it (from bit 12 on): the
+    logits are then packed, [H, count] of each request."""
     import torch
     from mla_kv_quant_amd import kernels
     cap = kernels.decode_split_cap(B, H, D, max_splits)
@@ -154,8 +171,19 @@ def fused_partials(logits, lse, B, H, D, max_splits):
     n = B * H * s1c
     lg = torch.full((B, H, max_splits + 1, D), float("nan"), dtype=logits.dtype, device=logits.device)
     ls = torch.full((B, H, max_splits + 1), float("nan"), dtype=lse.dtype, device=lse.device)
-    lg[:, :, :s1c] = logits.reshape(-1)[: n * D].view(B, H, s1c, D)
+    rows = logits.reshape(-1, D)
     ls[:, :, :s1c] = lse.reshape(-1)[:n].view(B, H, s1c)
+    if not fused_shares(B, H, D, max_splits):
+        lg[:, :, :s1c] = rows[:n].view(B, H, s1c, D)
+        return lg, ls
+    code = ls[:, 0, s1c - 1].contiguous().view(torch.int32).tolist()
+    assert (ls[:, :, s1c - 1].contiguous().view(torch.int32) == ls[:, :1, s1c - 1].contiguous().view(torch.int32)).all()
+    for b in range(B):
+        nq, first = code[b] & 0xFFF, code[b] >> 12
+        if first:
+            lg[b, :, :nq] = rows[(first - 1) * H:][:H * nq].view(H, nq, D)
+        else:
+            lg[b, :, :nq] = rows[b * H * s1c:][:H * s1c].view(H, s1c, D)[:, :nq]
     return lg, ls
 
 

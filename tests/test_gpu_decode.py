@@ -17,7 +17,7 @@ import torch
 from oracle import attention, window
 from mla_kv_quant_amd import kernels, synth
 from mla_kv_quant_amd.decode import packed_mla_decode_gf_fwd, prepare_gf_splits
-from tests.helpers import (alloc_slots, build_pool, fused_partials, fused_splits, gpu_pool_to_oracle,
+from tests.helpers import (alloc_slots, build_pool, fused_partials, fused_shares, fused_splits, gpu_pool_to_oracle,
                            gpu_written_pool, index_lists, make_queries, pool_to_gpu)
 
 pytestmark = pytest.mark.gpu
@@ -43,7 +43,8 @@ CASES = [
 WINDOWS = [(4, 16), (4, 8), (0, 0)]
 
 
-def run_decode(gp, q, slots, pages, lengths, reqs, page, splits, max_splits, P, W, sm_scale, max_reqs=None):
+def run_decode(gp, q, slots, pages, lengths, reqs, page, splits, max_splits, P, W, sm_scale, max_reqs=None,
+               seq_lens=True):
     B, H, DR = q.shape
     D = gp["codes"].shape[1] * 4
     indptr, indices = index_lists(slots, pages, page)
@@ -54,7 +55,8 @@ def run_decode(gp, q, slots, pages, lengths, reqs, page, splits, max_splits, P, 
     lse = torch.full((B, H, max_splits + 1), float("nan"), device=DEV)
     out = torch.empty(B, H, D, dtype=torch.bfloat16, device=DEV)
     kernels.decode_fwd(q.to(DEV), gp["codes"], gp["params"], gp["rope"], gp["hp"], indptr, indices,
-                       seq, req, ns, max_splits, logits, lse, out, sm_scale, P, W, page, max_reqs=max_reqs)
+                       seq if seq_lens else None, req, ns, max_splits, logits, lse, out, sm_scale, P, W, page,
+                       max_reqs=max_reqs)
     torch.cuda.synchronize()
     logits, lse = fused_partials(logits, lse, B, H, D, max_splits)
     return out.float().cpu(), logits.cpu(), lse.cpu()
@@ -430,3 +432,47 @@ def test_shared_blocks_read_every_head_of_a_strided_query(D, R, heads):
             plain, _, _ = run_decode(gp, q, *args, [3] * B, 3, P, W, sm)
             assert torch.equal(out, strided), H
             torch.testing.assert_close(out, plain, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("D,R,H,lengths,splits,page,outside", [
+    # every second request asks for one split, the others for all they may have
+    (512, 64, 16, [2000 + 31 * i for i in range(16)], [129 if i % 2 else 1 for i in range(16)], 64, []),
+    # requested counts that all fit the blocks although the batch may ask for more: not packed, unequal counts
+    (512, 64, 16, [500 + 67 * i for i in range(16)], [2 + i % 9 for i in range(16)], 16, []),
+    # lengths from kv_indptr, one token a page, an empty request among them
+    (512, 64, 16, [700, 0, 33, 2100, 64, 900, 20, 1500], [129] * 8, 1, []),
+    (256, 32, 40, [900, 41, 1800, 5, 640, 32], [65, 3, 129, 129, 1, 40], 1, []),
+    # requests without ring rows: no window, every position from its codes
+    (512, 64, 16, [400, 1000, 60, 20, 1700, 90], [129, 129, 50, 129, 1, 129], 64, [1, 3]),
+    (256, 32, 64, [300, 1200, 17, 800], [129, 64, 129, 129], 32, [0, 2]),
+    # all alike but for one requested count
+    (512, 64, 16, [1024] * 12, [129] * 11 + [2], 64, []),
+], ids=["every_second_one", "all_fit", "indptr", "indptr_256", "outside", "outside_h64", "one_count"])
+def test_shared_blocks_mixed_requests(D, R, H, lengths, splits, page, outside):
+    """What decides which sequence and split a shared block takes: requested
+    counts that differ, lengths from kv_indptr, requests without ring rows. Output
+    and LSE against the oracle; the partials, unpacked by the counts that the call
+    left, merge to the output (bf16 of an FP32 sum of as many terms: 2^-8), every
+    head has its request's count, within what the request asked for."""
+    P, W, max_splits = 4, 16, 129
+    sm = 1 / math.sqrt(192 if D == 512 else 96)
+    B = len(lengths)
+    assert fused_shares(B, H, D, max_splits)
+    gp, slots, pages, reqs = gpu_written_pool(lengths, D, R, P, W, page, seed=81, max_reqs=B + 1)
+    reqs = np.asarray([(-1, B + 7)[b % 2] if b in outside else reqs[b] for b in range(B)])
+    q = make_queries(B, H, D, R, sm, seed=83)
+    out, logits, lse = run_decode(gp, q, slots, pages, lengths, reqs, page, splits, max_splits, P, W, sm,
+                                  max_reqs=B + 1, seq_lens=page != 1)
+    live = [b for b in range(B) if lengths[b] > 0]
+    check_against_oracle(gpu_pool_to_oracle(gp), q, out, lse, slots, lengths, reqs, splits, P, W, sm, D,
+                         max_reqs=B + 1, batch_index=live, max_splits=max_splits)
+    asked = [max(ns - 1, 1) for ns in fused_splits(splits, H, D, max_splits)]
+    counts = torch.isfinite(logits).all(-1).sum(-1)
+    assert (counts == counts[:, :1]).all() and (counts >= 1).all()
+    assert (counts[:, 0] <= torch.tensor(asked)).all()
+    for b in live:
+        n = int(counts[b, 0])
+        assert (lse[b, :, n:asked[b]] == -1.0e4).all()
+        w = torch.softmax(lse[b, :, :n].double(), -1)
+        merged = (w[..., None] * logits[b, :, :n].double()).sum(1)
+        torch.testing.assert_close(out[b].double(), merged, rtol=2.0 ** -8, atol=1e-5)

@@ -356,7 +356,7 @@ def test_extend_at_the_edges_of_rows_and_tiles(D, R, H):
     ([6000], [9]),                           # one sequence, one or three blocks of rows: many chunks each
     ([3000, 0, 40, 5000], [1, 300, 30, 64]),  # cut and uncut sequences, a fresh one (causal: blocks of unequal keys)
     ([2050, 2047, 2048], [17, 16, 16]),       # lengths around the steps' multiples
-    ([800] * 70, [2] * 70),                   # more sequences than the lanes of a wave
+    ([2500] * 70, [2] * 70),                  # more sequences than the lanes of a wave
 ], ids=["one", "mixed", "edges", "many"])
 def test_extend_with_split_keys_matches_unsplit(D, R, H, prefixes, chunks):
     """A workspace with room for a plan splits keys; the result is that of a
@@ -391,7 +391,7 @@ def test_extend_with_split_keys_matches_unsplit(D, R, H, prefixes, chunks):
     whole, split = run(rows, rows), run(rows + spare, rows)
     assert torch.isfinite(split.float()).all()
     torch.testing.assert_close(split.float(), whole.float(), rtol=RTOL, atol=ATOL)
-    assert not torch.equal(split, whole) or B == 70  # keys were split
+    assert not torch.equal(split, whole)  # keys were split
     assert torch.equal(split, run(rows + spare + 999, rows))
     # one row short of the truth: a plan would need the key rows' last place
     short = kernels.extend_scratch_rows(B, H, D, R, max(chunks), rows - 1)
@@ -403,10 +403,11 @@ def test_extend_with_split_keys_matches_unsplit(D, R, H, prefixes, chunks):
         torch.testing.assert_close(split[s:e].double().cpu(), ref, rtol=RTOL, atol=ATOL)
 
 
-def _batch(B, seed, prefix, chunk, empty=0.0):
-    """Lengths of B sequences up to twice their means, a share of them without a chunk."""
+def _batch(B, seed, prefix, chunk, empty=0.0, long=()):
+    """Lengths of B sequences up to twice their means, a share of them without a
+    chunk, the prefixes in ``long`` (sequence, length) as given."""
     r = np.random.default_rng(seed)
-    return ([int(v) for v in r.integers(0, 2 * prefix + 1, B)],
+    return ([dict(long).get(b, int(v)) for b, v in enumerate(r.integers(0, 2 * prefix + 1, B))],
             [0 if r.random() < empty else int(v) for v in r.integers(1, 2 * chunk + 1, B)])
 
 
@@ -417,7 +418,7 @@ def _batch(B, seed, prefix, chunk, empty=0.0):
     (512, 16, *_batch(65, 2, 1300, 20, empty=0.3)),         # and one more sequence, some without a chunk
     (256, 16, *_batch(130, 3, 2300, 6)),
     (512, 16, *_batch(300, 4, 1700, 3, empty=0.2)),         # as many ranges as waves
-    (256, 8, *_batch(1200, 5, 2300, 2)),                    # more than two stages of lengths
+    (256, 8, *_batch(1200, 5, 2200, 2, long=((700, 60000), (1199, 90000)))),  # more than two stages of lengths
     (512, 16, [200] * 90 + [60000], [2] * 91),              # one long sequence behind many short ones
 ], ids=["b2", "b3", "b64", "b65", "b130", "b300", "b1200", "long_last"])
 def test_extend_plan_covers_every_key_of_every_row_once(D, H, prefixes, chunks):
@@ -444,8 +445,9 @@ def test_extend_plan_covers_every_key_of_every_row_once(D, H, prefixes, chunks):
     spare = kernels.extend_scratch_rows(B, H, D, R, max(chunks), rows)
     assert spare > 0
 
-    def run(ws):
-        out = torch.full((T, H, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    def run(ws, width=H * D):
+        # (an output whose rows are `width` elements apart)
+        out = torch.full((T, width), float("nan"), dtype=torch.bfloat16, device=DEV)[:, width - H * D:].unflatten(1, (H, D))
         kernels.extend_fwd(q, kc, qo, indptr, indices, torch.tensor(prefixes, device=DEV),
                            torch.arange(1, B + 1, device=DEV), codes, params, rope, hp, max(chunks), out, sm, P, W,
                            page, workspace=ws, key_rows=rows)
@@ -456,6 +458,8 @@ def test_extend_plan_covers_every_key_of_every_row_once(D, H, prefixes, chunks):
     split = run(ws)
     whole = run(torch.empty(rows, D + R, dtype=torch.float16, device=DEV))
     torch.testing.assert_close(split.float(), whole.float(), rtol=RTOL, atol=ATOL)
+    # rows that forbid 16-byte stores, from the blocks and from the merge
+    assert torch.equal(split, run(ws, H * D + 4))
 
     plan = ws[rows:].cpu().numpy().view(np.uint8).reshape(-1)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
@@ -467,7 +471,7 @@ def test_extend_plan_covers_every_key_of_every_row_once(D, H, prefixes, chunks):
     merge = np.dtype([("r0", "<i8"), ("nrows", "<i8"), ("qo0", "<i4"), ("slot0", "<i4"), ("n", "<i4"), ("pad", "<i4")])
     items = plan[256:256 + 64 * n_items].view(item)
     merges = plan[256 + 64 * max_items:][:32 * n_merges].view(merge)
-    assert 0 < n_items <= max_items
+    assert 0 < n_items <= max_items and n_merges > 0
     koffs = np.concatenate([[0], np.cumsum(np.asarray(prefixes) + np.asarray(chunks))])
     by_place = {}
     for it in items:
@@ -526,3 +530,40 @@ def test_extend_launches_more_blocks_than_one_dimension_holds(max_q_len):
     torch.cuda.synchronize()
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("D,H", [(512, 16), (256, 40)])
+def test_extend_chunks_longer_than_stated_go_without_a_plan(D, H):
+    """Chunks whose row blocks pass what the scratch was sized for: the plan
+    says so and the launch's blocks go without it. The rows within the stated
+    length have the bits of a workspace without scratch, those past it are left."""
+    R, P, W, page, pages = D // 8, 4, 16, 16, 64
+    prefix, chunk, stated = 6000, 9000, 1
+    g = torch.Generator(device=DEV).manual_seed(H)
+    codes = torch.randint(0, 256, (pages * page, D // 4), dtype=torch.uint8, device=DEV, generator=g)
+    params = torch.tensor([1.1, 1.5], device=DEV).expand(pages * page, D // 128, 2).contiguous()
+    rope = torch.randn(pages * page, R, device=DEV, generator=g).bfloat16()
+    hp = torch.randn(1 + 2 * (P + W), D, device=DEV, generator=g).bfloat16()
+    indptr = torch.tensor([0, -(-prefix // page)], dtype=torch.int32, device=DEV)
+    indices = torch.randint(0, pages, (-(-prefix // page),), dtype=torch.int32, device=DEV, generator=g)
+    sm = 1.0 / math.sqrt(96 if D == 256 else 192)
+    q = torch.randn(chunk, H, D + R, device=DEV, generator=g).bfloat16()
+    kc = torch.randn(chunk, D + R, device=DEV, generator=g).bfloat16()
+    rows = prefix + chunk
+    spare = kernels.extend_scratch_rows(1, H, D, R, stated, rows)
+    blocks = -(-stated * H // 128)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert 0 < spare and -(-chunk * H // 128) > blocks + min(2 * cus, blocks * -(-(-(-rows // (64 if D == 256 else 32))) // 4))
+    outs = []
+    for n in (rows, rows + spare):
+        outs.append(torch.full((chunk, H, D), float("nan"), dtype=torch.bfloat16, device=DEV))
+        ws = torch.empty(n, D + R, dtype=torch.float16, device=DEV)
+        kernels.extend_fwd(q, kc, torch.tensor([0, chunk], dtype=torch.int32, device=DEV), indptr, indices,
+                           torch.tensor([prefix], device=DEV), torch.ones(1, dtype=torch.int64, device=DEV), codes, params,
+                           rope, hp, stated, outs[-1], sm, P, W, page, workspace=ws, key_rows=rows)
+    torch.cuda.synchronize()
+    assert int(ws[rows:].view(torch.int32).reshape(-1)[0]) == -1  # no plan
+    written = 128 * blocks
+    assert torch.isfinite(outs[0].reshape(-1, D)[:written].float()).all()
+    assert torch.isnan(outs[0].reshape(-1, D)[written:].float()).all()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))

@@ -128,3 +128,132 @@ def test_captured_decode_step_replays_match_eager():
             ref, _ = attention.decode(pool_np, qh[..., :D], qh[..., D:], slots, lens, list(range(1, nreq + 1)), P, W,
                                       sm, D, "stored64", max_reqs=8)
             torch.testing.assert_close(og[li, :nreq].float().cpu().double(), ref, rtol=2e-2, atol=2e-3)
+
+
+def test_captured_shared_decode_replays_at_other_lengths():
+    """Sixteen requests that ask for more splits than there are compute units:
+    the blocks are shared by what the device buffers hold at the replay. One
+    captured call, replayed over equal lengths, ragged ones, requested counts that
+    all fit and empty requests, back and forth, each as the same call run eagerly
+    (whose scratch is its own), and against the oracle."""
+    D, R, H, P, W, page, S, B, cap = 512, 64, 16, 4, 16, 64, 129, 16, 2048
+    from mla_kv_quant_amd import kernels
+    from tests.helpers import fused_shares, gpu_written_pool, make_queries
+    assert fused_shares(B, H, D, S)
+    sm = 1 / math.sqrt(192)
+    gp, slots, pages, reqs = gpu_written_pool([cap] * B, D, R, P, W, page, seed=91)
+    q = make_queries(B, H, D, R, sm, seed=93).to(DEV)
+    pages_of = torch.from_numpy(np.stack([np.asarray(p, dtype=np.int32) for p in pages]))
+    st = {"indptr": torch.zeros(B + 1, dtype=torch.int32, device=DEV),
+          "indices": torch.zeros(B * cap // page, dtype=torch.int32, device=DEV),
+          "seq": torch.zeros(B, dtype=torch.int64, device=DEV), "ns": torch.zeros(B, dtype=torch.int32, device=DEV),
+          "req": torch.from_numpy(np.asarray(reqs)).to(DEV)}
+    outs = {k: [torch.empty(B, H, S + 1, D, device=DEV), torch.empty(B, H, S + 1, device=DEV),
+                torch.empty(B, H, D, dtype=torch.bfloat16, device=DEV)] for k in ("graph", "eager")}
+
+    def set_inputs(lens, ns):
+        counts = [-(-n // page) for n in lens]
+        flat = torch.cat([pages_of[b, :c] for b, c in enumerate(counts)] + [torch.zeros(1, dtype=torch.int32)])
+        st["indptr"].copy_(torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32))
+        st["indices"][:len(flat)].copy_(flat[:st["indices"].numel()])
+        st["seq"].copy_(torch.tensor(lens))
+        st["ns"].copy_(torch.tensor(ns, dtype=torch.int32))
+
+    def call(o):
+        kernels.decode_fwd(q, gp["codes"], gp["params"], gp["rope"], gp["hp"], st["indptr"], st["indices"], st["seq"],
+                           st["req"], st["ns"], S, o[0], o[1], o[2], sm, P, W, page, max_reqs=B + 1)
+
+    # (the window rows in the pool are those of a sequence of `cap` tokens, so every
+    # length here reads some of them at other positions: the eager call and the
+    # oracle read the same ones)
+    ragged = [cap, 100] + [300 + 110 * i for i in range(B - 2)]
+    steps = [([1024] * B, [S] * B), (ragged, [S] * B), ([1024] * B, [S] * B), (ragged, [3 + b % 5 for b in range(B)]),
+             ([0, 5, 0, cap] + [64 * i for i in range(1, B - 3)], [S] * B), ([cap] * B, [S if b % 3 else 1 for b in range(B)]),
+             (ragged, [S] * B)]
+    set_inputs([1] * B, [S] * B)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(outs["graph"])
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(outs["graph"])
+    pool_np = gpu_pool_to_oracle(gp)
+    for i, (lens, ns) in enumerate(steps):
+        set_inputs(lens, ns)
+        for o in outs.values():
+            o[0].fill_(float("nan")), o[1].fill_(float("nan")), o[2].fill_(float("nan"))
+        graph.replay()
+        call(outs["eager"])
+        torch.cuda.synchronize()
+        og, oe = outs["graph"][2], outs["eager"][2]
+        assert torch.equal(og, oe), f"replay {i} differs from the eager call"
+        live = [b for b in (0, 1, 3, 7, B - 1) if lens[b]]
+        ref, _ = attention.decode(pool_np, q.float().cpu()[..., :D], q.float().cpu()[..., D:], slots, lens, reqs, P, W, sm,
+                                  D, "stored64", max_reqs=B + 1, batch_index=live)
+        torch.testing.assert_close(og.double().cpu()[live], ref[live], rtol=2e-2, atol=2e-3)
+        assert (og.cpu()[[b for b in range(B) if not lens[b]]] == 0).all()
+
+
+def test_captured_extend_replays_at_other_lengths():
+    """A captured extend call makes its plan on the device: replayed over other
+    prefix and chunk lengths within the captured bounds it gives the bits of the
+    same call run eagerly; with more key rows than it was told of, into the room
+    for the plan, those of a call without that room."""
+    D, R, H, P, W, page, B, T, mq, pages = 512, 64, 16, 4, 16, 16, 4, 64, 40, 600
+    from mla_kv_quant_amd import kernels
+    g = torch.Generator(device=DEV).manual_seed(7)
+    cache = [torch.randint(0, 256, (pages * page, D // 4), dtype=torch.uint8, device=DEV, generator=g),
+             torch.tensor([1.1, 1.5], device=DEV).expand(pages * page, D // 128, 2).contiguous(),
+             torch.randn(pages * page, R, device=DEV, generator=g).bfloat16(),
+             torch.randn(1 + (B + 1) * (P + W), D, device=DEV, generator=g).bfloat16()]
+    sm = 1 / math.sqrt(192)
+    q = (torch.randn(T, H, D + R, device=DEV, generator=g) * (2.0 / (sm * math.sqrt(D + R)))).bfloat16()
+    kc = torch.randn(T, D + R, device=DEV, generator=g).bfloat16()
+    key_rows = 9000
+    spare = kernels.extend_scratch_rows(B, H, D, R, mq, key_rows)
+    assert spare > 0
+    st = {"qo": torch.zeros(B + 1, dtype=torch.int32, device=DEV), "indptr": torch.zeros(B + 1, dtype=torch.int32, device=DEV),
+          "indices": torch.randint(0, pages, (1000,), dtype=torch.int32, device=DEV, generator=g),
+          "pl": torch.zeros(B, dtype=torch.int64, device=DEV), "req": torch.arange(1, B + 1, device=DEV)}
+    ws = {k: torch.empty(key_rows + spare, D + R, dtype=torch.float16, device=DEV) for k in ("graph", "eager")}
+    out = {k: torch.empty(T, H, D, dtype=torch.bfloat16, device=DEV) for k in ("graph", "eager", "whole")}
+
+    def set_inputs(prefixes, chunks):
+        counts = [-(-n // page) for n in prefixes]
+        st["qo"].copy_(torch.tensor(np.concatenate([[0], np.cumsum(chunks)]), dtype=torch.int32))
+        st["indptr"].copy_(torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int32))
+        st["pl"].copy_(torch.tensor(prefixes))
+
+    def call(o, w, rows=key_rows):
+        kernels.extend_fwd(q, kc, st["qo"], st["indptr"], st["indices"], st["pl"], st["req"], *cache, mq, o, sm, P, W, page,
+                           workspace=w, key_rows=rows)
+
+    set_inputs([100] * B, [4] * B)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(out["graph"], ws["graph"])
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out["graph"], ws["graph"])
+    short = ([9300, 40, 0, 0], [16, 16, 16, 16])  # 9404 key rows: into the plan's room
+    steps = [([2200] * B, [16] * B), ([8000, 0, 300, 1], [40, 1, 0, 23]), ([2200] * B, [16] * B), short,
+             ([0, 0, 0, 8936], [1, 20, 3, 40]), ([50] * B, [10] * B), short, ([8000, 0, 300, 1], [40, 1, 0, 23])]
+    for i, (prefixes, chunks) in enumerate(steps):
+        set_inputs(prefixes, chunks)
+        for t in (*ws.values(), *out.values()):
+            t.fill_(float("nan"))
+        graph.replay()
+        call(out["eager"], ws["eager"])
+        rows = sum(prefixes) + sum(chunks)
+        call(out["whole"], torch.empty(rows, D + R, dtype=torch.float16, device=DEV), rows)
+        torch.cuda.synchronize()
+        n = sum(chunks)
+        assert torch.isfinite(out["whole"][:n].float()).all()
+        assert torch.equal(out["graph"].view(torch.int16), out["eager"].view(torch.int16)), f"replay {i}"
+        torch.testing.assert_close(out["graph"][:n].float(), out["whole"][:n].float(), rtol=2e-2, atol=2e-3)
+        split = not torch.equal(out["graph"][:n], out["whole"][:n])
+        assert split == (rows <= key_rows and max(prefixes) > 1000), i
