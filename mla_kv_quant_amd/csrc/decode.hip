@@ -142,21 +142,6 @@ __device__ __forceinline__ void expand_word(uint32_t w, const Lut& t, u32x4& c0,
 __device__ __forceinline__ void lds_store128(uint8_t* p, u32x4 v) { *reinterpret_cast<u32x4*>(p) = v; }
 __device__ __forceinline__ u32x4 lds_load128(const uint8_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
-// 64 bits of the output MFMA's B operand, read transposed out of the expanded
-// rows (ds_read_b64_tr_b16: within each 16-lane group, lane 4s + e receives
-// element e of the 8-byte chunks addressed by lanes s, s+4, s+8, s+12). Lane
-// (gq, la) addresses row 16h + 4gq + (la >> 2) at elements 16nb + 4(la & 3),
-// so it receives rows 16h + 4gq + 0..3 of element 16nb + la.
-template <int ROWB>
-__device__ __forceinline__ u32x2 read_vt(const uint8_t* buf, int gq, int la, int nb, int h) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const int row = 16 * h + 4 * gq + (la >> 2);
-  const int e = 16 * nb + 4 * (la & 3);
-  const uint8_t* p = buf + row * ROWB + 16 * ((e >> 3) ^ sw(row)) + 2 * (e & 7);
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p)));
-}
-
 template <int D, int R>
 struct TileRegs {
   u32x4 code[2][DGeo<D, R>::CV];  // packed words of the lane's group, M-blocks 0 / 1
@@ -621,7 +606,11 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   // only touches the low 3 bits of a 16-byte chunk index, so
   //   store of K-step j, M-block mb:  wb[mb][j & 1] + 128 (j >> 1)
   //   V^T read of N-block nb, half h: rb[nb & 3] + 128 (nb >> 2) + 16 ROWB h
-  // (read_vt's address, regrouped).
+  // The latter is 64 bits of the output MFMA's A operand, read transposed out of
+  // the expanded rows (ds_read_b64_tr_b16: within each 16-lane group, lane 4s + e
+  // receives element e of the 8-byte chunks addressed by lanes s, s+4, s+8, s+12):
+  // lane (gq, la) addresses row 16h + 4gq + (la >> 2) at elements 16nb + 4(la & 3),
+  // so it receives rows 16h + 4gq + 0..3 of element 16nb + la.
   uint8_t* wb[2][2];
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)

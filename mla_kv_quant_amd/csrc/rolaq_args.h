@@ -95,7 +95,7 @@ struct ExtendArgs {
   int B, H, P, W;
   int max_reqs;             // req_idx outside [0, max_reqs) reads no window rows
   float sm_scale;
-  uint16_t* ws;             // workspace: key rows [ws_rows, D + R] bf16 (gathered per call)
+  uint16_t* ws;             // workspace [ws_rows, D + R]: fp16 key rows (gathered per call), at its end the scratch
   int64_t ws_rows;
   uint16_t* out;            // [T, H, D] bf16, strides (o_st, o_sh)
   int64_t o_st, o_sh;

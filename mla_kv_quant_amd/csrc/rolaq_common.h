@@ -103,12 +103,6 @@ __device__ __forceinline__ T gload(const void* p) {
 // in [2^-24, 65504] that fit fp16's 11-bit significand, which covers every bf16
 // value in [2^-17, 65504]; beyond 65504 -> inf).
 __device__ __forceinline__ uint32_t bf16x2_to_f16x2(uint32_t v) { return pack_f16(bf16_lo(v), bf16_hi(v)); }
-// One dword of two fp16 -> the same two values as bf16 (exact for fp16 values
-// that are bf16 numbers, as the decode's levels and window rows are).
-__device__ __forceinline__ uint32_t f16x2_to_bf16x2(uint32_t v) {
-  const f16x2_t h = __builtin_bit_cast(f16x2_t, v);
-  return pack_bf16((float)h[0], (float)h[1]);
-}
 __device__ __forceinline__ u32x4 bf16x8_to_f16x8(u32x4 v) {
   return u32x4{bf16x2_to_f16x2(v.x), bf16x2_to_f16x2(v.y), bf16x2_to_f16x2(v.z), bf16x2_to_f16x2(v.w)};
 }
@@ -180,32 +174,12 @@ __device__ __forceinline__ void define_acc_macros() {
 #undef ROLAQ_ACC_CASES
 #undef ROLAQ_ACC_CASE
 
-// Four output accumulators, element j of each scaled by f_j in place when
+// Sixteen output accumulators, element j of each scaled by f_j in place when
 // need (a lane mask) is not 0. The branch is inside the asm: for the compiler
 // the accumulators flow through unchanged in their registers, so the rare
 // rescale adds no copies at a join. The leading waits cover the output MFMA
 // that last wrote them (tens of instructions earlier), the trailing ones an
 // MFMA that reads them next.
-__device__ __forceinline__ void scale_acc4(f32x4& a, f32x4& b, f32x4& c, f32x4& d, const float (&f)[4],
-                                           uint64_t need) {
-  float t0, t1, t2, t3;
-  asm volatile(
-      "s_cmp_lg_u64 %12, 0\n\t"
-      "s_cbranch_scc0 1f\n\t"
-      "s_nop 7\n\ts_nop 7\n\t"
-      "ROLAQ_ACC_SCALE %0, %4, %5, %6, %7, %8, %9, %10, %11\n\t"
-      "ROLAQ_ACC_SCALE %1, %4, %5, %6, %7, %8, %9, %10, %11\n\t"
-      "ROLAQ_ACC_SCALE %2, %4, %5, %6, %7, %8, %9, %10, %11\n\t"
-      "ROLAQ_ACC_SCALE %3, %4, %5, %6, %7, %8, %9, %10, %11\n\t"
-      "s_nop 7\n"
-      "1:"
-      : "+a"(a), "+a"(b), "+a"(c), "+a"(d), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
-      : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "s"(need)
-      : "scc");
-}
-
-// scale_acc4 over 16 accumulator tuples behind one test of the lane mask
-// (one branch instead of four when nothing is scaled)
 __device__ __forceinline__ void scale_acc16(f32x4 (&o)[16], const float (&f)[4], uint64_t need) {
   float t0, t1, t2, t3;
   asm volatile(
