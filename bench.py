@@ -467,14 +467,29 @@ def copy_probe(nbytes: int = 1 << 30, reps: int = 10) -> float:
     return 2.0 * nbytes / (ms * 1e-3) / 1e9
 
 
-def reported_decode_result(args, dev: str, name: str) -> dict:
-    """Decode at the library's own split policy (the reference's 129 splits requested,
-    capped by the library at one working block per CU): cfg3 (ragged large batch) and
-    cfg4a (MiniCPM3 shape), 4 layers with their own buffers; "serve_b8" / "serve_b16":
-    DeepSeek-V2-Lite shape at the reference's serving batch sizes (serve.py:157-158,164),
-    8 layers."""
+def splits_used(db) -> list[int]:
+    """Each request's split count (the window split's one included) in the fused call
+    as ``db`` is set up: what a call that shares its blocks leaves in the last LSE slot
+    of a head, else the capped request."""
     from mla_kv_quant_amd import kernels
 
+    cap = kernels.decode_split_cap(db.B, db.H, db.D, db.max_splits)
+    s1c = max(min(cap - 1, db.max_splits), 1) + 1
+    db.lse.zero_()
+    db.step()
+    code = db.lse.reshape(-1)[: db.B * db.H * s1c].view(db.B, db.H, s1c)[:, 0, -1].contiguous().view(torch.int32).tolist()
+    asked = [max(min(int(n), cap) - 1, 1) for n in db.ns.tolist()]
+    return [(c & 0xFFF if c else a) + 1 for c, a in zip(code, asked)]
+
+
+def reported_decode_result(args, dev: str, name: str) -> dict:
+    """Decode at the library's own split policy (the reference's 129 splits requested,
+    one working block per CU shared by the requests' lengths): cfg3 (ragged large batch)
+    and cfg4a (MiniCPM3 shape), 4 layers with their own buffers; "serve_b8" / "serve_b16":
+    DeepSeek-V2-Lite shape at the reference's serving batch sizes (serve.py:157-158,164),
+    8 layers. Stage 1 alone is timed where all requests have the same count (the stage's
+    own entry point takes requested counts and does not share); a ragged batch's fractions
+    are of the whole layer."""
     layers = 4
     if name == "cfg3":
         lens = np.random.default_rng(3).integers(2048, 8193, size=128)
@@ -491,33 +506,32 @@ def reported_decode_result(args, dev: str, name: str) -> dict:
                     f"(the reference's graph batch sizes, serve.py:157-158,164)")
     db.alloc_scratch(129)
     db.set_splits(129)  # the reference's static split count (serve.py:121,163,198)
-    head_blocks = -(-db.H // (16 if db.D == 512 else 48))
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    ns = min(129, -(-cus // (db.B * head_blocks)) + 1)  # equal counts, one working block per CU
     steps = max(5, args.steps // 2)
     time_loop(db.step, steps, args.warmup)  # a first pass over fresh buffers runs slower: not timed
     ms = float(np.median([time_loop(db.step, steps, 1) for _ in range(3)]))
     us = ms * 1000.0 / layers
-    # stage 1 alone (decode_partials honours the count and launches max_kv_splits + 1
-    # split rows) at equal counts, with scratch sized to them
-    db.alloc_scratch(ns)
-    db.set_splits(ns)
-    ms1 = float(np.median([time_loop(db.step_partials, steps, 1) for _ in range(3)]))
-    us1 = ms1 * 1000.0 / layers
-    ach1 = db.bytes_per_layer(with_out=False) / (us1 * 1e-6) / 1e9
+    used = splits_used(db)
     res = {
         "workload": workload,
         "us_per_layer": round(us, 3),
         "hbm_frac_layer": round(db.bytes_per_layer() / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
-        "stage1_us": round(us1, 3),
-        "stage1_gbs": round(ach1, 1),
-        "stage1_hbm_frac": round(ach1 / HBM_PEAK_GBS, 4),
-        "mfma_frac": round(db.flops_per_layer() / (us1 * 1e-6) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
+        "mfma_frac_layer": round(db.flops_per_layer() / (us * 1e-6) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
         "num_kv_splits_requested": 129,
-        "num_kv_splits_used": ns,
+        "num_kv_splits_used": used[0] if min(used) == max(used) else [min(used), max(used)],
         "tokens": int(db.lengths.sum()),
     }
-    print(f"[bench] {name}: {us:.2f} us/layer, stage 1 {us1:.2f} us ({ach1:.0f} GB/s)", file=sys.stderr, flush=True)
+    text = f"splits {min(used)} .. {max(used)}"
+    if min(used) == max(used):
+        # decode_partials honours the count and launches max_kv_splits + 1 split rows:
+        # scratch sized to the count
+        db.alloc_scratch(used[0])
+        db.set_splits(used[0])
+        us1 = float(np.median([time_loop(db.step_partials, steps, 1) for _ in range(3)])) * 1000.0 / layers
+        ach1 = db.bytes_per_layer(with_out=False) / (us1 * 1e-6) / 1e9
+        res.update(stage1_us=round(us1, 3), stage1_gbs=round(ach1, 1), stage1_hbm_frac=round(ach1 / HBM_PEAK_GBS, 4),
+                   mfma_frac=round(db.flops_per_layer() / (us1 * 1e-6) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4))
+        text = f"stage 1 {us1:.2f} us ({ach1:.0f} GB/s)"
+    print(f"[bench] {name}: {us:.2f} us/layer, {text}", file=sys.stderr, flush=True)
     del db
     torch.cuda.empty_cache()
     return res
