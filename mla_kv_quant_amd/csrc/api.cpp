@@ -271,13 +271,16 @@ int decode_args(const char* who, const void* q, int64_t q_stride_b, int64_t q_st
 
 // The most splits the fused decode gives one request. `each` quantized splits
 // give every compute unit a working block over the batch's (sequence, head
-// block) pairs; the units are shared by the requests' lengths (share_blocks in
-// decode.hip), up to four times `each` for one request. Past 64 splits the
-// merge costs what the share gives (four requests of 26000 .. 65536 tokens, 20
-// heads at D = 256: 53.8 us with 64 each, 55.3 us shared), so up to four
-// requests have `each` as they are. Plus the window split, and never more than
-// the caller's maximum. The merged output does not depend on the split count
-// (up to FP32 summation order).
+// block) pairs. A request may have more where the units are shared by the
+// requests' lengths (share_blocks in decode.hip): up to four times `each`, and
+// past 64 no more than `each`, as the merge then costs what the share gives (four
+// requests of 26000 .. 65536 tokens, 20 heads at D = 256: 53.8 us with 64 each,
+// 55.3 us shared). So with 256 units and one head block two or four requests have
+// `each` = 128 or 64, which fit and are not shared; three have 86 at most, which
+// do not fit together and are. Plus the window split, and never more than the
+// caller's maximum. The split count changes the output in FP32 summation order
+// and in the rounding of the fp16 probabilities, each wave having a softmax
+// reference of its own.
 int fused_split_cap(int B, int H, int D, int max_kv_splits) {
   const int64_t units = int64_t(B) * rolaq_decode_head_blocks(D, H);
   const int64_t each = (cu_count() + units - 1) / units;
