@@ -309,7 +309,6 @@ void fused_layout(rolaq::DecodeArgs* a, int B, int H, int D, int max_kv_splits) 
   const bool share = B > 1 && B < blocks && B <= rolaq::kShareRequests && a->S1 > 2;
   a->blocks = share && most > blocks && blocks < 4096 ? int(blocks) : 0;
   a->blocks_each = a->blocks / B;
-  a->div_b = (1u << 20) / (uint32_t)B + 1;
 }
 
 }  // namespace

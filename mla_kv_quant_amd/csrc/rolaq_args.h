@@ -25,7 +25,6 @@ struct DecodeArgs {
   int S1;        // max_kv_splits + 1
   int blocks;    // > 0: blocks per head block, shared by the requests by their lengths (fused call); 0: equal rows
   int blocks_each;  // blocks / B
-  uint32_t div_b;   // floor(p / B) = (p div_b) >> 20 for block numbers p < 4096 and B <= 256
   int max_reqs;  // requests with ring rows; req_idx outside [0, max_reqs) reads no window rows
   int B, H, P, W;
   float sm_scale;
