@@ -569,7 +569,11 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   const int s0 = uniform(it.s0), s1 = uniform(it.s1), slot = uniform(it.slot);
   // the block's first and last query token, within the sequence; keys are
   // counted from the item's first one on
-  const int64_t t_first = uniform(r0 / a.H), t_last = uniform(min(nrows - 1, r0 + BM - 1) / a.H);
+  // (a 64-bit division is some 150 instructions of a start that is bound by them)
+  auto token_of = [&](int64_t row) {
+    return nrows >> 31 == 0 ? (int64_t)((uint32_t)row / (uint32_t)a.H) : row / a.H;
+  };
+  const int64_t t_first = uniform(token_of(r0)), t_last = uniform(token_of(min(nrows - 1, r0 + BM - 1)));
   const int key0 = s0 * KT;
   const int64_t koff = uniform(it.koff) + key0;
   const int kend = (int)min(prefix + t_last + 1, (int64_t)s1 * KT) - key0;
@@ -585,7 +589,10 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
   auto row_of = [&](int lane32) {
     const int rest = (int)(r0 - t_first * a.H) + RW * wave + lane32;  // from the first token's head 0
     Row r{r0 + RW * wave + lane32 < nrows, t_first, 0};
-    if (r.ok) r.t += rest / a.H, r.h = rest % a.H;
+    if (r.ok) {
+      const uint32_t t = (uint32_t)rest / (uint32_t)a.H;  // (rest >= 0)
+      r.t += t, r.h = rest - (int)t * a.H;
+    }
     return r;
   };
   // They are copied to LDS as whole rows (like a key tile, into ring buffers
@@ -599,13 +606,25 @@ __global__ __launch_bounds__((64 * ExtGeo<D, R>::WAVES), 1) void extend_kernel(E
     const Row r = row_of(la32);
     qp = r.ok ? (int)(prefix + r.t) - key0 : -(1 << 30);
     const int64_t mine = reinterpret_cast<int64_t>(a.q + (qo0 + r.t) * a.q_st + r.h * a.q_sh);
+    // nine pieces are whole rows, 8 at D = 512 and 16 at D = 256, whose places
+    // repeat in the next nine but for the swizzle's bit of row 8: the places are
+    // worked out once (a start is bound by its instructions)
+    constexpr int kTurn = 9, kTurnRows = kTurn * 64 / CPR;
+    static_assert(kTurnRows * CPR == kTurn * 64 && RW % kTurnRows == 0, "whole rows per turn");
+    const int lo = (int)mine, hi = (int)(mine >> 32);
 #pragma unroll
-    for (int j = 0; j < RW * CPR / 64; ++j) {
+    for (int j = 0; j < kTurn; ++j) {
       const int ci = 64 * j + lane, row = ci / CPR, pc = ci - row * CPR;
-      const uint64_t src = (uint64_t)__shfl(mine, row) + 16 * (pc ^ ext_sw<D>(row));
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                   ::"s"(lds0 + kQBuf * G::TILE + RW * RB * wave + 1024 * j), "v"(src)
-                   : "memory", "m0");
+      const uint32_t off = 16 * (pc ^ ext_sw<D>(row));
+#pragma unroll
+      for (int k = 0; k < RW / kTurnRows; ++k) {
+        const uint64_t base = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * row + 4 * kTurnRows * k, lo) |
+                              (uint64_t)(uint32_t)__builtin_amdgcn_ds_bpermute(4 * row + 4 * kTurnRows * k, hi) << 32;
+        const uint64_t src = base + (off ^ (16 * ext_sw<D>(kTurnRows * k)));
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                     ::"s"(lds0 + kQBuf * G::TILE + RW * RB * wave + 1024 * (j + kTurn * k)), "v"(src)
+                     : "memory", "m0");
+      }
     }
   }
   const float c2 = a.sm_scale * kLog2e;
