@@ -35,6 +35,16 @@ def test_pool_workspace_follows_the_key_rows_alone(D, R):
     assert pool.extend_workspace(20001) is not ws
 
 
+def test_a_plan_needs_longer_keys_where_blocks_nearly_fill_the_card():
+    """24 steps of keys (twice the mean) up to 7/8 of the compute units, 64 from
+    there. 256 units (the count without a device); 64-key steps, a block per 128
+    query rows and sequence."""
+    D, R, B, rows = 256, 32, 4, lambda blocks: blocks // 4 * 128
+    for blocks, keys, split in ((220, 12 * 64, True), (220, 12 * 64 - 1, False), (224, 32 * 64 - 1, False),
+                                (224, 32 * 64, True), (256, 32 * 64 - 1, False), (256, 32 * 64, True)):
+        assert (kernels.extend_scratch_rows(B, 1, D, R, rows(blocks), B * keys) > 0) == split, (blocks, keys)
+
+
 def test_refused_extend_calls_keep_their_errors():
     from mla_kv_quant_amd.extend import packed_mla_extend_fwd
 
