@@ -60,7 +60,7 @@ _Tensor = torch.Tensor
 def _need_all(device, specs):
     """``specs``: (tensor, name, dtype, ndim or None) of contiguous tensors on ``device``."""
     for t, name, dtype, ndim in specs:
-        if isinstance(t, _Tensor) and t.dtype is dtype and t.device == device and (ndim is None or t.ndim == ndim) \
+        if isinstance(t, _Tensor) and t.dtype is dtype and t.device == device and (t.ndim == ndim or ndim is None) \
                 and t.is_contiguous():
             continue
         _need(t, name, dtype, device, ndim)
