@@ -789,7 +789,11 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
   // conversions (all of them at once held up the rope rows behind 2000 cycles of
   // the texture path), the first tile's loads behind the set-up (they have the
   // window tile's time to land), and its buffer is left as it is (the window
-  // tile writes all of it).
+  // tile writes all of it). With three head groups, whose set-up is three times
+  // as long, the first tile's loads go out ahead of it as in the other waves: 128
+  // requests of 4000 tokens, 40 heads, 48.2 us a layer, 47.7 so; 64 of 16384 76.5 and
+  // 76.1; 16 of 4000 21.3 and 21.4 (two groups: 64 of 1300 .. 16000 40.4 and 40.7).
+  constexpr bool kSpread = NC > 0 && HG < 3;
   auto setup = [&](auto fill, auto between) {
     // this wave's buffer starts as zeros (see the pending-output rule below),
     // the softmax state, and the query operands (unless blocks are shared,
@@ -850,19 +854,20 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
     lookup(0, pgc);
     lookup(min(1, nl), pgn);
     window_pages();
-    if constexpr (NC > 0) {
+    if constexpr (kSpread) {
       __builtin_amdgcn_sched_barrier(0);
       load_q();
       __builtin_amdgcn_sched_barrier(0);
     }
     window_row_bases();
 #pragma unroll
-    for (int j = 0; j < (NC == 0 ? KL : KL / 2); ++j) window_rows(j);
+    for (int j = 0; j < (kSpread ? KL / 2 : KL); ++j) window_rows(j);
+    if constexpr (NC > 0 && !kSpread) load_q();
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (NC == 0) setup(std::true_type{}, nothing);
     __builtin_amdgcn_sched_barrier(0);
     window_rope();
-    if constexpr (NC > 0) {
+    if constexpr (kSpread) {
       __builtin_amdgcn_sched_barrier(0);
       setup(std::false_type{}, [&](int j) {
         if (j >= KL / 2) window_rows(j);
@@ -871,6 +876,8 @@ __global__ __launch_bounds__(kThreads, 1) void decode_stage1(DecodeArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
     load(0, pgc, dn);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NC > 0 && !kSpread) setup(std::true_type{}, nothing);
     __builtin_amdgcn_sched_barrier(0);
     window_tile();
     first = false;
